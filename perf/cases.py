@@ -199,3 +199,92 @@ def tolerance(case):
     if case["kind"] in ("maxavg_train", "op_train", "separate_train"):
         return {"rel": 8e-3, "max": 0.98}
     return {"rel": 2e-6, "max": 3e-5}
+
+
+def exact(case, seed):
+    """The outputs in 64 bits by plain torch: the volume of every image-1 row block formed whole, reduced and let go.
+    None stands where the definition leaves a choice (the gradient of a maximum with two candidates that agree to the
+    last bits goes to either) and for the lookups, whose gathers no dense form gives in reasonable time."""
+    kind = case["kind"]
+    if kind.startswith("lookup"):
+        return None
+    s = prepare(case, seed)
+    train = kind.endswith("train")
+    with torch.no_grad():
+        if kind.startswith("separate"):
+            outs = _exact_separate(s)
+            return [outs, [None] * 4] if train else tuple(outs)
+        f1, f2 = s["f1"].double(), s["f2"].double()
+        outs = _exact_max_avg(f1, f2)
+        if kind.startswith("maxavg"):
+            return [outs, [None] * 2] if train else tuple(outs)
+        comp = _exact_weighted(f1, f2, s["a_u"].double(), s["a_v"].double())
+        if not train:
+            return tuple(outs), tuple(comp)
+        # (d_a_u = sum_u S g_cu and d_a_v = sum_v S g_cv: the same sums with the gradients as weights)
+        d_v, d_u = _exact_weighted(f1, f2, s["grads"][3].double(), s["grads"][2].double())
+        return [outs + comp, [None, None, d_u, d_v]]
+
+
+def _volume_blocks(f1, f2):
+    """(batch entry, image-1 rows, their volume (rows, W1, H2, W2)), at most about 2^27 entries at a time."""
+    B, H1, W1, C = f1.shape
+    _, H2, W2, _ = f2.shape
+    rows = max(1, 2 ** 27 // (W1 * H2 * W2))
+    for b in range(B):
+        flat = f2[b].reshape(H2 * W2, C).t().contiguous()
+        for i in range(0, H1, rows):
+            part = f1[b, i:i + rows]
+            yield b, slice(i, i + rows), (part.reshape(-1, C) @ flat).view(part.shape[0], W1, H2, W2)
+
+
+def _exact_max_avg(f1, f2):
+    B, H1, W1, _ = f1.shape
+    out_u, out_v = f1.new_empty(B, H1, W1, 2, f2.shape[1]), f1.new_empty(B, H1, W1, 2, f2.shape[2])
+    for b, rows, vol in _volume_blocks(f1, f2):
+        out_u[b, rows] = torch.stack((vol.amax(3), vol.mean(3)), 2)
+        out_v[b, rows] = torch.stack((vol.amax(2), vol.mean(2)), 2)
+    return [out_u, out_v]
+
+
+def _exact_weighted(f1, f2, over_v, over_u):
+    """sum_v S over_v[k, v] and sum_u S over_u[k, u] for every image-1 pixel and channel k."""
+    B, H1, W1, K, _ = over_v.shape
+    out_u, out_v = f1.new_empty(B, H1, W1, K, f2.shape[1]), f1.new_empty(B, H1, W1, K, f2.shape[2])
+    for b, rows, vol in _volume_blocks(f1, f2):
+        for k in range(K):
+            out_u[b, rows, :, k] = (vol * over_v[b, rows, :, k, None, :]).sum(3)
+            out_v[b, rows, :, k] = (vol * over_u[b, rows, :, k, :, None]).sum(2)
+    return [out_u, out_v]
+
+
+def _exact_attention(conv, sep):
+    """softmax over the displacement axis of the 3x3x3 convolution of sep (B,H1,W1,2,L): (B,H1,W1,K,L)."""
+    x = torch.nn.functional.pad(sep.permute(0, 3, 4, 1, 2), (1,) * 6)
+    w, bias = conv.weight.double(), conv.bias.double()
+    L, H, W = x.shape[2] - 2, x.shape[3] - 2, x.shape[4] - 2
+    z = bias.view(1, -1, 1, 1, 1).expand(x.shape[0], -1, L, H, W).clone()
+    for d in range(27):
+        t, i, j = d // 9, d // 3 % 3, d % 3
+        for c in range(2):
+            z += w[:, c, t, i, j].view(1, -1, 1, 1, 1) * x[:, c:c + 1, t:t + L, i:i + H, j:j + W]
+    return z.softmax(2).permute(0, 3, 4, 1, 2).contiguous()
+
+
+def _exact_separate(s):
+    f1 = s["fmap1"].double().permute(0, 2, 3, 1).contiguous() / math.sqrt(s["fmap1"].shape[1])
+    fmap2 = s["fmap2"].double()
+    H, W = fmap2.shape[2:]
+    levels = []
+    for _ in range(4):
+        f2 = fmap2.permute(0, 2, 3, 1).contiguous()
+        sep = _exact_max_avg(f1, f2)
+        over_v, over_u = (_exact_attention(conv, x) for conv, x in zip(s["attention"], sep[::-1]))
+        comp = _exact_weighted(f1, f2, over_v, over_u)
+        level = []
+        for x, c, L in zip(sep[::-1], comp[::-1], (W, H)):
+            v = torch.cat((x, c), 3).permute(0, 3, 4, 1, 2)
+            level.append(torch.nn.functional.interpolate(v, (L, H, W), mode="trilinear", align_corners=True))
+        levels.append(level)
+        fmap2 = torch.nn.functional.avg_pool2d(fmap2, 2, 2)
+    return [torch.cat([l[i] for l in levels], 1) for i in range(2)]
