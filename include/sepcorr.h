@@ -25,9 +25,14 @@
  *  - Backward entry points need scratch memory: query sepcorr_backward_workspace_bytes() and pass a
  *    device buffer of at least that size (256-byte aligned).  Its contents on entry are ignored.
  *  - Forward entry points take scratch memory optionally (sepcorr_forward_workspace_bytes(), 256-byte aligned,
- *    contents on entry ignored; NULL is allowed).  With it the sweep is dealt out to the chip in pieces smaller
- *    than a 32-pixel tile where whole tiles would leave compute units idle (e.g. 440 tiles on 256 units); results
- *    are deterministic either way and differ from each other only in the rounding of the sums over u.
+ *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels and at least 256 steps (128
+ *    pixels of image 1 x 32 columns of a row of image 2) run on the 16-bit matrix units, every fp32 operand as two
+ *    halves with a power-of-two scale per pixel, at the accuracy of fp32 products (csrc/split_sweep.hip); without a
+ *    workspace (or with one smaller than sepcorr_forward_levels_workspace_bytes() of the one level) they take their
+ *    scratch from the stream's memory pool, which costs host time on each call.  The other sizes, and calls without a workspace
+ *    under stream capture, run the fp32 sweep: with a workspace it is dealt out in pieces smaller than a 32-pixel tile
+ *    where whole tiles would leave compute units idle; with and without one the results differ only in the rounding
+ *    of the sums over u.
  */
 #ifndef SEPCORR_H
 #define SEPCORR_H
@@ -109,7 +114,8 @@ int sepcorr_max_avg_forward(const float *f1, const float *f2, float *out_u, floa
                             void *workspace, size_t workspace_bytes, void *stream);
 
 /* Scratch bytes a forward entry point can make use of for these sizes (K = 2 for the max/avg entry points); 0 when
- * whole tiles already fill the chip. */
+ * whole 32-pixel tiles already fill the chip.  sepcorr_forward_levels_workspace_bytes() with one level gives what the
+ * sweep on the 16-bit matrix units takes at those sizes too. */
 size_t sepcorr_forward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C, int K);
 
 /*

@@ -7,6 +7,8 @@ device memory and the current stream only; the arithmetic happens in libsepcorr.
 Checks mirror CHECK_CUDA / CHECK_CONTIGUOUS (MemorySaver_cuda.cpp:6-8) and add the dtype and
 shape agreement the reference leaves unchecked; every violation raises RuntimeError.
 """
+import ctypes
+
 import torch
 
 from . import _lib
@@ -56,10 +58,13 @@ def _workspace(lib, dims, device):
 
 
 def _fwd_workspace(lib, dims, K, device):
-    """Optional scratch of the forward-type sweeps (lets them use the whole chip when tiles do not divide evenly)."""
+    """Optional scratch of the forward-type sweeps (the split operands of the 16-bit matrix units; pieces of tiles)."""
     n = lib.sepcorr_forward_workspace_bytes(*dims, K)
-    if n == 0:
-        return None, None, 0
+    if n == 0:   # (whole tiles fill the chip: only the sweep with split operands can use any)
+        B, H1, W1, H2, W2, C = dims
+        if not 32 <= C <= 256:
+            return None, None, 0
+        n = lib.sepcorr_forward_levels_workspace_bytes((ctypes.c_int * 1)(H2), (ctypes.c_int * 1)(W2), 1, B, H1, W1, C, K)
     ws = torch.empty(n, dtype=torch.uint8, device=device)
     return ws, ws.data_ptr(), n
 
@@ -381,7 +386,6 @@ def attention_logits_backward_levels(seps, weight, grad_logits, d_sep_init=None,
 # --- several pyramid levels per call (the caller's loop over levels, core/corr.py:416-457)
 
 def _levels_setup(f1, f2_levels, K):
-    import ctypes
     _check("img1_features_l0", f1, ndim=4)
     B, H1, W1, C = f1.shape
     lv = list(f2_levels)

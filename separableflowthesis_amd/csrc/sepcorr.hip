@@ -38,6 +38,7 @@
 
 #include "sepcorr.h"
 #include "sepcorr_internal.h"
+#include "split_sweep.h"
 
 // This file is compiled once per part (see the Makefile) so that its many kernel instantiations build in parallel:
 // part 0 holds the C ABI and the state shared by all parts, every other part holds the explicit instantiations of
@@ -3123,10 +3124,72 @@ size_t fwd_split_bytes(int B, int H1, int W1, int H2, int W2, int K) {
     return best;
 }
 
+// Scratch for any forward-type sweep of these sizes (K <= 2 also: max/average), whichever kernels run it.
+size_t sweep_bytes(int B, int H1, int W1, int H2, int W2, int C, int K) {
+    const size_t plain = fwd_split_bytes(B, H1, W1, H2, W2, K);
+    const size_t ma = split_sweep_bytes(B, H1 * W1, &H2, &W2, 1, C, SPLIT_ARGMAX, 0);
+    const size_t wt = split_sweep_bytes(B, H1 * W1, &H2, &W2, 1, C, SPLIT_WEIGHTED, K < KCH ? K : KCH);
+    return std::max(plain, std::max(ma, wt));
+}
+
+// What a forward entry point insists on when it is given a workspace: nothing where whole tiles fill the chip.
+size_t fwd_need(int B, int H1, int W1, int H2, int W2, int C, int K) {
+    return fwd_split_bytes(B, H1, W1, H2, W2, K) > 0 ? sweep_bytes(B, H1, W1, H2, W2, C, K) : 0;
+}
+
 }  // namespace
 namespace sepcorr_impl {
+// The sweep on the 16-bit matrix units (split_sweep.hip), where it takes the sizes: 0 launched, 1 not taken, negative on
+// error.  A caller who gives no scratch, or less than it takes, gets the same sweep, its scratch from the stream's memory pool for the length of
+// the call, so that the results do not depend on the workspace; the fp32 sweep runs where nothing may be allocated (under
+// stream capture too) or the pool has nothing left.
+template <int MODE, int KC>
+int try_split(const FwdArgs &a, int B, hipStream_t s) {
+    if (a.f2_planes) return 1;
+    SplitArgs p;
+    memset(&p, 0, sizeof(p));
+    p.f1 = a.f1; p.B = B; p.N1 = a.N1; p.C = a.C; p.KT = a.KT; p.k0 = a.k0; p.logits = a.logits; p.dlog = a.dlog;
+    p.nlev = a.nlev > 1 ? a.nlev : 1;
+    for (int l = 0; l < p.nlev; ++l) {
+        SplitLevel &L = p.lev[l];
+        const FwdLevel &F = a.lev[l];
+        L.f2 = F.f2; L.wv = F.wv; L.wu = F.wu; L.out_u = F.out_u; L.out_v = F.out_v; L.am_u = F.am_u; L.am_v = F.am_v;
+        L.st_wv = F.st_wv; L.st_wu = F.st_wu; L.z_ou = F.z_ou; L.st_ou = F.st_ou; L.dot_ou = F.dot_ou;
+        L.z_ov = F.z_ov; L.st_ov = F.st_ov; L.dot_ov = F.dot_ov;
+        L.H2 = F.H2; L.W2 = F.W2;
+    }
+    constexpr int mode = is_weighted(MODE) ? SPLIT_WEIGHTED : MODE == MODE_ARGMAX ? SPLIT_ARGMAX : SPLIT_MAXAVG;
+    constexpr int kc = is_weighted(MODE) ? KC : 0;
+    ProfScope ps(p.nlev > 1 ? (kc ? "fwd_weighted_levels" : "fwd_maxavg_levels") : (kc ? "fwd_weighted" : "fwd_maxavg"), s);
+    int rc = a.ws != nullptr ? split_sweep(mode, kc, p, a.ws, a.ws_bytes, s) : 1;
+    if (rc == 1 && !t_no_alloc) {
+        int h2[4], w2[4];
+        for (int l = 0; l < p.nlev; ++l) { h2[l] = p.lev[l].H2; w2[l] = p.lev[l].W2; }
+        const size_t bytes = split_sweep_bytes(B, a.N1, h2, w2, p.nlev, a.C, mode, kc);
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        void *ws = nullptr;
+        if (bytes > 0 && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
+            hipMallocAsync(&ws, bytes, s) == hipSuccess) {
+            rc = split_sweep(mode, kc, p, ws, bytes, s);
+            (void)hipFreeAsync(ws, s);
+        } else {
+            (void)hipGetLastError();
+        }
+    }
+    if (rc == 1) ps.on = false;   // (the sweep that runs instead has a bracket of its own)
+    return rc;
+}
+
 template <int MODE, int KC, int UR>
 int launch_fwd(FwdArgs a, int B, hipStream_t s) {
+    {   // the kernels read the level's pointers and sizes from lev[0]
+        FwdLevel &L = a.lev[0];
+        L.f2 = a.f2; L.wv = a.wv; L.wu = a.wu; L.out_u = a.out_u; L.out_v = a.out_v; L.am_u = a.am_u; L.am_v = a.am_v;
+        L.st_wv = a.st_wv; L.st_wu = a.st_wu; L.z_ou = a.z_ou; L.st_ou = a.st_ou; L.dot_ou = a.dot_ou;
+        L.z_ov = a.z_ov; L.st_ov = a.st_ov; L.dot_ov = a.dot_ov;
+        L.H2 = a.H2; L.W2 = a.W2;
+    }
+    if (const int rc = try_split<MODE, KC>(a, B, s); rc <= 0) return rc;
     constexpr int NPART = (is_weighted(MODE)) ? KC : 3;
     const bool may_deal = a.ws != nullptr && !a.f2_planes;
     WaveGrid wg;
@@ -3155,13 +3218,8 @@ int launch_fwd(FwdArgs a, int B, hipStream_t s) {
     if (!shape(may_deal) && may_deal) shape(false);
     a.nvc = wg.nvc;
     a.vpasses = wg.vpasses;
-    {   // the kernel reads the level's pointers and sizes from lev[0]
-        FwdLevel &L = a.lev[0];
-        L.f2 = a.f2; L.wv = a.wv; L.wu = a.wu; L.out_u = a.out_u; L.out_v = a.out_v; L.am_u = a.am_u; L.am_v = a.am_v;
-        L.st_wv = a.st_wv; L.st_wu = a.st_wu; L.z_ou = a.z_ou; L.st_ou = a.st_ou; L.dot_ou = a.dot_ou;
-        L.z_ov = a.z_ov; L.st_ov = a.st_ov; L.dot_ov = a.dot_ov;
-        L.H2 = a.H2; L.W2 = a.W2; L.nvc = a.nvc; L.stage = a.stage;
-    }
+    a.lev[0].nvc = a.nvc;
+    a.lev[0].stage = a.stage;
     dim3 grid(B * a.tiles_per_batch);
     const dim3 block(64 * nW);
     a.sk_total = 0;
@@ -3230,7 +3288,9 @@ int launch_fwd_levels(FwdArgs a, int B, hipStream_t s) {
     constexpr int NPART = is_weighted(MODE) ? KC : 3;
     constexpr int NCHO = is_weighted(MODE) ? KC : 2;
     constexpr int nW = 4;
-    if (a.nlev < 2 || a.nlev > 4 || a.ws == nullptr || a.C % 32 != 0) return SEPCORR_EINVAL;
+    if (a.nlev < 2 || a.nlev > 4) return SEPCORR_EINVAL;
+    if (const int rc = try_split<MODE, KC>(a, B, s); rc <= 0) return rc;
+    if (a.ws == nullptr || a.C % 32 != 0) return SEPCORR_EINVAL;
     int steps = 0, h2max = 0, w2max = 0;
     for (int l = 0; l < a.nlev; ++l) {
         FwdLevel &L = a.lev[l];
@@ -3591,7 +3651,7 @@ struct BwdWs {
 BwdWs bwd_ws(const Dims &d) {
     BwdWs w;
     const size_t part = df2_part_bytes(d), uwt = df1_uwt_bytes(d), sk = df1_shape(d).bytes;
-    w.fwd_bytes = fwd_split_bytes(d.B, d.H1, d.W1, d.H2, d.W2, MAX_K);
+    w.fwd_bytes = sweep_bytes(d.B, d.H1, d.W1, d.H2, d.W2, d.C, MAX_K);
     w.aliased = sk > 0 || w.fwd_bytes > 0;
     if (w.aliased) {
         w.off_uwt = 0;
@@ -3948,7 +4008,7 @@ int check_workspace(const Dims &d, void *ws, size_t ws_bytes) {
 // Scratch of a forward-type sweep is optional: without it every workgroup takes a whole pixel tile.
 int check_fwd_workspace(const Dims &d, int K, void *ws, size_t ws_bytes) {
     if (ws == nullptr) return SEPCORR_OK;
-    const size_t need = fwd_split_bytes(d.B, d.H1, d.W1, d.H2, d.W2, K);
+    const size_t need = fwd_need(d.B, d.H1, d.W1, d.H2, d.W2, d.C, K);
     if (ws_bytes < need)
         return fail(SEPCORR_EWORKSPACE, "sepcorr: forward workspace of %zu bytes given, %zu needed (or pass NULL)", ws_bytes, need);
     if (reinterpret_cast<uintptr_t>(ws) & 255) return fail(SEPCORR_EWORKSPACE, "sepcorr: workspace must be 256-byte aligned");
@@ -4066,7 +4126,7 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap) {
 
 size_t sepcorr_forward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C, int K) {
     if (B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1 || K < 1) return 0;
-    return fwd_split_bytes(B, H1, W1, H2, W2, K);
+    return fwd_need(B, H1, W1, H2, W2, C, K);
 }
 
 int sepcorr_max_avg_forward(const float *f1, const float *f2, float *out_u, float *out_v, int B, int H1, int W1, int H2,
@@ -4254,7 +4314,7 @@ size_t sepcorr_compression_backward_from_logits_workspace_bytes(int B, int H1, i
     const Dims d = {B, H1, W1, H2, W2, C};
     const size_t rows = (size_t)B * H1 * W1 * K;
     const size_t dots = 2 * ((rows * sizeof(float) + 255) & ~(size_t)255);
-    if (!with_features) return ((fwd_split_bytes(B, H1, W1, H2, W2, K) + 255) & ~(size_t)255) + dots;
+    if (!with_features) return ((sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255) + dots;
     const size_t a_bytes = ((rows * W2 * sizeof(float) + 255) & ~(size_t)255) + ((rows * H2 * sizeof(float) + 255) & ~(size_t)255);
     return bwd_ws(d).total + dots + a_bytes;
 }
@@ -4279,10 +4339,10 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t rows = (size_t)B * H1 * W1 * K;
     const size_t dot_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
-    const size_t sweep_bytes = d_f1 ? bwd_ws(d).total : (fwd_split_bytes(B, H1, W1, H2, W2, K) + 255) & ~(size_t)255;
+    const size_t own_bytes = d_f1 ? bwd_ws(d).total : (sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255;
     char *base = static_cast<char *>(workspace);
-    float *dot_u = reinterpret_cast<float *>(base + sweep_bytes);               // sum_u g_cu * comp_u = sum_v a_u * d_a_u
-    float *dot_v = reinterpret_cast<float *>(base + sweep_bytes + dot_bytes);   // sum_v g_cv * comp_v = sum_u a_v * d_a_v
+    float *dot_u = reinterpret_cast<float *>(base + own_bytes);               // sum_u g_cu * comp_u = sum_v a_u * d_a_u
+    float *dot_v = reinterpret_cast<float *>(base + own_bytes + dot_bytes);   // sum_v g_cv * comp_v = sum_u a_v * d_a_v
     {
         const dim3 grid(row_groups(rows)), block(256);
         ProfScope ps("row_dots", s);
@@ -4297,12 +4357,12 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     soft.dlog = 1;
     soft.z_ou = logits_v; soft.st_ou = stats_v; soft.dot_ou = dot_v;
     soft.z_ov = logits_u; soft.st_ov = stats_u; soft.dot_ov = dot_u;
-    const size_t fwd_bytes = fwd_split_bytes(B, H1, W1, H2, W2, d_f1 ? MAX_K : K);
+    const size_t fwd_bytes = sweep_bytes(B, H1, W1, H2, W2, C, d_f1 ? MAX_K : K);
     int rc = weighted_forward(d, f1, f2, g_cv, g_cu, d_logits_v, d_logits_u, K, fwd_bytes ? workspace : nullptr, fwd_bytes, s, &soft);
     if (rc || d_f1 == nullptr) return rc;
     // feature gradients: the weights themselves, formed once from logits and statistics behind the other scratch
-    float *a_u = reinterpret_cast<float *>(base + sweep_bytes + 2 * dot_bytes);
-    float *a_v = reinterpret_cast<float *>(base + sweep_bytes + 2 * dot_bytes + ((rows * W2 * sizeof(float) + 255) & ~(size_t)255));
+    float *a_u = reinterpret_cast<float *>(base + own_bytes + 2 * dot_bytes);
+    float *a_v = reinterpret_cast<float *>(base + own_bytes + 2 * dot_bytes + ((rows * W2 * sizeof(float) + 255) & ~(size_t)255));
     {
         const dim3 grid(row_groups(rows)), block(256);
         ProfScope ps("softmax_apply", s);
@@ -4352,16 +4412,19 @@ int check_levels(const int *h2, const int *w2, int nlev, int B, int H1, int W1, 
     }
     return SEPCORR_OK;
 }
-size_t levels_sweep_bytes(const int *h2, const int *w2, int nlev, int B, int H1, int W1, int K) {
+size_t levels_sweep_bytes(const int *h2, const int *w2, int nlev, int B, int H1, int W1, int C, int K) {
     int w2max = 0;
     size_t single = 0;
     for (int l = 0; l < nlev; ++l) {
         if (w2[l] > w2max) w2max = w2[l];
-        const size_t n = fwd_split_bytes(B, H1, W1, h2[l], w2[l], K);
+        const size_t n = sweep_bytes(B, H1, W1, h2[l], w2[l], C, K);   // (level by level, where one launch cannot take them all)
         if (n > single) single = n;
     }
     const size_t multi = fwd_levels_bytes(B * ((H1 * W1 + TP - 1) / TP), nlev, w2max, K);
-    return ((multi > single ? multi : single) + 255) & ~(size_t)255;
+    size_t n = std::max(multi, single);
+    n = std::max(n, split_sweep_bytes(B, H1 * W1, h2, w2, nlev, C, SPLIT_ARGMAX, 0));
+    n = std::max(n, split_sweep_bytes(B, H1 * W1, h2, w2, nlev, C, SPLIT_WEIGHTED, K < KCH ? K : KCH));
+    return (n + 255) & ~(size_t)255;
 }
 }  // namespace
 
@@ -4370,7 +4433,7 @@ size_t sepcorr_forward_levels_workspace_bytes(const int *h2, const int *w2, int 
     for (int l = 0; l < nlev; ++l)
         if (h2[l] < 1 || w2[l] < 1) return 0;
     // + the row dot products of the backward call (two per level)
-    return levels_sweep_bytes(h2, w2, nlev, B, H1, W1, K) + 2 * (size_t)nlev * ((((size_t)B * H1 * W1 * K * sizeof(float)) + 255) & ~(size_t)255);
+    return levels_sweep_bytes(h2, w2, nlev, B, H1, W1, C, K) + 2 * (size_t)nlev * ((((size_t)B * H1 * W1 * K * sizeof(float)) + 255) & ~(size_t)255);
 }
 
 int sepcorr_max_argmax_avg_forward_levels(const float *f1, const float *const *f2_levels, const int *h2, const int *w2, int nlev,
@@ -4384,7 +4447,7 @@ int sepcorr_max_argmax_avg_forward_levels(const float *f1, const float *const *f
     for (int l = 0; l < nlev; ++l)
         if (!f2_levels[l] || !out_u[l] || !out_v[l] || !argmax_u[l] || !argmax_v[l])
             return fail(SEPCORR_EINVAL, "sepcorr: a pointer of level %d is NULL", l);
-    const size_t need = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, 2);
+    const size_t need = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, C, 2);
     if (workspace != nullptr && (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255)))
         return fail(SEPCORR_EWORKSPACE, "sepcorr: %zu bytes of 256-byte aligned workspace needed (or NULL), got %zu", need, workspace_bytes);
     hipStream_t s = static_cast<hipStream_t>(stream);
@@ -4442,7 +4505,7 @@ int soft_levels(const float *f1, const float *const *f2, const int *h2, const in
         soft.st_wv = lev[l].st_wv; soft.st_wu = lev[l].st_wu;
         soft.z_ou = lev[l].z_ou; soft.st_ou = lev[l].st_ou; soft.dot_ou = lev[l].dot_ou;
         soft.z_ov = lev[l].z_ov; soft.st_ov = lev[l].st_ov; soft.dot_ov = lev[l].dot_ov;
-        const size_t n = fwd_split_bytes(B, H1, W1, h2[l], w2[l], K);
+        const size_t n = sweep_bytes(B, H1, W1, h2[l], w2[l], C, K);
         if (int rc = weighted_forward(d, f1, f2[l], lev[l].wv, lev[l].wu, lev[l].out_u, lev[l].out_v, K, n && ws ? ws : nullptr, n, s, &soft))
             return rc;
     }
@@ -4460,7 +4523,7 @@ int sepcorr_compression_forward_from_logits_levels(const float *f1, const float 
     REQUIRE_PTR(comp_u); REQUIRE_PTR(comp_v);
     LevelDims ld;
     if (int rc = check_levels(h2, w2, nlev, B, H1, W1, C, K, &ld)) return rc;
-    const size_t need = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, K);
+    const size_t need = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, C, K);
     if (workspace != nullptr && (workspace_bytes < need || (reinterpret_cast<uintptr_t>(workspace) & 255)))
         return fail(SEPCORR_EWORKSPACE, "sepcorr: %zu bytes of 256-byte aligned workspace needed (or NULL), got %zu", need, workspace_bytes);
     FwdLevel lev[4];
@@ -4491,7 +4554,7 @@ int sepcorr_compression_backward_from_logits_levels(const float *f1, const float
         return fail(SEPCORR_EWORKSPACE, "sepcorr: %zu bytes of 256-byte aligned workspace needed, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t sweep = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, K);
+    const size_t sweep = levels_sweep_bytes(h2, w2, nlev, B, H1, W1, C, K);
     const size_t rows = (size_t)B * H1 * W1 * K;
     const size_t dot_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
     char *base = static_cast<char *>(workspace) + sweep;

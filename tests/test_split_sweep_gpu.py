@@ -1,0 +1,121 @@
+"""Forward-type sweeps whose operands are split into two 16-bit halves (csrc/split_sweep.hip) against float64.
+
+Sizes at the edges of its tiles: pixels around multiples of 128, columns around multiples of 32, channels around the
+16/64/128/256 its channel steps are padded to, and pixels it cannot split (inf, NaN, magnitudes outside [2^-24, 2^24)),
+which it multiplies in fp32.
+"""
+import pytest
+import torch
+
+from separableflowthesis_amd import _lib
+from tests._util import op_inputs
+
+pytestmark = pytest.mark.gpu
+
+# (B, H1, W1, H2, W2, C); all large enough for the split sweep (at least 256 steps of 128 pixels x 32 columns)
+SHAPES = [(1, 25, 41, 37, 33, 32), (2, 16, 40, 30, 64, 33), (1, 43, 48, 23, 65, 64), (1, 23, 50, 31, 31, 65),
+          (1, 18, 36, 29, 70, 128), (3, 9, 43, 40, 36, 130), (1, 31, 33, 36, 32, 255), (2, 24, 37, 26, 97, 256),
+          (1, 32, 128, 9, 1, 96), (1, 12, 24, 11, 290, 48)]
+
+
+def _call(name, outs, ins, dims, scratch, extra=(), K=2):
+    lib = _lib.load()
+    n = lib.sepcorr_forward_workspace_bytes(*dims, K) if scratch else 0
+    ws = torch.empty(max(n, 256), dtype=torch.uint8, device=ins[0].device)
+    _lib.check(getattr(lib, name)(*(t.data_ptr() for t in ins), *(t.data_ptr() for t in outs), *dims, *extra,
+                                  ws.data_ptr() if n else None, n, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+
+
+def _max_avg(f1, f2, dims, scratch=True, argmax=True):
+    B, H1, W1, H2, W2, C = dims
+    e = lambda *s, **k: torch.empty(*s, device=f1.device, **k)
+    outs = [e(B, H1, W1, 2, H2), e(B, H1, W1, 2, W2)]
+    if argmax:
+        outs += [e(B, H1, W1, 1, H2, dtype=torch.int32), e(B, H1, W1, 1, W2, dtype=torch.int32)]
+    _call("sepcorr_max_argmax_avg_forward" if argmax else "sepcorr_max_avg_forward", outs, [f1, f2], dims, scratch)
+    return outs
+
+
+def _volume(f1, f2):
+    B, H1, W1, C = f1.shape
+    return (f1.reshape(B, H1 * W1, C) @ f2.reshape(B, -1, C).transpose(1, 2).contiguous()).view(B, H1, W1, *f2.shape[1:3])
+
+
+def _bound(f1, f2, extra=0):
+    """Largest error of one product sum: 2^-21 of sum |a b| for what the halves do not hold, and one rounding of at most
+    2^-24 of it per addition (three products per channel, `extra` additions of the reduction behind it)."""
+    C = f1.shape[-1]
+    return (8 + 3 * C + extra + 8) * 2.0 ** -24 * _volume(f1.double().abs(), f2.double().abs())
+
+
+@pytest.mark.parametrize("dims", SHAPES, ids=str)
+def test_max_argmax_avg(device, dims):
+    f1, f2, _ = op_inputs(*dims, seed=5)
+    vol, err = _volume(f1.double(), f2.double()), _bound(f1, f2, sum(dims[3:5]))
+    out_u, out_v, am_u, am_v = (t.cpu() for t in _max_avg(f1.to(device), f2.to(device), dims))
+    for out, am, d in ((out_u, am_u, 4), (out_v, am_v, 3)):
+        worst = err.amax(d)
+        assert ((out[:, :, :, 0] - vol.amax(d)).abs() <= worst).all()
+        assert ((out[:, :, :, 1] - vol.mean(d)).abs() <= err.mean(d)).all()
+        # the index points at a value that is the maximum but for the rounding of both
+        at = vol.gather(d, am[:, :, :, 0].long().unsqueeze(d)).squeeze(d)
+        assert (vol.amax(d) - at <= 2 * worst).all()
+    plain = _max_avg(f1.to(device), f2.to(device), dims, argmax=False)
+    assert torch.equal(plain[0].cpu(), out_u) and torch.equal(plain[1].cpu(), out_v)
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5])
+@pytest.mark.parametrize("dims", SHAPES[1::2], ids=str)
+def test_weighted(device, dims, K):
+    B, H1, W1, H2, W2, C = dims
+    f1, f2, g = op_inputs(*dims, seed=6)
+    a_u, a_v = torch.randn(B, H1, W1, K, W2, generator=g), torch.randn(B, H1, W1, K, H2, generator=g)
+    outs = [torch.empty(B, H1, W1, K, H2, device=device), torch.empty(B, H1, W1, K, W2, device=device)]
+    _call("sepcorr_compression_forward", outs, [t.to(device) for t in (f1, f2, a_u, a_v)], dims, True, (K,), K)
+    vol, err = _volume(f1.double(), f2.double()), _bound(f1, f2, H2 + W2 + 2)
+    for k in range(K):
+        wu, wv = a_u[:, :, :, k, None, :].double(), a_v[:, :, :, k, :, None].double()
+        assert ((outs[0][:, :, :, k].cpu() - (vol * wu).sum(4)).abs() <= (err * wu.abs()).sum(4)).all()
+        assert ((outs[1][:, :, :, k].cpu() - (vol * wv).sum(3)).abs() <= (err * wv.abs()).sum(3)).all()
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 2.0 ** 30, 2.0 ** -30, 0.0])
+@pytest.mark.parametrize("where", ["f1", "f2", "both"])
+def test_pixels_without_halves(device, value, where):
+    dims = (1, 25, 41, 37, 40, 48)
+    f1, f2, _ = op_inputs(*dims, seed=7)
+    if where != "f2":
+        f1[0, 3, 7] = value if abs(value) < 1 else f1[0, 3, 7]   # a whole tiny (or zero) pixel, or one large channel
+        f1[0, 3, 7, 11] = value
+    if where != "f1":
+        f2[0, 30, 39] = value if abs(value) < 1 else f2[0, 30, 39]
+        f2[0, 30, 39, 11] = value
+    got = [t.cpu() for t in _max_avg(f1.to(device), f2.to(device), dims)]
+    vol = torch.einsum("bijc,buvc->bijuv", f1.double(), f2.double())
+    scale = max(1.0, abs(value) ** 2) if abs(value) < float("inf") else 1.0
+    for out, am, d in ((got[0], got[2], 4), (got[1], got[3], 3)):
+        best = vol.nan_to_num(nan=-float("inf"), posinf=float("inf"), neginf=-float("inf")).amax(d)   # (NaN never wins)
+        assert torch.allclose(out[:, :, :, 0].double(), best, rtol=1e-5, atol=1e-5 * scale)
+        assert torch.allclose(out[:, :, :, 1].double(), vol.mean(d), rtol=1e-5, atol=1e-5 * scale, equal_nan=True)
+        at = vol.gather(d, am[:, :, :, 0].long().unsqueeze(d)).squeeze(d)
+        assert ((best - at).abs() <= 1e-5 * scale)[best.isfinite()].all()
+
+
+def test_without_scratch_the_same_bits(device):
+    dims = SHAPES[7]
+    f1, f2, _ = op_inputs(*dims, seed=9)
+    for a, b in zip(_max_avg(f1.to(device), f2.to(device), dims), _max_avg(f1.to(device), f2.to(device), dims, scratch=False)):
+        assert torch.equal(a, b)
+
+
+def test_small_features_keep_their_accuracy(device):
+    """Every pixel has a scale of its own: features of 1e-6 beside features of 1e6 lose nothing."""
+    dims = (1, 24, 48, 30, 64, 64)
+    f1, f2, g = op_inputs(*dims, seed=8)
+    f1 *= 10.0 ** torch.randint(-6, 7, f1.shape[:3] + (1,), generator=g)
+    f2 *= 10.0 ** torch.randint(-6, 7, f2.shape[:3] + (1,), generator=g)
+    vol, err = _volume(f1.double(), f2.double()), _bound(f1, f2, sum(dims[3:5]))
+    out_u, out_v = (t.cpu() for t in _max_avg(f1.to(device), f2.to(device), dims)[:2])
+    assert ((out_u[:, :, :, 0] - vol.amax(4)).abs() <= err.amax(4)).all()
+    assert ((out_v[:, :, :, 1] - vol.mean(3)).abs() <= err.mean(3)).all()
