@@ -25,8 +25,8 @@
  *  - Backward entry points need scratch memory: query sepcorr_backward_workspace_bytes() and pass a
  *    device buffer of at least that size (256-byte aligned).  Its contents on entry are ignored.
  *  - Forward entry points take scratch memory optionally (sepcorr_forward_workspace_bytes(), 256-byte aligned,
- *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels and at least 256 steps (128
- *    pixels of image 1 x 32 columns of a row of image 2) run on the 16-bit matrix units, every fp32 operand as two
+ *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels with
+ *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units, every fp32 operand as two
  *    halves with a power-of-two scale per pixel, at the accuracy of fp32 products (csrc/split_sweep.hip); without a
  *    workspace (or with one smaller than sepcorr_forward_levels_workspace_bytes() of the one level) they take their
  *    scratch from the stream's memory pool, which costs host time on each call.  The other sizes, and calls without a workspace

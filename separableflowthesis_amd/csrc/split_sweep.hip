@@ -744,15 +744,22 @@ SplitPlan plan(int B, int N1, const int *h2, const int *w2, int nlev, int C, int
     p.q = mode == SPLIT_WEIGHTED ? kc : mode == SPLIT_ARGMAX ? 3 : 2;
     p.npt = (N1 + TPX - 1) / TPX;
     long blocks = 0;
-    for (int l = 0; l < nlev; ++l) blocks += (long)B * ((w2[l] + 31) / 32) * h2[l];
+    double pairs = 0;
+    for (int l = 0; l < nlev; ++l) {
+        blocks += (long)B * ((w2[l] + 31) / 32) * h2[l];
+        pairs += (double)B * N1 * h2[l] * w2[l];
+    }
     const size_t per_pt = (size_t)blocks * p.q * TPX * sizeof(float);
     long fit = (long)(kPartLimit / per_pt);
     if (fit < 1) fit = 1;
     p.slabs = (int)((p.npt + fit - 1) / fit);
     p.npt_slab = (p.npt + p.slabs - 1) / p.slabs;
     const long steps = blocks * p.npt_slab;
-    // with fewer steps than compute units (B=1, 24x32: 144) the fp32 sweep's two launches are as fast as the three here
-    if (steps < kPlaces) return p;
+    // The three launches and the hand-over through scratch take 26 us at the least, the fp32 sweep two launches and its
+    // matrix work.  Measured (fp32 sweep / this one, max/average): B=1, 24x64, C=256 37.5 / 33.2 us, B=4, 20x40 37.6 /
+    // 38.6, B=2, 32x64 54 / 39; C=72 24x64 28.0 / 27.8, B=2, 32x64 34.6 / 29.2; C=32 B=2, 32x64 29.8 / 29.0, 47x90 52 / 40:
+    // the line lies where pairs (C + 64) reach 1e9 (3.1 million pairs at C=256, 10 million at C=32).
+    if (pairs * (C + 64) < 1e9) return p;
     for (int l = 0; l < nlev; ++l)
         if ((size_t)h2[l] * block_bytes(p.nk) >= (1u << 30)) return p;
     if (steps > (1L << 30) || blocks > (1L << 24)) return p;

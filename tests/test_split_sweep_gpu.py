@@ -4,6 +4,8 @@ Sizes at the edges of its tiles: pixels around multiples of 128, columns around 
 16/64/128/256 its channel steps are padded to, and pixels it cannot split (inf, NaN, magnitudes outside [2^-24, 2^24)),
 which it multiplies in fp32.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -12,15 +14,21 @@ from tests._util import op_inputs
 
 pytestmark = pytest.mark.gpu
 
-# (B, H1, W1, H2, W2, C); all large enough for the split sweep (at least 256 steps of 128 pixels x 32 columns)
-SHAPES = [(1, 25, 41, 37, 33, 32), (2, 16, 40, 30, 64, 33), (1, 43, 48, 23, 65, 64), (1, 23, 50, 31, 31, 65),
-          (1, 18, 36, 29, 70, 128), (3, 9, 43, 40, 36, 130), (1, 31, 33, 36, 32, 255), (2, 24, 37, 26, 97, 256),
-          (1, 32, 128, 9, 1, 96), (1, 12, 24, 11, 290, 48)]
+# (B, H1, W1, H2, W2, C); all large enough for the split sweep: B H1 W1 H2 W2 (C + 64) of 1e9 and a little more
+SHAPES = [(1, 50, 82, 74, 35, 32), (2, 40, 64, 61, 34, 33), (1, 63, 65, 33, 65, 64), (1, 51, 91, 62, 31, 65),
+          (1, 36, 73, 33, 70, 128), (3, 21, 43, 55, 36, 130), (1, 47, 48, 42, 35, 255), (2, 24, 49, 27, 97, 256),
+          (1, 96, 172, 401, 1, 96), (1, 48, 65, 11, 290, 48)]
+
+
+def test_sizes_take_the_split_sweep():
+    for B, H1, W1, H2, W2, C in SHAPES:
+        assert B * H1 * W1 * H2 * W2 * (C + 64) >= 1e9
 
 
 def _call(name, outs, ins, dims, scratch, extra=(), K=2):
     lib = _lib.load()
-    n = lib.sepcorr_forward_workspace_bytes(*dims, K) if scratch else 0
+    h2, w2 = (ctypes.c_int * 1)(dims[3]), (ctypes.c_int * 1)(dims[4])
+    n = lib.sepcorr_forward_levels_workspace_bytes(h2, w2, 1, *dims[:3], dims[5], K) if scratch else 0
     ws = torch.empty(max(n, 256), dtype=torch.uint8, device=ins[0].device)
     _lib.check(getattr(lib, name)(*(t.data_ptr() for t in ins), *(t.data_ptr() for t in outs), *dims, *extra,
                                   ws.data_ptr() if n else None, n, torch.cuda.current_stream().cuda_stream))
@@ -83,7 +91,7 @@ def test_weighted(device, dims, K):
 @pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan"), 2.0 ** 30, 2.0 ** -30, 0.0])
 @pytest.mark.parametrize("where", ["f1", "f2", "both"])
 def test_pixels_without_halves(device, value, where):
-    dims = (1, 25, 41, 37, 40, 48)
+    dims = (1, 50, 81, 62, 40, 48)
     f1, f2, _ = op_inputs(*dims, seed=7)
     if where != "f2":
         f1[0, 3, 7] = value if abs(value) < 1 else f1[0, 3, 7]   # a whole tiny (or zero) pixel, or one large channel
@@ -111,7 +119,7 @@ def test_without_scratch_the_same_bits(device):
 
 def test_small_features_keep_their_accuracy(device):
     """Every pixel has a scale of its own: features of 1e-6 beside features of 1e6 lose nothing."""
-    dims = (1, 24, 48, 30, 64, 64)
+    dims = (1, 48, 96, 30, 64, 64)
     f1, f2, g = op_inputs(*dims, seed=8)
     f1 *= 10.0 ** torch.randint(-6, 7, f1.shape[:3] + (1,), generator=g)
     f2 *= 10.0 ** torch.randint(-6, 7, f2.shape[:3] + (1,), generator=g)
