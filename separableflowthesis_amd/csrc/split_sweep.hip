@@ -325,25 +325,26 @@ __global__ void __launch_bounds__(256) split_finish_kernel(const SplitArgs a) {
 }
 #endif
 
-// Up to two weight channels (and the max/avg modes) fit 256 registers: two workgroups per compute unit, one wave's
-// reductions run beside the other's matrix work.  Three and four channels take the whole register file, and a wave reduces
-// one row while it multiplies the next.  (All modes the second way, B=2, 55x128: max/avg 0.175 instead of 0.162 ms.)
-__host__ __device__ constexpr bool pipelined(int mode, int kc) { return mode == SPLIT_WEIGHTED && kc > 2; }
+// The max/avg modes and one weight channel fit 256 registers: two workgroups per compute unit, one wave's reductions run
+// beside the other's matrix work.  More channels take the whole register file, and a wave reduces one row while it
+// multiplies the next.  Both ways measured at C=256: max/avg, B=2, 55x128 0.149 ms with two workgroups and 0.166 with one;
+// two channels over the four levels of 47x156 0.225 and 0.212.
+__host__ __device__ constexpr bool pipelined(int mode, int kc) { return mode == SPLIT_WEIGHTED && kc > 1; }
 
 // NK: channel steps of 16 (C <= 16 NK, the rest zeros).  Measured at B=2, 55x128, C=256: max/avg/argmax 0.454 ms with the
-// fp32 sweep, 0.162 ms here (+ 0.013 split_prepare_kernel, 0.032 split_finish_kernel); four weighted sums 0.474 and
-// 0.203 ms (+ 0.013 and 0.034).  The matrix instructions alone take 0.061 ms at 2.4 GHz; what is left is the vector work
-// of the reductions, the reads of the row block from LDS and the barrier of every step.
+// fp32 sweep, 0.149 ms here (+ 0.013 split_prepare_kernel, 0.032 split_finish_kernel); four weighted sums 0.474 and
+// 0.192 ms (+ 0.013 and 0.034).  The matrix instructions alone take 0.061 ms at 2.4 GHz; what is left is the vector work
+// of the reductions, the reads of the row block from LDS and the beginning and end of every step.
 template <int MODE, int KC, int NK>
 __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_kernel(const SplitArgs a) {
     constexpr bool WT = MODE == SPLIT_WEIGHTED;
     constexpr bool PIPE = pipelined(MODE, KC);
     constexpr int Q = WT ? KC : (MODE == SPLIT_ARGMAX ? 3 : 2);
-    constexpr int BLK = block_bytes(NK), BF = BLK / 4;
-    extern __shared__ float smem[];                       // two row blocks, then the u-indexed weights of each wave
+    constexpr int BLK = block_bytes(NK), BF = BLK / 4, NBUF = PIPE ? 3 : 2;
+    extern __shared__ float smem[];                       // NBUF row blocks, then the u-indexed weights of each wave
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, pl = lane & 31, h = lane >> 5;
-    float *wus = smem + 2 * BF + wave * (KC * 128);       // [k][row & 3][pixel]
+    float *wus = smem + NBUF * BF + wave * (KC * 128);       // [k][row & 3][pixel]
     const int wg = xcd_contiguous(blockIdx.x, gridDim.x);
     const long T = a.steps;
     const int g0 = (int)(wg * T / a.G), g1 = (int)((wg + 1) * T / a.G);
@@ -364,12 +365,16 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
         constexpr int NDMA = (2 * NK + 4) / 4;   // KBs of a row block per wave
         auto dma = [&](int u, int buf, int i) {
             const int kb = 4 * i + wave;
-            if (kb < 2 * NK + 1)
+            if (4 * i + 3 < 2 * NK + 1 || kb < 2 * NK + 1)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)(smem + buf * BF + kb * 256), 16,
                                                          lane * 16, u * BLK + kb * 1024, 0, 0);
         };
 #pragma unroll
         for (int i = 0; i < NDMA; ++i) dma(ua, 0, i);
+        if constexpr (PIPE) {
+#pragma unroll
+            for (int i = 0; i < NDMA; ++i) dma(ua + 1, 1, i);
+        }
         // Everything a piece begins with is requested before any of it is waited for (in turn it takes 10 us).
         float vmax[16], vsum[16], wvr[KC][16], rv[KC][16];   // running state over u, accumulator layout, in units of 1 / back
         int vidx[16];
@@ -562,12 +567,12 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
         // The products of a row block; `beside(s)` is what the vector units do beside the matrix work of channel step s.
         // Operands are read two channel steps before they are used.  The order is fixed here: left to itself the
         // compiler either reads everything at once (and spills) or waits for every read, and puts the vector work last.
-        // The next row is requested a KB at a time between the matrix instructions (all requests at once hold the wave up
-        // for 700 cycles; behind a piece's last row they fetch one that is not used, or zeros).  The factors that scale
+        // Row `next` is requested into row block nbuf a KB at a time between the matrix instructions (all requests at once hold the wave up
+        // for 700 cycles; behind a piece's last row they fetch what follows it in the scratch, which is not used).  The factors that scale
         // row u back are in `fac` at the end and the block's mark in `mark`.
         v4f fac[4];
         int mark = 0;
-        auto multiply = [&](int u, int buf, auto beside) {
+        auto multiply = [&](int next, int buf, int nbuf, auto beside) {
             const char *blk = reinterpret_cast<const char *>(smem + buf * BF) + lane * 16;
             const float *tail = smem + buf * BF + 2 * NK * 256;
             v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
@@ -588,7 +593,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                     mark = __float_as_int(tail[MARK]);
                 }
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s % 3], fh[s], acc, 0, 0, 0);
-                if (s < NDMA) dma(u + 1, buf ^ 1, s);
+                if (s < NDMA) dma(next, nbuf, s);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s % 3], fl[s], acc, 0, 0, 0);
                 acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s % 3], fh[s], acc, 0, 0, 0);
                 beside(s);
@@ -624,21 +629,27 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
         // (edge: the chunk has columns beyond the image, which the maxima over a row leave out)
         auto sweep = [&](auto edge) {
             if constexpr (PIPE) {
-                scale_back(multiply(ua, 0, nothing), x);
+                // Rows are requested two steps ahead, into three blocks: a step (1600 cycles and more) is too short for
+                // what the last requests of the step before take.  At the end of a step all but this step's requests
+                // have to be there: of the wave's outstanding memory operations the latest 2 NK / 4 are among those.
+                auto step_end = [] { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NK / 2) : "memory"); };
+                scale_back(multiply(ua + 2, 0, 2, nothing), x);
                 if (marked()) multiply_fp32(ua, x);
-                __syncthreads();
+                step_end();
+                int buf = 1;
                 for (int u = ua + 1; u < ub; ++u) {
-                    const int buf = (u - ua) & 1;
+                    const int nbuf = buf == 0 ? 2 : buf - 1;   // the block of row u - 1, which every wave is done with
                     if (u > ua + 1) flush();
                     begin(u - 1);
-                    const v16f acc = multiply(u, buf, [&](int s) {
+                    const v16f acc = multiply(u + 2, buf, nbuf, [&](int s) {
 #pragma unroll
                         for (int e = 0; e < PER; ++e) take(edge, PER * s + e, x[PER * s + e]);
                     });
                     finish();
                     scale_back(acc, x);
                     if (marked()) multiply_fp32(u, x);
-                    __syncthreads();
+                    step_end();
+                    buf = buf == 2 ? 0 : buf + 1;
                 }
                 if (ub > ua + 1) flush();
                 begin(ub - 1);
@@ -650,7 +661,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 for (int u = ua; u < ub; ++u) {
                     const int buf = (u - ua) & 1;
                     if (u > ua) flush();
-                    scale_back(multiply(u, buf, nothing), x);
+                    scale_back(multiply(u + 1, buf, buf ^ 1, nothing), x);
                     if (marked()) multiply_fp32(u, x);
                     begin(u);
 #pragma unroll
@@ -685,7 +696,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
 
 template <int MODE, int KC>
 int launch_sweep(const SplitArgs &a, int nk, hipStream_t s) {
-    const size_t lds = 2 * (size_t)block_bytes(nk) + (MODE == SPLIT_WEIGHTED ? 4 * KC * 128 * sizeof(float) : 0);
+    const size_t lds = (pipelined(MODE, KC) ? 3 : 2) * (size_t)block_bytes(nk) + (MODE == SPLIT_WEIGHTED ? 4 * KC * 128 * sizeof(float) : 0);
     auto k = nk == 4 ? split_sweep_kernel<MODE, KC, 4> : nk == 8 ? split_sweep_kernel<MODE, KC, 8> : split_sweep_kernel<MODE, KC, 16>;
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
