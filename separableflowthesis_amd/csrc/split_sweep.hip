@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
             for (int i = 0; i < NDMA; ++i) dma(ua + 1, 1, i);
         }
         // Everything a piece begins with is requested before any of it is waited for (in turn it takes 10 us).
-        float vmax[16], vsum[16], wvr[KC][16], rv[KC][16];   // running state over u, accumulator layout, in units of 1 / back
+        float vmax[16], vsum[16], wvr[KC][16], rv[KC][16];   // running state over u, accumulator layout
         int vidx[16];
         float wpre[KC][2], wm[KC], wil[KC], vm[KC], vil[KC];
         if constexpr (WT) {
@@ -475,7 +475,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
             if (PIPE) asm volatile("" : "+a"(fl[s]));
         }
         float *part = L.part + (((size_t)bc * H2) * Q) * N1p + pt * TPX + 32 * wave + pl;
-        // What a lane holds of a row, scaled back for fmap2's pixels, goes into the running state and into out_u's parts:
+        // What a lane holds of a row, scaled back, goes into the running state and into out_u's parts:
         // begin(u), the registers one by one, finish(u).
         float red[KC], redw[KC], red_m = 0.f, red_s = 0.f;
         int red_i = 0, red_u = 0;
@@ -525,7 +525,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 for (int k = 0; k < KC; ++k) {
                     float lo, hi;
                     wave_halves(red[k], lo, hi);
-                    sk[k] = (lo + hi) * back;
+                    sk[k] = lo + hi;
                 }
 #pragma unroll
                 for (int k = 0; k < KC; k += 2)   // lanes of half 0 store the even channels, of half 1 the odd ones
@@ -543,10 +543,10 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                     float i_lo, i_hi;
                     wave_halves(__int_as_float(red_i), i_lo, i_hi);
                     const bool take_hi = m_hi > m_lo || (m_hi == m_lo && __float_as_int(i_hi) < __float_as_int(i_lo));
-                    pend[0] = h ? (take_hi ? i_hi : i_lo) : (take_hi ? m_hi : m_lo) * back;
-                    pend[Q - 2] = (s_lo + s_hi) * back;
+                    pend[0] = h ? (take_hi ? i_hi : i_lo) : (take_hi ? m_hi : m_lo);
+                    pend[Q - 2] = s_lo + s_hi;
                 } else {
-                    pend[0] = (h ? s_lo + s_hi : maxnum(m_lo, m_hi)) * back;
+                    pend[0] = h ? s_lo + s_hi : maxnum(m_lo, m_hi);
                 }
             }
         };
@@ -602,7 +602,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
             return acc;
         };
         constexpr int PER = 16 / NK;   // accumulator registers reduced beside one channel step
-        // a block with a marked pixel: fp32 products straight from the inputs, in the units of the others
+        // a block with a marked pixel: fp32 products straight from the inputs
         auto multiply_fp32 = [&](int u, float (&x)[16]) {
             const int v = 32 * vc + pl;
             const bool vok = v < W2;
@@ -612,16 +612,17 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
 #pragma unroll 1
             for (int c = h; c < C + h; c += 2)
                 acc = __builtin_amdgcn_mfma_f32_32x32x2f32((vok && c < C) ? q[c] : 0.f, (pok && c < C) ? f1p[c] : 0.f, acc, 0, 0, 0);
-            const float unit = pok ? 1.f / back : 0.f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] = 32 * vc + vmap(r, h) < W2 ? acc[r] * unit : 0.f;
+            for (int r = 0; r < 16; ++r) x[r] = 32 * vc + vmap(r, h) < W2 ? acc[r] : 0.f;
         };
         auto marked = [&] { return fbad || __builtin_amdgcn_readfirstlane(mark) != 0; };
+        // (both factors here, so that the running state is in the units of the results: a state that `back` is applied to at
+        // the end overflows for products of marked blocks and for weights that the results themselves have room for)
         auto scale_back = [&](const v16f &acc, float (&x)[16]) {
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[4 * g4 + e] = acc[4 * g4 + e] * fac[g4][e];
+                for (int e = 0; e < 4; ++e) x[4 * g4 + e] = acc[4 * g4 + e] * fac[g4][e] * back;
         };
         __syncthreads();
         float x[16];
@@ -684,8 +685,8 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 v4f x;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    if constexpr (WT) x[e] = rv[q][4 * g4 + e] * back;
-                    else x[e] = q == 0 ? vmax[4 * g4 + e] * back : q == 1 ? vsum[4 * g4 + e] * back : __int_as_float(vidx[4 * g4 + e]);
+                    if constexpr (WT) x[e] = rv[q][4 * g4 + e];
+                    else x[e] = q == 0 ? vmax[4 * g4 + e] : q == 1 ? vsum[4 * g4 + e] : __int_as_float(vidx[4 * g4 + e]);
                 }
                 const int v = 32 * vc + vmap(4 * g4, h);
                 if (!whole) *reinterpret_cast<v4f *>(slot + (q * 16 + g4) * 256) = x;

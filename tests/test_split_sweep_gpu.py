@@ -110,6 +110,37 @@ def test_pixels_without_halves(device, value, where):
         assert ((best - at).abs() <= 1e-5 * scale)[best.isfinite()].all()
 
 
+@pytest.mark.parametrize("magnitude", [1.0, 2.0 ** -20])
+def test_large_products_stay_finite(device, magnitude):
+    """Products up to 2^126 and weights up to 2^112 come out finite where their sums are: an fmap2 channel of +-2^e beside
+    features of `magnitude` (one of 2^120 has no halves and is multiplied in fp32)."""
+    dims = (1, 50, 82, 74, 35, 32)
+    B, H1, W1, H2, W2, C = dims
+    f1, f2, g = op_inputs(*dims, seed=10)
+    f1 = f1 * magnitude
+    f1[..., 11] = magnitude
+    for e, u, v in ((120, 30, 20), (100, 50, 33), (22, 60, 3)):
+        f2[0, u, v, 11], f2[0, u + 5, v, 11] = 2.0 ** e, -2.0 ** e
+    vol, err = _volume(f1.double(), f2.double()), _bound(f1, f2, H2 + W2)
+    out_u, out_v = (t.cpu().double() for t in _max_avg(f1.to(device), f2.to(device), dims)[:2])
+    for out, d in ((out_u, 4), (out_v, 3)):
+        assert out.isfinite().all()
+        assert ((out[:, :, :, 0] - vol.amax(d)).abs() <= err.amax(d)).all()
+        assert ((out[:, :, :, 1] - vol.mean(d)).abs() <= err.mean(d)).all()
+    # the weights take the place of the large features: the sums stay below 2^124
+    f2.clamp_(-8, 8)
+    a_u, a_v = (torch.randn(B, H1, W1, 4, n, generator=g) * 2.0 ** 112 for n in (W2, H2))
+    vol, err = _volume(f1.double(), f2.double()), _bound(f1, f2, H2 + W2 + 2)
+    for K in (1, 4):
+        outs = [torch.empty(B, H1, W1, K, n, device=device) for n in (H2, W2)]
+        ws = [a_u[:, :, :, :K].contiguous(), a_v[:, :, :, :K].contiguous()]
+        _call("sepcorr_compression_forward", outs, [t.to(device) for t in [f1, f2] + ws], dims, True, (K,), K)
+        for k in range(K):
+            wu, wv = a_u[:, :, :, k, None, :].double(), a_v[:, :, :, k, :, None].double()
+            assert ((outs[0][:, :, :, k].cpu() - (vol * wu).sum(4)).abs() <= (err * wu.abs()).sum(4)).all()
+            assert ((outs[1][:, :, :, k].cpu() - (vol * wv).sum(3)).abs() <= (err * wv.abs()).sum(3)).all()
+
+
 def test_without_scratch_the_same_bits(device):
     dims = SHAPES[7]
     f1, f2, _ = op_inputs(*dims, seed=9)
