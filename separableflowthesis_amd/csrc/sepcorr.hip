@@ -1464,7 +1464,12 @@ __global__ void __launch_bounds__(512) fwd_kernel(const FwdArgs a) {
 #pragma unroll
                         for (int k = 0; k < KC; ++k) {
                             const size_t row = bp_e * a.KT + a.k0 + k;
-                            ke->lev[lvl].out_v[row * W2 + v] = soft_dlog ? dlogit(ke->lev[lvl].z_ov, ke->lev[lvl].st_ov, ke->lev[lvl].dot_ov, row, row * W2 + v, rv[k][r]) : rv[k][r];
+                            float x = rv[k][r];
+                            if (soft_dlog) {   // (as merge_pieces does it: either may finish a tile, with the same bits)
+                                const float r3[3] = {ke->lev[lvl].st_ov[2 * row], 1.f / ke->lev[lvl].st_ov[2 * row + 1], ke->lev[lvl].dot_ov[row]};
+                                x = dlogit3(ke->lev[lvl].z_ov[row * W2 + v], r3, x);
+                            }
+                            ke->lev[lvl].out_v[row * W2 + v] = x;
                         }
                     } else {
                         ke->lev[lvl].out_v[(bp_e * 2 + 0) * W2 + v] = vmax[r];

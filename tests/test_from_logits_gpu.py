@@ -137,3 +137,20 @@ def test_from_logits_at_benchmark_sizes(device, B):
         assert_close(cv[sl], rcv, "compression_output_v")
         for got, ref, n in zip((d1, d2, dz_u, dz_v), r, ("d_f1", "d_f2", "d_logits_u", "d_logits_v")):
             assert_close(got[sl], ref.grad, n, scale_atol=True)
+
+
+def test_logit_gradients_repeat_exactly(device):
+    """Rows of odd length, tiles in pieces: whichever piece of a tile is done last finishes it, with the same bits."""
+    shape, K = (2, 5, 7, 5, 7, 16), 4
+    B, H1, W1, H2, W2, C = shape
+    f1, f2, g = op_inputs(*shape, seed=51)
+    z_u, z_v = _logits(B, H1, W1, H2, W2, K, g)
+    g_cu, g_cv = torch.randn(B, H1, W1, K, H2, generator=g), torch.randn(B, H1, W1, K, W2, generator=g)
+    f1, f2, z_u, z_v, g_cu, g_cv = (t.to(device) for t in (f1, f2, z_u, z_v, g_cu, g_cv))
+    ms = _ms()
+    cu, cv, st_u, st_v = ms.compression_forward_from_logits(f1, f2, z_u, z_v)
+    call = lambda features: ms.compression_backward_from_logits(f1, f2, z_u, z_v, st_u, st_v, cu, cv, g_cu, g_cv, need_features=features)[2:]
+    first = call(False)
+    for _ in range(200):   # (other kernels and waits in between: the pieces then end in another order now and then)
+        for features in (True, False):
+            assert all(torch.equal(a, b) for a, b in zip(call(features), first))
