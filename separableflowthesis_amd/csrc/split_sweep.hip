@@ -4,13 +4,14 @@
 // time and reduced at once, over the columns v of fmap2 into out_u and over its rows u into out_v.
 //
 // Contraction.  A pixel's channels are scaled by a power of two that brings the largest of them into [2^14, 2^15) and
-// each is written as h + l, h = fp16(x), l = fp16(x - h): 22 significant bits, and everything below 2^-25 of the
-// pixel's largest channel comes out at least as fine as 2^-39 of it.  A product is h h + h l + l h: three
+// each is written as h + 2^-11 l, h = fp16(x), l = fp16(2^11 (x - h)): 22 significant bits down to 2^-28 of the pixel's
+// largest channel (both halves of a smaller one are subnormal), 2^-50 of it below.  Pixels with more than a few
+// channels that are smaller still but not zero are marked (below).  A product is h h + 2^-11 (h l + l h): three
 // v_mfma_f32_32x32x16_f16, which accumulate in fp32, in place of eight v_mfma_f32_32x32x2_f32 of twice the length.
 // What is left out (l l) and what the halves do not hold are below the rounding of the fp32 sum, and a sum of 256
 // products is rounded 48 times instead of 128.
 // Scaling by powers of two is exact and taken back in fp32.  A pixel that has no such form (a channel that is inf or
-// NaN, or whose largest channel lies outside [2^-24, 2^24)) is marked, and 32x32 blocks with a marked pixel are
+// NaN, whose largest channel lies outside [2^-24, 2^24), or max(2, C / 32) channels below 2^-28 of that) is marked, and 32x32 blocks with a marked pixel are
 // multiplied with fp32 MFMAs straight from the inputs.
 //
 // Work split.  A step = 128 pixels p x 32 columns v of one row u: the workgroup's four waves own 32 pixels each, whose
@@ -81,6 +82,7 @@ __device__ __forceinline__ bool pixel_scale(unsigned m, float &fwd, float &back)
     back = __uint_as_float((e - 14u) << 23);
     return true;
 }
+constexpr float LOW_UNIT = 1.f / 2048.f;   // low halves are held times 2^11: they are as far from the subnormals as high ones
 // (a marked pixel has factor 0 and may hold inf: its halves are zeros, not NaN)
 __device__ __forceinline__ void split8(const float (&x)[8], float f, v8h &h, v8h &l) {
 #pragma unroll
@@ -88,7 +90,7 @@ __device__ __forceinline__ void split8(const float (&x)[8], float f, v8h &h, v8h
         const float y = f == 0.f ? 0.f : x[e] * f;
         const _Float16 hh = (_Float16)y;
         h[e] = hh;
-        l[e] = (_Float16)(y - (float)hh);
+        l[e] = (_Float16)((y - (float)hh) * (1.f / LOW_UNIT));
     }
 }
 constexpr unsigned OOB = 0x80000000u;   // a byte offset above every buffer size used here: reads as zero
@@ -177,7 +179,7 @@ __global__ void __launch_bounds__(256) split_prepare_kernel(const SplitArgs a) {
     const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, (unsigned)n * a.C * 4u);
     constexpr int M = NK / 4;                            // 8 lanes x 8 channels = 4 channel steps
     float x[M][8];
-    unsigned m = 0;
+    unsigned m = 0, tiny = 0;
 #pragma unroll
     for (int t = 0; t < M; ++t) {
         load8(rs, ok ? (unsigned)v * a.C * 4u : OOB, 64 * t + 8 * j, a.C, vec, x[t]);
@@ -186,8 +188,19 @@ __global__ void __launch_bounds__(256) split_prepare_kernel(const SplitArgs a) {
     }
 #pragma unroll
     for (int d = 1; d < 8; d <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, d));
+    // Non-zero channels below 2^-28 of the largest: a few are let pass, each with an error below 2^-50 of the largest.
+    // (Among 256 normal ones a single one is found once in some 600 000 pixels; beside one channel of 2^14 times the
+    // others two are found in one pixel of 12 000, beside one of 2^20 eight in one of a million.)
+    const unsigned least = m > (28u << 23) ? (m & 0x7f800000u) - (28u << 23) : 0;
+#pragma unroll
+    for (int t = 0; t < M; ++t)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) tiny += magnitude(x[t][e]) - 1u < least - 1u && least > 0;
+#pragma unroll
+    for (int d = 1; d < 8; d <<= 1) tiny += (unsigned)__shfl_xor((int)tiny, d);
     float f, back;
-    const bool good = pixel_scale(m, f, back);
+    const bool good = pixel_scale(m, f, back) && tiny < max(2u, (unsigned)a.C / 32);
+    if (!good) f = 0.f, back = 1.f;
 #pragma unroll
     for (int t = 0; t < M; ++t) {
         v8h h, lo;
@@ -341,6 +354,13 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
     constexpr bool PIPE = pipelined(MODE, KC);
     constexpr int Q = WT ? KC : (MODE == SPLIT_ARGMAX ? 3 : 2);
     constexpr int BLK = block_bytes(NK), BF = BLK / 4, NBUF = PIPE ? 3 : 2;
+    // The low halves' products are summed apart, in units of LOW_UNIT.  The max/avg modes have no registers left for a second
+    // accumulator at NK = 16 (argmax would spill 29): they sum the products of the low halves first, scale the sum and read
+    // the high halves from LDS once more for the rest.  Measured at B=2, 55x128, C=256 (whole call; one accumulator with low
+    // halves in units of 1, which loses bits of small channels, first): argmax 187 us, 196 as it is, 201 with two
+    // accumulators; max/average 170, 180, 176 (kept like argmax, so that both give the same bits); one channel 168, 175, 171;
+    // four channels 216 and 220.
+    constexpr bool TWO_ACC = WT || NK < 16;
     extern __shared__ float smem[];                       // NBUF row blocks, then the u-indexed weights of each wave
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const int lane = threadIdx.x & 63, pl = lane & 31, h = lane >> 5;
@@ -575,31 +595,35 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
         auto multiply = [&](int next, int buf, int nbuf, auto beside) {
             const char *blk = reinterpret_cast<const char *>(smem + buf * BF) + lane * 16;
             const float *tail = smem + buf * BF + 2 * NK * 256;
-            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, cross = acc;
             v8h ah[3], al[3];
-            auto fetch = [&](int s) {
-                ah[s % 3] = *reinterpret_cast<const v8h *>(blk + s * 2048);
-                al[s % 3] = *reinterpret_cast<const v8h *>(blk + s * 2048 + 1024);
+            auto fetch = [&](int t) {   // step t: channel step t mod NK; the second pass over them needs no low halves
+                ah[t % 3] = *reinterpret_cast<const v8h *>(blk + (t % NK) * 2048);
+                if (t < NK) al[t % 3] = *reinterpret_cast<const v8h *>(blk + t * 2048 + 1024);
             };
+            constexpr int NT = TWO_ACC ? NK : 2 * NK;
             fetch(0);
             fetch(1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int s = 0; s < NK; ++s) {
-                if (s + 2 < NK) fetch(s + 2);
-                if (s == NK - 2) {
+            for (int t = 0; t < NT; ++t) {
+                if (t + 2 < NT) fetch(t + 2);
+                if (t == NT - 2) {
 #pragma unroll
                     for (int g4 = 0; g4 < 4; ++g4) fac[g4] = *reinterpret_cast<const v4f *>(tail + 8 * g4 + 4 * h);
                     mark = __float_as_int(tail[MARK]);
                 }
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s % 3], fh[s], acc, 0, 0, 0);
-                if (s < NDMA) dma(next, nbuf, s);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[s % 3], fl[s], acc, 0, 0, 0);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[s % 3], fh[s], acc, 0, 0, 0);
-                beside(s);
+                if (t == NK) acc = cross * LOW_UNIT;
+                if (TWO_ACC || t >= NK) acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t % 3], fh[t % NK], acc, 0, 0, 0);
+                if (t < NDMA) dma(next, nbuf, t);
+                if (t < NK) {
+                    cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[t % 3], fh[t], cross, 0, 0, 0);
+                    cross = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[t % 3], fl[t], cross, 0, 0, 0);
+                }
+                beside(t);
                 __builtin_amdgcn_sched_barrier(0);
             }
-            return acc;
+            return TWO_ACC ? acc + cross * LOW_UNIT : acc;
         };
         constexpr int PER = 16 / NK;   // accumulator registers reduced beside one channel step
         // a block with a marked pixel: fp32 products straight from the inputs

@@ -110,6 +110,57 @@ def test_pixels_without_halves(device, value, where):
         assert ((best - at).abs() <= 1e-5 * scale)[best.isfinite()].all()
 
 
+def _outlier(f1, f2, r, g):
+    f1[..., 0], f2[..., 0] = 2.0 ** r, 0.0
+
+
+def _outliers_on_both_sides(f1, f2, r, g):
+    f1[..., 0], f2[..., 0] = 2.0 ** r, 0.0
+    f1[..., 1], f2[..., 1] = 0.0, 2.0 ** r
+
+
+def _channel_scales(f1, f2, r, g):
+    s = 2.0 ** torch.randint(-r // 2, r // 2 + 1, f1.shape[-1:], generator=g)
+    s[0] = 1.0
+    f1 *= s
+    f2 /= s
+
+
+@pytest.mark.parametrize("C", [256, 64])
+@pytest.mark.parametrize("mode", ["max_avg", 1, 4])
+@pytest.mark.parametrize("change", [_outlier, _outliers_on_both_sides, _channel_scales])
+def test_range_within_a_pixel(device, change, mode, C):
+    """Channels of very different magnitude within a pixel.  None of the changes alters a product that is not zero, so the
+    error (2-norm) stays what it is without them, but for the larger one of blocks that are multiplied in fp32: a sum of
+    256 products is rounded 128 times there and 16 times (the small cross terms aside) with halves, which gives sqrt(8)
+    times the error; 3 times is allowed."""
+    dims = (1, 48, 64, 47, 64, C)
+    B, H1, W1, H2, W2, _ = dims
+    errors = {}
+    for r in (None, 12, 18, 20, 22, 24, 27, 32, 48):
+        f1, f2, g = op_inputs(*dims, seed=11)
+        for f in (f1, f2):
+            f[..., :2] = 0.0
+        weights = [torch.randn(B, H1, W1, mode, n, generator=g) for n in (W2, H2)] if mode != "max_avg" else []
+        if r is not None:
+            change(f1, f2, r, g)
+        vol = _volume(f1.double(), f2.double())
+        if mode == "max_avg":
+            out_u, out_v = (t.cpu().double() for t in _max_avg(f1.to(device), f2.to(device), dims)[:2])
+            got = [out_u[:, :, :, 1], out_v[:, :, :, 1], out_u[:, :, :, 0], out_v[:, :, :, 0]]
+            want = [vol.mean(4), vol.mean(3), vol.amax(4), vol.amax(3)]
+        else:
+            outs = [torch.empty(B, H1, W1, mode, n, device=device) for n in (H2, W2)]
+            _call("sepcorr_compression_forward", outs, [t.to(device) for t in [f1, f2] + weights], dims, True, (mode,), mode)
+            got = [t.cpu().double() for t in outs]
+            want = [torch.stack([(vol * weights[0][:, :, :, k, None, :]).sum(4) for k in range(mode)], 3),
+                    torch.stack([(vol * weights[1][:, :, :, k, :, None]).sum(3) for k in range(mode)], 3)]
+        errors[r] = [((a - b).norm() / b.norm()).item() for a, b in zip(got, want)]
+    print(errors)
+    for r, error in errors.items():
+        assert all(e <= 3 * e0 for e, e0 in zip(error, errors[None])), (r, error, errors[None])
+
+
 @pytest.mark.parametrize("magnitude", [1.0, 2.0 ** -20])
 def test_large_products_stay_finite(device, magnitude):
     """Products up to 2^126 and weights up to 2^112 come out finite where their sums are: an fmap2 channel of +-2^e beside
