@@ -11,7 +11,7 @@
 // What is left out (l l) and what the halves do not hold are below the rounding of the fp32 sum, and a sum of 256
 // products is rounded 48 times instead of 128.
 // Scaling by powers of two is exact and taken back in fp32.  A pixel that has no such form (a channel that is inf or
-// NaN, whose largest channel lies outside [2^-24, 2^24), or max(2, C / 32) channels below 2^-28 of that) is marked, and 32x32 blocks with a marked pixel are
+// NaN, whose largest channel lies outside [2^-60, 2^61), or max(2, C / 32) channels below 2^-28 of that) is marked, and 32x32 blocks with a marked pixel are
 // multiplied with fp32 MFMAs straight from the inputs.
 //
 // Work split.  A step = 128 pixels p x 32 columns v of one row u: the workgroup's four waves own 32 pixels each, whose
@@ -77,7 +77,7 @@ __device__ __forceinline__ int xcd_contiguous(int bid, int n) {
 __device__ __forceinline__ bool pixel_scale(unsigned m, float &fwd, float &back) {
     const unsigned e = m >> 23;
     if (m == 0) { fwd = 1.f; back = 1.f; return true; }
-    if (e < 103 || e > 150) { fwd = 0.f; back = 1.f; return false; }
+    if (e < 67 || e > 187) { fwd = 0.f; back = 1.f; return false; }
     fwd = __uint_as_float((268u - e) << 23);
     back = __uint_as_float((e - 14u) << 23);
     return true;
@@ -110,6 +110,35 @@ __device__ __forceinline__ void load8(__amdgpu_buffer_rsrc_t r, unsigned off, in
     }
 }
 __device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
+
+// A block with a marked pixel: fp32 products straight from the inputs, this lane's pixel of image 1 at byte o1 of n1, of
+// fmap2 at byte o2 of n2 (OOB: none), the first `cols` columns of this lane's half.  16 channels a turn; a lane's eight are contiguous, and the next turn's are on their
+// way.  A function of its own: its registers would otherwise be taken from the sweep's.
+// B=2, 55x128, max/average: 0.18 ms without a marked pixel, 0.44 with one in image 1, 0.86 with all of them marked; with one
+// channel a turn 0.88 and 2.78 ms, the fp32 sweep 0.44.
+__device__ __attribute__((noinline)) v16f products_fp32(const float *f1, unsigned n1, unsigned o1, const float *f2, unsigned n2, unsigned o2,
+                                                        int C_in, int cols) {
+    const int C = __builtin_amdgcn_readfirstlane(C_in), h = (threadIdx.x >> 5) & 1;
+    const __amdgpu_buffer_rsrc_t r1 = make_rsrc(f1, n1), r2 = make_rsrc(f2, n2);
+    const bool vec = (C & 3) == 0;
+    v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float y[8], z[8];
+    load8(r2, o2, 8 * h, C, vec, y);
+    load8(r1, o1, 8 * h, C, vec, z);
+#pragma unroll 1
+    for (int c = 16; c < C + 16; c += 16) {
+        float yn[8], zn[8];
+        load8(r2, o2, c + 8 * h, C, vec, yn);
+        load8(r1, o1, c + 8 * h, C, vec, zn);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(y[e], z[e], acc, 0, 0, 0);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) y[e] = yn[e], z[e] = zn[e];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = vmap(r, 0) < cols ? acc[r] : 0.f;   // (an inf of image 1 times nothing is no NaN)
+    return acc;
+}
 
 // The workgroups that hold the steps [t0, t1) when T steps are dealt out evenly to G workgroups.
 __device__ __forceinline__ void pieces_of(long t0, long t1, int G, long T, int &w0, int &w1) {
@@ -357,13 +386,12 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
     // The low halves' products are summed apart, in units of LOW_UNIT.  The max/avg modes have no registers left for a second
     // accumulator at NK = 16 (argmax would spill 29): they sum the products of the low halves first, scale the sum and read
     // the high halves from LDS once more for the rest.  Measured at B=2, 55x128, C=256 (whole call; one accumulator with low
-    // halves in units of 1, which loses bits of small channels, first): argmax 187 us, 196 as it is, 201 with two
-    // accumulators; max/average 170, 180, 176 (kept like argmax, so that both give the same bits); one channel 168, 175, 171;
-    // four channels 216 and 220.
+    // halves in units of 1, which loses bits of small channels, first): argmax 185 us, 189 as it is, 197 with two
+    // accumulators; max/average 169, 178, 174 (kept like argmax, so that both give the same bits); one channel 166, 175, 168;
+    // four channels 215, 229 and 223.
     constexpr bool TWO_ACC = WT || NK < 16;
     extern __shared__ float smem[];                       // NBUF row blocks, then the u-indexed weights of each wave
     const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int lane = threadIdx.x & 63, pl = lane & 31, h = lane >> 5;
     float *wus = smem + NBUF * BF + wave * (KC * 128);       // [k][row & 3][pixel]
     const int wg = xcd_contiguous(blockIdx.x, gridDim.x);
     const long T = a.steps;
@@ -371,6 +399,12 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
     const int N1 = a.N1, C = a.C, N1p = a.npt * TPX;
 
     for (int g = g0; g < g1;) {
+        // (max/avg modes: derived afresh for every piece.  What follows from them is otherwise worked out ahead of the loop over
+        // the pieces, spilled and read back one by one where a piece begins; argmax, B=2, 55x128: 192 -> 189 us.  One weight
+        // channel has the registers for it: 168 us as it is, 175 afresh.)
+        int tid = threadIdx.x;
+        if constexpr (!WT) keep_here(tid);
+        const int lane = tid & 63, pl = lane & 31, h = lane >> 5;
         int l = a.nlev - 1;
         while (l > 0 && g < a.lev[l].step0) --l;
         const SplitLevel &L = a.lev[l];
@@ -378,6 +412,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
         const int t = (g - L.step0) / H2, ua = (g - L.step0) - t * H2, ub = min(H2, ua + g1 - g);
         const int pt = t % a.npt, bc = t / a.npt, vc = bc % nvc, b = bc / nvc;
         g += ub - ua;
+        const int cols = W2 - 32 * vc - 4 * h;   // register r holds column vmap(r, 0) of this half: one of the image if below
         const int pix = (a.pt0 + pt) * TPX + 32 * wave + pl;
         const bool pok = pix < N1;
         const size_t bp = (size_t)b * N1 + (pok ? pix : 0);
@@ -526,7 +561,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 vsum[r] += y;
                 if constexpr (MODE == SPLIT_ARGMAX) vidx[r] = y > vmax[r] ? red_u : vidx[r];
                 vmax[r] = maxnum(vmax[r], y);
-                const float z = (edge && 32 * vc + vmap(r, h) >= W2) ? -INFINITY : y;
+                const float z = (edge && vmap(r, 0) >= cols) ? -INFINITY : y;
                 if constexpr (MODE == SPLIT_ARGMAX) red_i = z > red_m ? vmap(r, 0) : red_i;
                 red_m = maxnum(red_m, z);
                 keep_here(vmax[r]);
@@ -626,27 +661,22 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
             return TWO_ACC ? acc + cross * LOW_UNIT : acc;
         };
         constexpr int PER = 16 / NK;   // accumulator registers reduced beside one channel step
-        // a block with a marked pixel: fp32 products straight from the inputs
         auto multiply_fp32 = [&](int u, float (&x)[16]) {
-            const int v = 32 * vc + pl;
-            const bool vok = v < W2;
-            const float *f1p = a.f1 + bp * C;
-            const float *q = L.f2 + (((size_t)b * H2 + u) * W2 + (vok ? v : 0)) * C;
-            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-            for (int c = h; c < C + h; c += 2)
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32((vok && c < C) ? q[c] : 0.f, (pok && c < C) ? f1p[c] : 0.f, acc, 0, 0, 0);
+            const int v = 32 * vc + pl, first = (a.pt0 + pt) * TPX;
+            const v16f acc = products_fp32(a.f1 + ((size_t)b * N1 + first) * C, (unsigned)min(TPX, N1 - first) * C * 4u,
+                                           pok ? (unsigned)(32 * wave + pl) * C * 4u : OOB, L.f2 + ((size_t)b * H2 + u) * W2 * C,
+                                           (unsigned)W2 * C * 4u, v < W2 ? (unsigned)v * C * 4u : OOB, C, cols);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) x[r] = 32 * vc + vmap(r, h) < W2 ? acc[r] : 0.f;
+            for (int r = 0; r < 16; ++r) x[r] = acc[r];
         };
-        auto marked = [&] { return fbad || __builtin_amdgcn_readfirstlane(mark) != 0; };
         // (both factors here, so that the running state is in the units of the results: a state that `back` is applied to at
         // the end overflows for products of marked blocks and for weights that the results themselves have room for)
-        auto scale_back = [&](const v16f &acc, float (&x)[16]) {
+        auto products = [&](const v16f &acc, int u, float (&x)[16]) {
 #pragma unroll
             for (int g4 = 0; g4 < 4; ++g4)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) x[4 * g4 + e] = acc[4 * g4 + e] * fac[g4][e] * back;
+            if (fbad || __builtin_amdgcn_readfirstlane(mark) != 0) multiply_fp32(u, x);
         };
         __syncthreads();
         float x[16];
@@ -658,8 +688,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 // what the last requests of the step before take.  At the end of a step all but this step's requests
                 // have to be there: of the wave's outstanding memory operations the latest 2 NK / 4 are among those.
                 auto step_end = [] { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(NK / 2) : "memory"); };
-                scale_back(multiply(ua + 2, 0, 2, nothing), x);
-                if (marked()) multiply_fp32(ua, x);
+                products(multiply(ua + 2, 0, 2, nothing), ua, x);
                 step_end();
                 int buf = 1;
                 for (int u = ua + 1; u < ub; ++u) {
@@ -671,8 +700,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                         for (int e = 0; e < PER; ++e) take(edge, PER * s + e, x[PER * s + e]);
                     });
                     finish();
-                    scale_back(acc, x);
-                    if (marked()) multiply_fp32(u, x);
+                    products(acc, u, x);
                     step_end();
                     buf = buf == 2 ? 0 : buf + 1;
                 }
@@ -686,8 +714,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
                 for (int u = ua; u < ub; ++u) {
                     const int buf = (u - ua) & 1;
                     if (u > ua) flush();
-                    scale_back(multiply(u + 1, buf, buf ^ 1, nothing), x);
-                    if (marked()) multiply_fp32(u, x);
+                    products(multiply(u + 1, buf, buf ^ 1, nothing), u, x);
                     begin(u);
 #pragma unroll
                     for (int r = 0; r < 16; ++r) take(edge, r, x[r]);
