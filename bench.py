@@ -10,7 +10,7 @@ with attention; where the library runs the max/avg backward as gathers instead o
 are executed and counted, and the algorithmic figure (7 passes over the same time) and the timing of the all-dense
 step stand beside it (`algorithmic_tflops`, `all_dense`).  `ms_per_step` is the figure to compare builds by.  The same line
 carries a `configs` table with all five benchmark configurations (ms/step, TFLOP/s, fraction of the
-fp32 MFMA peak, peak HBM allocated, dominant-kernel roofline), the CPU baseline (full-4D torch path on
+MFMA peak, peak HBM allocated, dominant-kernel roofline), the CPU baseline (full-4D torch path on
 the host cores, one thread and all threads) and, as extras, the caller-level measurements.
 """
 import argparse
@@ -26,6 +26,8 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 PEAK_FP32_MFMA_TFLOPS = 157.3   # 256 CU x 256 flop/clk x 2.4 GHz
+# a product of two fp32 operands held as two 16-bit halves each is three 16-bit products: 256 CU x 4096 flop/clk x 2.4 GHz / 3
+PEAK_SPLIT_MFMA_TFLOPS = 838.9
 METRIC = "fused corr-separation fwd+bwd ms and MFMA TFLOP/s at B=2, C=256, 55×128"
 C = 256
 
@@ -40,8 +42,13 @@ WORKLOADS = {
 OPS_TEXT = "(f=max/argmax/avg fwd, c=compression fwd, C=compression bwd, F=max/avg bwd)"
 PASSES = {"f": 1, "c": 1, "C": 3, "F": 2}
 # kernels that execute one contraction pass (W = 2*B*N1*N2*C flops) per launch
-SWEEP_KERNELS = ("fwd_maxavg", "fwd_weighted", "df1_comp", "df2_comp", "df1_maxavg", "df2_maxavg", "df1_both", "df2_both")
+SWEEP_KERNELS = ("fwd_maxavg", "fwd_weighted", "fwd_maxavg_split", "fwd_weighted_split", "df1_comp", "df2_comp", "df1_maxavg", "df2_maxavg", "df1_both", "df2_both")
 _MIB = 2 ** 20
+
+
+def mfma_peak(label):
+    """Rate of fp32 products on the matrix instructions that the kernel of this label uses."""
+    return PEAK_SPLIT_MFMA_TFLOPS if label.endswith("_split") else PEAK_FP32_MFMA_TFLOPS
 
 
 def measured_traffic(workload):
@@ -69,9 +76,9 @@ def algorithmic_bytes(label, B, N, H, W, Kp):
     """Bytes a launch must move at least: every input read once, every output written once (fp32/int32)."""
     feat = B * N * C
     per_p_u, per_p_v = B * N * H, B * N * W          # one channel of a *_u / *_v tensor
-    if label == "fwd_maxavg":
+    if label.startswith("fwd_maxavg"):
         n = 2 * feat + 3 * (per_p_u + per_p_v)         # f1, f2; max, avg, argmax of both volumes
-    elif label == "fwd_weighted":
+    elif label.startswith("fwd_weighted"):
         n = 2 * feat + 2 * Kp * (per_p_u + per_p_v)    # f1, f2; K' weights in, K' sums out, both volumes
     else:
         fields = {"maxavg": 3, "comp": 2 * Kp, "both": 3 + 2 * Kp}[label.split("_")[1]]
@@ -350,7 +357,7 @@ class Workload:
             ent = {"avg_ms": round(avg, 4), "launches_per_step": round(len(ts) / max(1, profile_steps), 2)}
             if nm in SWEEP_KERNELS:
                 ent["tflops"] = round(Wf / (avg * 1e-3) / 1e12, 2)
-                ent["frac_of_peak"] = round(ent["tflops"] / PEAK_FP32_MFMA_TFLOPS, 4)
+                ent["frac_of_peak"] = round(ent["tflops"] / mfma_peak(nm), 4)
             kernels[nm] = ent
         dom = max((k for k in kernels if k in SWEEP_KERNELS),
                   key=lambda k: kernels[k]["avg_ms"] * kernels[k]["launches_per_step"])
@@ -364,6 +371,8 @@ class Workload:
         gathered = any(k.endswith("_gather") for k in kernels)
         executed = passes - (PASSES["F"] if gathered else 0)
         value = executed * Wf / (ms * 1e-3) / 1e12
+        # what the executed passes take at the peak of the matrix instructions each of them runs on
+        floor_ms = sum(k["launches_per_step"] * Wf / mfma_peak(nm) / 1e9 for nm, k in kernels.items() if nm in SWEEP_KERNELS)
         dense = None
         if gathered:
             prev_mode = self.lib.sepcorr_set_max_avg_backward(1)
@@ -372,23 +381,22 @@ class Workload:
             finally:
                 self.lib.sepcorr_set_max_avg_backward(prev_mode)
             dense = {"ms_per_step": round(dms, 4), "tflops": round(passes * Wf / (dms * 1e-3) / 1e12, 3),
-                     "frac_of_fp32_mfma_peak": round(passes * Wf / (dms * 1e-3) / 1e12 / PEAK_FP32_MFMA_TFLOPS, 4),
                      "what": "the same step with sepcorr_set_max_avg_backward(SEPCORR_MAXAVG_DENSE): every pass a contraction"}
-        roofline = {"bound": "mfma", "kernel": dom, "achieved": ach, "peak": PEAK_FP32_MFMA_TFLOPS, "unit": "TFLOP/s",
-                    "frac": round(ach / PEAK_FP32_MFMA_TFLOPS, 4), "traffic": traffic.get(dom),
+        roofline = {"bound": "mfma", "kernel": dom, "achieved": ach, "peak": mfma_peak(dom), "unit": "TFLOP/s",
+                    "frac": round(ach / mfma_peak(dom), 4), "traffic": traffic.get(dom),
                     "algorithmic_bytes": algorithmic_bytes(dom, B, N, H, W, Kp),
                     "algorithmic_flop": Wf, "avg_launch_ms": kernels[dom]["avg_ms"]}
         return {
             "workload": f"{self.name}: B={B}, C={C}, {H}x{W}, K'={Kp}, ops={ops}",
             "ms_per_step": round(ms, 4), "tflops": round(value, 3),
-            "frac_of_fp32_mfma_peak": round(value / PEAK_FP32_MFMA_TFLOPS, 4),
+            "mfma_floor_ms": round(floor_ms, 4), "frac_of_mfma_floor": round(floor_ms / ms, 4),
             "contraction_passes": passes, "gflop_per_step": round(passes * Wf / 1e9, 2),
             "contraction_passes_executed": executed,
             "algorithmic_tflops": round(algorithmic, 3),
             "max_avg_backward": ("gather" if gathered else "dense") if "F" in ops else None,
             "all_dense": dense,
-            "note": ("tflops / frac_of_fp32_mfma_peak count the contraction_passes_executed passes that ran on the matrix "
-                     "cores; the max/avg backward ran as gathers of feature rows instead of its two contractions; "
+            "note": ("tflops counts the contraction_passes_executed passes that ran on the matrix cores, mfma_floor_ms is what they "
+                     "take at the peak of the matrix instructions that each runs on; the max/avg backward ran as gathers of feature rows instead of its two contractions; "
                      "algorithmic_tflops counts all contraction_passes of the reference's formulation over the same time; "
                      "all_dense is the same step with every pass a contraction")
                     if gathered else None,
@@ -578,7 +586,8 @@ def main():
                    "contraction_passes_executed": head["contraction_passes_executed"],
                    "algorithmic_tflops": head["algorithmic_tflops"], "max_avg_backward": head["max_avg_backward"],
                    "all_dense": head["all_dense"], "note": head["note"],
-                   "frac_of_fp32_mfma_peak": head["frac_of_fp32_mfma_peak"],
+                   "mfma_floor_ms": head["mfma_floor_ms"], "frac_of_mfma_floor": head["frac_of_mfma_floor"],
+                   "arithmetic": "fp32 inputs, sums and outputs; *_split kernels take every operand as two fp16 halves, the others fp32 MFMA",
                    "peak_hbm_allocated_mib": head["peak_hbm_allocated_mib"],
                    "backward_workspace_mib": head["backward_workspace_mib"],
                    "volume_4d_never_allocated_mib": head["volume_4d_never_allocated_mib"]},
@@ -594,7 +603,7 @@ def main():
             "what": "same inputs and outputs as the headline step (d_f1, d_f2 are the sums of the two operators' "
                     "gradients), via sepcorr_compression_backward(d_f1=d_f2=NULL) + sepcorr_fused_backward"}
         # The headline step with the forward sweeps and d_f1 contracting in three bf16 planes per operand: an option
-        # of this library (sepcorr_set_contraction), not the headline arithmetic, which is fp32 MFMA throughout.
+        # of this library (sepcorr_set_contraction), not the headline arithmetic.
         prev_mode = lib.sepcorr_set_contraction(1)
         try:
             pms = wl.time(wl.step, args.steps, args.warmup)

@@ -3165,7 +3165,7 @@ int try_split(const FwdArgs &a, int B, hipStream_t s) {
     }
     constexpr int mode = is_weighted(MODE) ? SPLIT_WEIGHTED : MODE == MODE_ARGMAX ? SPLIT_ARGMAX : SPLIT_MAXAVG;
     constexpr int kc = is_weighted(MODE) ? KC : 0;
-    ProfScope ps(p.nlev > 1 ? (kc ? "fwd_weighted_levels" : "fwd_maxavg_levels") : (kc ? "fwd_weighted" : "fwd_maxavg"), s);
+    ProfScope ps(p.nlev > 1 ? (kc ? "fwd_weighted_levels_split" : "fwd_maxavg_levels_split") : (kc ? "fwd_weighted_split" : "fwd_maxavg_split"), s);
     int rc = a.ws != nullptr ? split_sweep(mode, kc, p, a.ws, a.ws_bytes, s) : 1;
     if (rc == 1 && !t_no_alloc) {
         int h2[4], w2[4];

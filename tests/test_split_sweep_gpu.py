@@ -20,9 +20,26 @@ SHAPES = [(1, 50, 82, 74, 35, 32), (2, 40, 64, 61, 34, 33), (1, 63, 65, 33, 65, 
           (1, 96, 172, 401, 1, 96), (1, 48, 65, 11, 290, 48)]
 
 
-def test_sizes_take_the_split_sweep():
-    for B, H1, W1, H2, W2, C in SHAPES:
-        assert B * H1 * W1 * H2 * W2 * (C + 64) >= 1e9
+def _labels_of(fn):
+    """Labels of the kernels that fn() launches, by the library's own kernel timing."""
+    lib = _lib.load()
+    lib.sepcorr_profile_enable(1)
+    try:
+        fn()
+        torch.cuda.synchronize()
+    finally:
+        names, ms = ctypes.create_string_buffer(1 << 14), (ctypes.c_float * 256)()
+        n = lib.sepcorr_profile_collect(names, len(names), ms, 256)
+        lib.sepcorr_profile_enable(0)
+    return set(names.value.decode().split("\n")[:n])
+
+
+@pytest.mark.parametrize("dims", SHAPES, ids=str)
+def test_sizes_take_the_split_sweep(device, dims):
+    f1, f2 = (torch.randn(dims[0], *hw, dims[5], device=device) for hw in (dims[1:3], dims[3:5]))
+    for argmax in (True, False):
+        for scratch in (True, False):
+            assert _labels_of(lambda: _max_avg(f1, f2, dims, scratch, argmax)) == {"fwd_maxavg_split"}
 
 
 def _call(name, outs, ins, dims, scratch, extra=(), K=2):
