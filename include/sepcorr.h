@@ -26,7 +26,8 @@
  *    device buffer of at least that size (256-byte aligned).  Its contents on entry are ignored.
  *  - Forward entry points take scratch memory optionally (sepcorr_forward_workspace_bytes(), 256-byte aligned,
  *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels with
- *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units (csrc/split_sweep.hip), every fp32 operand as two
+ *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units (csrc/split_sweep.hip; sepcorr_set_contraction()
+ *    can choose fp32 ones instead), every fp32 operand as two
  *    halves with a power-of-two scale per pixel: within 2^-22 of itself, or, where a channel is below 2^-28 of its pixel's largest,
  *    within 2^-50 of that (pixels with max(2, C/32) such channels are multiplied in fp32).  With fewer roundings of
  *    each sum the error of the results is below that of the fp32 sweep (C=256: 1.6e-7 against 3.0e-7); without a
@@ -69,7 +70,10 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap);
 /*
  * Arithmetic of the contractions of the forward sweeps (max/avg, max/argmax/avg, compression forward and the
  * attention-gradient pass of the compression backward) and of d_f1; no counterpart in the reference.
- *   SEPCORR_CONTRACT_FP32    fp32 MFMA (the initial choice).
+ *   SEPCORR_CONTRACT_SPLIT   forward sweeps of 32 <= C <= 256 channels and at least 1e9 of B H1 W1 H2 W2 (C + 64) with every
+ *                            fp32 operand as two 16-bit halves (the note on scratch memory above), fp32 MFMA
+ *                            elsewhere (the initial choice).
+ *   SEPCORR_CONTRACT_FP32    fp32 MFMA throughout.
  *   SEPCORR_CONTRACT_BF16X3  every fp32 operand is written exactly as the sum of three bf16 numbers and the
  *                            product taken as the six largest of the nine plane products, with bf16 MFMA
  *                            accumulating in fp32.  What is dropped is below 2^-24 of each product, so results
@@ -84,6 +88,7 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap);
  */
 #define SEPCORR_CONTRACT_FP32 0
 #define SEPCORR_CONTRACT_BF16X3 1
+#define SEPCORR_CONTRACT_SPLIT 2
 int sepcorr_set_contraction(int mode);
 
 /*
@@ -168,8 +173,8 @@ int sepcorr_max_argmax_avg_backward(const float *f1, const float *f2,
  * counterpart in the reference.  The scratch memory is an array of SEPCORR_STATIC_SCRATCH_BYTES bytes inside the
  * library's device image (one copy per GPU, held until the process ends) instead of a workspace argument; the
  * call allocates nothing, creates no streams or events and runs all its kernels on `stream`.
- *   - It always contracts in fp32: results are bit-equal to the workspace variant's under SEPCORR_CONTRACT_FP32 (the
- *     default); with sepcorr_set_contraction(SEPCORR_CONTRACT_BF16X3) the workspace variant's dense d_f1 takes the
+ *   - It always contracts in fp32: results are bit-equal to the workspace variant's (which runs no forward sweep) unless
+ *     SEPCORR_CONTRACT_BF16X3 is set; with sepcorr_set_contraction(SEPCORR_CONTRACT_BF16X3) the workspace variant's dense d_f1 takes the
  *     bf16-plane kernels (which allocate stream-ordered memory) and the two agree to rounding only.
  *   - Sizes that need more scratch than SEPCORR_STATIC_SCRATCH_BYTES are refused with SEPCORR_EWORKSPACE; use the
  *     workspace variant for them.  (Any size whose sepcorr_backward_workspace_bytes() fits is accepted; that figure

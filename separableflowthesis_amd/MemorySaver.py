@@ -729,7 +729,7 @@ def lookup1d_backward(coords, grad_out, shape, coord_channel, clamp_unit, num_le
     return d_corr
 
 
-CONTRACT_FP32, CONTRACT_BF16X3 = 0, 1
+CONTRACT_FP32, CONTRACT_BF16X3, CONTRACT_SPLIT = 0, 1, 2
 MAXAVG_AUTO, MAXAVG_DENSE, MAXAVG_GATHER = 0, 1, 2
 
 
@@ -742,8 +742,9 @@ def set_max_avg_backward(mode):
 
 
 def set_contraction(mode):
-    """Arithmetic of the forward sweeps' contraction: CONTRACT_FP32 (fp32 MFMA) or CONTRACT_BF16X3 (three bf16
-    planes per operand, fp32 accumulation; C == 256 only, fp32 elsewhere).  Process-wide; returns the previous mode.
-    Not a function of the reference."""
+    """Arithmetic of the forward sweeps' contraction: CONTRACT_SPLIT (initially; two 16-bit halves per operand where the
+    sizes suit, fp32 accumulation; fp32 MFMA elsewhere), CONTRACT_FP32 (fp32 MFMA throughout) or CONTRACT_BF16X3 (three
+    bf16 planes per operand, fp32 accumulation; C == 256 only, fp32 elsewhere).  Process-wide; returns the previous
+    mode.  Not a function of the reference."""
     return _lib.load().sepcorr_set_contraction(int(mode))
 

@@ -74,7 +74,7 @@ class AlternateCorrBlockSepflow:
         if (fused and attention_weights is not None
                 and (self.max_avg_function is ComputeMaxArgmaxAvgFunction or not torch.is_grad_enabled())
                 and 1 < self.num_levels <= 4 and self.pyramid_mode != "level"
-                and MemorySaver.set_contraction(-1) == MemorySaver.CONTRACT_FP32):
+                and MemorySaver.set_contraction(-1) != MemorySaver.CONTRACT_BF16X3):
             # the whole pyramid as one autograd node; the levels above level 0 share launches
             attention1, attention2 = attention_weights
             if (self.fmap1_l0.dtype == torch.float32 and self.fmap2_l0.dtype == torch.float32

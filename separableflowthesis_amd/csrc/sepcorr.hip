@@ -3150,7 +3150,7 @@ namespace sepcorr_impl {
 // stream capture too) or the pool has nothing left.
 template <int MODE, int KC>
 int try_split(const FwdArgs &a, int B, hipStream_t s) {
-    if (a.f2_planes) return 1;
+    if (a.f2_planes || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 1;
     SplitArgs p;
     memset(&p, 0, sizeof(p));
     p.f1 = a.f1; p.B = B; p.N1 = a.N1; p.C = a.C; p.KT = a.KT; p.k0 = a.k0; p.logits = a.logits; p.dlog = a.dlog;
@@ -3418,8 +3418,8 @@ int xcd_order_enabled() {
     return on;
 }
 
-// Contraction of the forward sweeps: fp32 MFMA, or three bf16 planes where the shape allows (C == 256, rows of at
-// most 256 columns).  sepcorr_set_contraction() selects;
+// Contraction of the forward sweeps: two 16-bit halves (split_sweep.hip) where the sizes suit, fp32 MFMA, or three
+// bf16 planes where the shape allows (C == 256, rows of at most 256 columns).  sepcorr_set_contraction() selects;
 // SEPCORR_BF16X3=1 in the environment makes the planes the initial choice.  fmap2 is split once per call into
 // stream-ordered memory that is released, in stream order, when the call returns.
 }  // namespace
@@ -3428,7 +3428,7 @@ namespace sepcorr_impl {
 std::atomic<int> g_maxavg_backward{SEPCORR_MAXAVG_AUTO};
 std::atomic<int> g_contraction{[] {
     const char *e = getenv("SEPCORR_BF16X3");
-    return e && e[0] == '1' ? SEPCORR_CONTRACT_BF16X3 : SEPCORR_CONTRACT_FP32;
+    return e && e[0] == '1' ? SEPCORR_CONTRACT_BF16X3 : SEPCORR_CONTRACT_SPLIT;
 }()};
 }  // namespace sepcorr_impl
 #endif
@@ -4099,7 +4099,7 @@ int sepcorr_set_max_avg_backward(int mode) {
 }
 
 int sepcorr_set_contraction(int mode) {
-    if (mode != SEPCORR_CONTRACT_FP32 && mode != SEPCORR_CONTRACT_BF16X3) return g_contraction.load();
+    if (mode != SEPCORR_CONTRACT_FP32 && mode != SEPCORR_CONTRACT_BF16X3 && mode != SEPCORR_CONTRACT_SPLIT) return g_contraction.load();
     return g_contraction.exchange(mode);
 }
 

@@ -42,6 +42,25 @@ def test_sizes_take_the_split_sweep(device, dims):
             assert _labels_of(lambda: _max_avg(f1, f2, dims, scratch, argmax)) == {"fwd_maxavg_split"}
 
 
+@pytest.mark.parametrize("mode,label", [("CONTRACT_FP32", "fwd_maxavg"), ("CONTRACT_BF16X3", "fwd_maxavg"), ("CONTRACT_SPLIT", "fwd_maxavg_split")])
+def test_contraction_modes(device, mode, label):
+    """fp32 products when they are asked for, also by the planes' mode where the planes do not apply (C = 128)."""
+    from separableflowthesis_amd import MemorySaver
+    dims = SHAPES[4]
+    f1, f2, _ = op_inputs(*dims, seed=13)
+    f1, f2 = f1.to(device), f2.to(device)
+    previous = MemorySaver.set_contraction(getattr(MemorySaver, mode))
+    try:
+        assert previous == MemorySaver.CONTRACT_SPLIT
+        for scratch in (True, False):
+            assert _labels_of(lambda: _max_avg(f1, f2, dims, scratch)) == {label}
+        B, H1, W1, H2, W2, _ = dims
+        a_u, a_v = (torch.randn(B, H1, W1, 2, n, device=device) for n in (W2, H2))
+        assert _labels_of(lambda: MemorySaver.compression_forward(f1, f2, a_u, a_v)) == {label.replace("maxavg", "weighted")}
+    finally:
+        MemorySaver.set_contraction(previous)
+
+
 def _call(name, outs, ins, dims, scratch, extra=(), K=2):
     lib = _lib.load()
     h2, w2 = (ctypes.c_int * 1)(dims[3]), (ctypes.c_int * 1)(dims[4])
