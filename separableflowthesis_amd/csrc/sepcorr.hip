@@ -3129,12 +3129,18 @@ size_t fwd_split_bytes(int B, int H1, int W1, int H2, int W2, int K) {
     return best;
 }
 
+// Scratch for any split sweep of up to K channels: a launch of fewer quantities can want more than one of many, since
+// the pixel range is cut into slabs by what a launch of its own kind leaves in scratch.
+size_t split_bytes(int B, int N1, const int *h2, const int *w2, int nlev, int C, int K) {
+    size_t n = std::max(sepcorr_split_sweep_bytes(B, N1, h2, w2, nlev, C, SPLIT_MAXAVG, 0),
+                        sepcorr_split_sweep_bytes(B, N1, h2, w2, nlev, C, SPLIT_ARGMAX, 0));
+    for (int kc = 1; kc <= KCH && kc <= K; ++kc) n = std::max(n, sepcorr_split_sweep_bytes(B, N1, h2, w2, nlev, C, SPLIT_WEIGHTED, kc));
+    return n;
+}
+
 // Scratch for any forward-type sweep of these sizes (K <= 2 also: max/average), whichever kernels run it.
 size_t sweep_bytes(int B, int H1, int W1, int H2, int W2, int C, int K) {
-    const size_t plain = fwd_split_bytes(B, H1, W1, H2, W2, K);
-    const size_t ma = split_sweep_bytes(B, H1 * W1, &H2, &W2, 1, C, SPLIT_ARGMAX, 0);
-    const size_t wt = split_sweep_bytes(B, H1 * W1, &H2, &W2, 1, C, SPLIT_WEIGHTED, K < KCH ? K : KCH);
-    return std::max(plain, std::max(ma, wt));
+    return std::max(fwd_split_bytes(B, H1, W1, H2, W2, K), split_bytes(B, H1 * W1, &H2, &W2, 1, C, K));
 }
 
 // What a forward entry point insists on when it is given a workspace: nothing where whole tiles fill the chip.
@@ -3170,7 +3176,7 @@ int try_split(const FwdArgs &a, int B, hipStream_t s) {
     if (rc == 1 && !t_no_alloc) {
         int h2[4], w2[4];
         for (int l = 0; l < p.nlev; ++l) { h2[l] = p.lev[l].H2; w2[l] = p.lev[l].W2; }
-        const size_t bytes = split_sweep_bytes(B, a.N1, h2, w2, p.nlev, a.C, mode, kc);
+        const size_t bytes = sepcorr_split_sweep_bytes(B, a.N1, h2, w2, p.nlev, a.C, mode, kc);
         hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
         void *ws = nullptr;
         if (bytes > 0 && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusNone &&
@@ -4426,9 +4432,7 @@ size_t levels_sweep_bytes(const int *h2, const int *w2, int nlev, int B, int H1,
         if (n > single) single = n;
     }
     const size_t multi = fwd_levels_bytes(B * ((H1 * W1 + TP - 1) / TP), nlev, w2max, K);
-    size_t n = std::max(multi, single);
-    n = std::max(n, split_sweep_bytes(B, H1 * W1, h2, w2, nlev, C, SPLIT_ARGMAX, 0));
-    n = std::max(n, split_sweep_bytes(B, H1 * W1, h2, w2, nlev, C, SPLIT_WEIGHTED, K < KCH ? K : KCH));
+    const size_t n = std::max(std::max(multi, single), split_bytes(B, H1 * W1, h2, w2, nlev, C, K));
     return (n + 255) & ~(size_t)255;
 }
 }  // namespace

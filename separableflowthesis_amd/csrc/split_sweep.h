@@ -38,8 +38,9 @@ struct SplitArgs {
     float *slots;
 };
 
-// Scratch split_sweep() wants, 0 where it does not take the sizes.  kc: channels of one launch (0: max/average).
-size_t split_sweep_bytes(int B, int N1, const int *h2, const int *w2, int nlev, int C, int mode, int kc);
+// Scratch split_sweep() wants, 0 where it does not take the sizes.  kc: channels of one launch (0: max/average).  (C
+// linkage: a host test holds the library's workspace queries against it.)
+extern "C" size_t sepcorr_split_sweep_bytes(int B, int N1, const int *h2, const int *w2, int nlev, int C, int mode, int kc);
 // Runs the sweep when the sizes suit it and ws_bytes suffice; returns 1 without launching anything otherwise, 0 when
 // it was launched, a negative SEPCORR_ code on error.
 int split_sweep(int mode, int kc, SplitArgs a, void *ws, size_t ws_bytes, hipStream_t s);

@@ -835,7 +835,7 @@ SplitPlan plan(int B, int N1, const int *h2, const int *w2, int nlev, int C, int
 }
 }  // namespace
 
-size_t split_sweep_bytes(int B, int N1, const int *h2, const int *w2, int nlev, int C, int mode, int kc) {
+size_t sepcorr_split_sweep_bytes(int B, int N1, const int *h2, const int *w2, int nlev, int C, int mode, int kc) {
     const SplitPlan p = plan(B, N1, h2, w2, nlev, C, mode, kc);
     return p.ok ? p.bytes() : 0;
 }

@@ -173,3 +173,47 @@ def test_missing_library_fails_loudly(monkeypatch):
     monkeypatch.setattr(_lib, "LIB_PATH", "/nonexistent/libsepcorr.so")
     with pytest.raises(RuntimeError, match="no CPU fallback"):
         _lib.load()
+
+
+MAXAVG, ARGMAX, WEIGHTED = 0, 1, 2   # of sepcorr_split_sweep_bytes
+
+
+def _split_bytes(lib, B, N1, sizes, C, mode, kc):
+    h2, w2 = (ctypes.c_int * len(sizes))(*(h for h, _ in sizes)), (ctypes.c_int * len(sizes))(*(w for _, w in sizes))
+    return lib.sepcorr_split_sweep_bytes(B, N1, h2, w2, len(sizes), C, mode, kc)
+
+
+def test_workspace_queries_cover_the_split_sweeps():
+    """What each entry point's query gives is enough for every sweep on 16-bit halves that the entry point launches: max/average,
+    with argmax, and the channel groups of K (of four, then the rest), over single levels and pyramids of square
+    correlations."""
+    lib = ctypes.CDLL(_lib.LIB_PATH)
+    for n, (r, a) in _lib.SIGNATURES.items():
+        getattr(lib, n).restype, getattr(lib, n).argtypes = r, a
+    lib.sepcorr_split_sweep_bytes.restype = ctypes.c_size_t
+    g = torch.Generator().manual_seed(0)
+    sizes = [(1, 67, 240), (1, 100, 180), (1, 104, 184), (1, 96, 172), (2, 116, 114), (4, 89, 99), (12, 40, 120)]
+    for _ in range(400):
+        r = torch.rand(3, generator=g)
+        sizes.append((int(12 ** r[0]), int(16 * (136 / 16) ** r[1]), int(24 * 10 ** r[2])))
+    taken = 0
+    for i, (B, H, W) in enumerate(sizes):
+        C = (256, 256, 100, 32)[i % 4] if i >= 7 else 256
+        dims, align = (B, H, W, H, W, C), lambda n: (n + 255) // 256 * 256
+        for levels in ([(H, W)], [(H >> l, W >> l) for l in range(4)]):
+            h2, w2 = (ctypes.c_int * len(levels))(*(h for h, _ in levels)), (ctypes.c_int * len(levels))(*(w for _, w in levels))
+            wanted = {K: [_split_bytes(lib, B, H * W, levels, C, WEIGHTED, kc) for kc in {min(K, 4), K % 4} - {0}] for K in range(1, 9)}
+            max_avg = [_split_bytes(lib, B, H * W, levels, C, mode, 0) for mode in (MAXAVG, ARGMAX)]
+            taken += max_avg[0] > 0
+            for K in range(1, 9):
+                need = max(wanted[K] + (max_avg if K == 2 else []))
+                dots = 2 * len(levels) * align(B * H * W * K * 4)
+                assert lib.sepcorr_forward_levels_workspace_bytes(h2, w2, len(levels), B, H, W, C, K) - dots >= need, (dims, levels, K)
+                if len(levels) == 1:
+                    one = lib.sepcorr_forward_workspace_bytes(*dims, K)
+                    assert one == 0 or one >= need, (dims, K)
+                    assert lib.sepcorr_backward_workspace_bytes(*dims) >= max(wanted[K]), (dims, K)
+                    for features in (0, 1):
+                        n = lib.sepcorr_compression_backward_from_logits_workspace_bytes(*dims, K, features)
+                        assert n - 2 * align(B * H * W * K * 4) >= max(wanted[K]), (dims, K, features)
+    assert taken > 200
