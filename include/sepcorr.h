@@ -27,15 +27,15 @@
  *  - Forward entry points take scratch memory optionally (sepcorr_forward_workspace_bytes(), 256-byte aligned,
  *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels with
  *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units (csrc/split_sweep.hip; sepcorr_set_contraction()
- *    can choose fp32 ones instead), every fp32 operand as two
- *    halves with a power-of-two scale per pixel: within 2^-22 of itself, or, where a channel is below 2^-28 of its pixel's largest,
- *    within 2^-50 of that (pixels with max(2, C/32) such channels are multiplied in fp32).  With fewer roundings of
- *    each sum the error of the results is below that of the fp32 sweep (C=256: 1.6e-7 against 3.0e-7); without a
- *    workspace (or with one smaller than sepcorr_forward_levels_workspace_bytes() of the one level) they take their
- *    scratch from the stream's memory pool, which costs host time on each call.  The other sizes, and calls without a workspace
- *    under stream capture, run the fp32 sweep: with a workspace it is dealt out in pieces smaller than a 32-pixel tile
- *    where whole tiles would leave compute units idle; with and without one the results differ only in the rounding
- *    of the sums over u.
+ *    can choose fp32 ones instead), every fp32 operand as two halves with a power-of-two scale per pixel: within 2^-22
+ *    of itself, or, where a channel is below 2^-28 of its pixel's largest, within 2^-50 of that (pixels with
+ *    max(2, C/32) such channels are multiplied in fp32).  With fewer roundings of each sum the error of the results is
+ *    below that of the fp32 sweep (C=256: 1.6e-7 against 3.0e-7).  Without a workspace (or with less than
+ *    sepcorr_forward_levels_workspace_bytes() of the one level) they take their scratch, up to some 200 MB, from the stream's
+ *    memory pool: 11 us of host time, and where the stream is waited for after each call 65 us, or 340 us beyond 64 MiB, of
+ *    mapping it anew.  The other sizes, and calls without a workspace under stream capture, run the fp32 sweep: with a
+ *    workspace it is dealt out in pieces smaller than a 32-pixel tile where whole tiles would leave compute units idle;
+ *    with and without one the results differ only in the rounding of the sums over u.
  */
 #ifndef SEPCORR_H
 #define SEPCORR_H
@@ -121,8 +121,8 @@ int sepcorr_max_avg_forward(const float *f1, const float *f2, float *out_u, floa
                             void *workspace, size_t workspace_bytes, void *stream);
 
 /* Scratch bytes a forward entry point can make use of for these sizes (K = 2 for the max/avg entry points); 0 when
- * whole 32-pixel tiles already fill the chip.  sepcorr_forward_levels_workspace_bytes() with one level gives what the
- * sweep on the 16-bit matrix units takes at those sizes too. */
+ * whole 32-pixel tiles already fill the chip and the sweep on 16-bit halves is not taken or takes so long (0.5 ms and more) that
+ * the memory pool serves (to give it a workspace all the same ask sepcorr_forward_levels_workspace_bytes() with one level). */
 size_t sepcorr_forward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C, int K);
 
 /*

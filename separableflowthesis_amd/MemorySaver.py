@@ -60,9 +60,10 @@ def _workspace(lib, dims, device):
 def _fwd_workspace(lib, dims, K, device):
     """Optional scratch of the forward-type sweeps (the split operands of the 16-bit matrix units; pieces of tiles)."""
     n = lib.sepcorr_forward_workspace_bytes(*dims, K)
-    if n == 0:   # (whole tiles fill the chip: only the sweep with split operands can use any)
+    if n == 0:
         B, H1, W1, H2, W2, C = dims
-        if not 32 <= C <= 256:
+        # (from here on the sweep with split operands would take its scratch from the stream's memory pool)
+        if not 32 <= C <= 256 or B * H1 * W1 * H2 * W2 * (C + 64) < 1e11:
             return None, None, 0
         n = lib.sepcorr_forward_levels_workspace_bytes((ctypes.c_int * 1)(H2), (ctypes.c_int * 1)(W2), 1, B, H1, W1, C, K)
     ws = torch.empty(n, dtype=torch.uint8, device=device)

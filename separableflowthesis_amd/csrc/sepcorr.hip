@@ -3143,6 +3143,12 @@ size_t sweep_bytes(int B, int H1, int W1, int H2, int W2, int C, int K) {
     return std::max(fwd_split_bytes(B, H1, W1, H2, W2, K), split_bytes(B, H1 * W1, &H2, &W2, 1, C, K));
 }
 
+// Up to this much work (pairs of pixels times channels + 64) the query gives what a split sweep takes also where the fp32 sweep
+// would want nothing: taking it from the memory pool instead (try_split) costs a caller who waits for the stream between the
+// calls up to 0.34 ms.  Larger sweeps take 0.5 ms and more.
+[[maybe_unused]] constexpr double kQueryWork = 1e11;
+double sweep_work(int B, int N1, int H2, int W2, int C) { return (double)B * N1 * H2 * W2 * (C + 64); }
+
 // What a forward entry point insists on when it is given a workspace: nothing where whole tiles fill the chip.
 size_t fwd_need(int B, int H1, int W1, int H2, int W2, int C, int K) {
     return fwd_split_bytes(B, H1, W1, H2, W2, K) > 0 ? sweep_bytes(B, H1, W1, H2, W2, C, K) : 0;
@@ -3153,7 +3159,10 @@ namespace sepcorr_impl {
 // The sweep on the 16-bit matrix units (split_sweep.hip), where it takes the sizes: 0 launched, 1 not taken, negative on
 // error.  A caller who gives no scratch, or less than it takes, gets the same sweep, its scratch from the stream's memory pool for the length of
 // the call, so that the results do not depend on the workspace; the fp32 sweep runs where nothing may be allocated (under
-// stream capture too) or the pool has nothing left.
+// stream capture too) or the pool has nothing left.  Taking and returning the scratch costs 11 us of host time, but when
+// the stream is waited for between the calls its mapping is paid for every time: 65 us up to 64 MiB, 340 us above, in
+// one piece or several.  Waited for like that, max/average at C=256 (fp32 sweep without scratch / this one): 48x64 127 / 107 us,
+// B=4, 48x64 228 / 429, B=2, 55x128 471 / 523, 100x180 2406 / 861; not waited for 115 / 45, 225 / 92, 456 / 184, 2387 / 518.
 template <int MODE, int KC>
 int try_split(const FwdArgs &a, int B, hipStream_t s) {
     if (a.f2_planes || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 1;
@@ -4137,7 +4146,8 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap) {
 
 size_t sepcorr_forward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C, int K) {
     if (B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1 || K < 1) return 0;
-    return fwd_need(B, H1, W1, H2, W2, C, K);
+    const size_t need = fwd_need(B, H1, W1, H2, W2, C, K);
+    return need == 0 && sweep_work(B, H1 * W1, H2, W2, C) < kQueryWork ? split_bytes(B, H1 * W1, &H2, &W2, 1, C, K) : need;
 }
 
 int sepcorr_max_avg_forward(const float *f1, const float *f2, float *out_u, float *out_v, int B, int H1, int W1, int H2,
@@ -4502,7 +4512,7 @@ int soft_levels(const float *f1, const float *const *f2, const int *h2, const in
             case 3: rc = launch_fwd_levels<MODE_SOFT, 3, 1>(a, B, s); break;
             default: rc = launch_fwd_levels<MODE_SOFT, 4, 1>(a, B, s); break;
         }
-        if (rc == SEPCORR_EINVAL && k0 == 0) one_launch = false;   // shapes outside the one-launch path
+        if (rc == SEPCORR_EINVAL) one_launch = false;   // shapes outside the one-launch path (or no scratch left for these channels)
         else if (rc) return rc;
     }
     if (one_launch) return SEPCORR_OK;
