@@ -3662,7 +3662,9 @@ Df1Shape df1_shape(const Dims &d) {
 // Layout of a backward call's workspace.  Regions: split partial sums of d_f2; transposed (p,u) weights of d_f1 and,
 // behind them, the pieces of a split d_f1; scratch of the weight-gradient sweep (a forward-type sweep).  When any
 // kernel is dealt out in pieces the call keeps to one stream (such kernels want the whole chip), its kernels run one
-// after the other, and the regions of different kernels share the same memory.
+// after the other, and the regions of different kernels share the same memory; so too where the sweep runs on 16-bit halves,
+// which always takes scratch.  (Whole tiles, d_f1 and d_f2 beside each other / after each other: compression backward B=4,
+// 64x64, C=256 783 / 746 us, C=128 512 / 474; fused backward 759 / 702 and 536 / 450; at no measured size worse.)
 struct BwdWs {
     bool aliased;
     size_t off_uwt, off_df1sk, fwd_bytes, own_total, total;   // own_total: without the weight-gradient sweep
@@ -4060,6 +4062,15 @@ bool gather_overlap(const Dims &d) {
     return rows >= 300000 && (size_t)d.H2 * d.W2 * d.C * 4 <= ((size_t)4 << 20);
 }
 
+// Whether d_f1 and d_f2 of the dense max/avg backward run beside each other: unless one of them is dealt out in pieces, and
+// with C > 128 not where the weight gradients' sweep would have scratch either.  Measured (beside / after each other): C=128
+// B=4, 64x64 327 / 359 us, B=8, 64x64 611 / 692, B=6, 72x112 2086 / 2351, 96x168 1535 / 1467; C=256 649 / 608, 1181 / 1174,
+// 3962 / 3942, 3141 / 2940.  (Up to 128 channels d_f1 in whole tiles uses no scratch: nothing is shared.)
+bool dense_overlap(const Dims &d) {
+    if (!bwd_ws(d).aliased) return true;
+    return d.C <= 128 && df1_shape(d).bytes == 0 && fwd_split_bytes(d.B, d.H1, d.W1, d.H2, d.W2, MAX_K) == 0;
+}
+
 int maxavg_backward(const Dims &d, bool gather, const float *f1, const float *f2, const int32_t *am_u, const int32_t *am_v,
                     const float *g_u, const float *g_v, float *d_f1, float *d_f2, void *ws, hipStream_t s1, hipStream_t s,
                     hipStream_t s2 = nullptr, hipEvent_t s2_done = nullptr) {
@@ -4212,7 +4223,7 @@ int sepcorr_max_argmax_avg_backward(const float *f1, const float *f2, const int3
     if (int rc = check_dims(d, 2)) return rc;
     if (int rc = check_workspace(d, workspace, workspace_bytes)) return rc;
     const bool gather = maxavg_by_gather(d);
-    ForkJoin fj(static_cast<hipStream_t>(stream), gather ? gather_overlap(d) : !bwd_ws(d).aliased);
+    ForkJoin fj(static_cast<hipStream_t>(stream), gather ? gather_overlap(d) : dense_overlap(d));
     // d_f1 aside, d_f2 on the caller's stream
     // the join event of side stream b serves as "table ready" in between: nothing else is recorded on b before the join
     const int rc = maxavg_backward(d, gather, f1, f2, argmax_u, argmax_v, grad_u, grad_v, d_f1, d_f2, workspace, fj.sa, fj.user,

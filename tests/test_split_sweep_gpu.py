@@ -265,3 +265,23 @@ def test_small_features_keep_their_accuracy(device):
     out_u, out_v = (t.cpu() for t in _max_avg(f1.to(device), f2.to(device), dims)[:2])
     assert ((out_u[:, :, :, 0] - vol.amax(4)).abs() <= err.amax(4)).all()
     assert ((out_v[:, :, :, 1] - vol.mean(3)).abs() <= err.mean(3)).all()
+
+
+@pytest.mark.parametrize("dims", [(4, 64, 64, 64, 64, 128), (8, 32, 64, 33, 61, 100), (4, 64, 64, 16, 64, 64)], ids=str)
+def test_dense_max_avg_backward_on_two_streams(device, dims):
+    """Whole tiles and up to 128 channels: d_f1 and d_f2 run beside each other with the workspace that they would share
+    otherwise.  The same bits as one after the other (as the library's kernel timing runs them)."""
+    from separableflowthesis_amd import MemorySaver
+    B, H1, W1, H2, W2, C = dims
+    f1, f2 = (torch.randn(B, *hw, C, device=device) for hw in ((H1, W1), (H2, W2)))
+    _, _, am_u, am_v = _max_avg(f1, f2, dims)
+    g_u, g_v = (torch.randn(B, H1, W1, 2, n, device=device) for n in (H2, W2))
+    previous = MemorySaver.set_max_avg_backward(MemorySaver.MAXAVG_DENSE)
+    try:
+        call = lambda: MemorySaver.max_argmax_avg_backward(f1, f2, am_u, am_v, g_u, g_v)
+        serial = []
+        _labels_of(lambda: serial.extend(call()))
+        for _ in range(5):
+            assert all(torch.equal(a, b) for a, b in zip(call(), serial))
+    finally:
+        MemorySaver.set_max_avg_backward(previous)
