@@ -26,8 +26,8 @@
  *    device buffer of at least that size (256-byte aligned).  Its contents on entry are ignored.
  *  - Forward entry points take scratch memory optionally (sepcorr_forward_workspace_bytes(), 256-byte aligned,
  *    contents on entry ignored; NULL is allowed).  Sweeps of 32 <= C <= 256 channels with
- *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units (csrc/split_sweep.hip; sepcorr_set_contraction()
- *    can choose fp32 ones instead), every fp32 operand as two halves with a power-of-two scale per pixel: within 2^-22
+ *    B H1 W1 H2 W2 (C + 64) >= 1e9 run on the 16-bit matrix units (csrc/split_sweep.hip, which has an exception for three
+ *    weight channels at C = 32; sepcorr_set_contraction() can choose fp32 ones instead), every fp32 operand as two halves with a power-of-two scale per pixel: within 2^-22
  *    of itself, or, where a channel is below 2^-28 of its pixel's largest, within 2^-50 of that (pixels with
  *    max(2, C/32) such channels are multiplied in fp32).  With fewer roundings of each sum the error of the results is
  *    below that of the fp32 sweep (C=256: 1.6e-7 against 3.0e-7).  Without a workspace (or with less than

@@ -159,9 +159,16 @@ __device__ __forceinline__ void store_v(const SplitArgs &a, const SplitLevel &L,
         dst = L.out_v + row * W2 + v;
         if (a.dlog) {
             const float m = L.st_ov[2 * row], il = 1.f / L.st_ov[2 * row + 1], dot = L.dot_ov[row];
+            v4f z = {0.f, 0.f, 0.f, 0.f};
+            if (v + 4 <= W2) {
+                __builtin_memcpy(&z, L.z_ov + row * W2 + v, 16);
+            } else {
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
-                if (v + e < W2) x[e] = __expf(L.z_ov[row * W2 + v + e] - m) * il * (x[e] - dot);
+                for (int e = 0; e < 4; ++e)
+                    if (v + e < W2) z[e] = L.z_ov[row * W2 + v + e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) x[e] = __expf(z[e] - m) * il * (x[e] - dot);
         }
     } else if (MODE == SPLIT_ARGMAX && q == 2) {
         dst = reinterpret_cast<float *>(L.am_v + bp * W2 + v);
@@ -169,8 +176,11 @@ __device__ __forceinline__ void store_v(const SplitArgs &a, const SplitLevel &L,
         dst = L.out_v + (bp * 2 + q) * W2 + v;
         if (q == 1) x = x / (float)L.H2;
     }
-    if ((W2 & 3) == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0) {
-        *reinterpret_cast<v4f *>(dst) = x;
+    // (16 bytes at a 4-byte aligned address: rows of any length.  Four stores of 4 bytes in rows that are not a multiple of 4 long
+    // cost a piece some 10 us: B=3, four levels of 47x115, C=56, K=4 450 us, 410 us like this, 350 with the fp32 sweep; C=256,
+    // K=2 over four levels of 47x156 229 and 217.)
+    if (v + 4 <= W2) {
+        __builtin_memcpy(dst, &x, 16);
     } else {
 #pragma unroll
         for (int e = 0; e < 4; ++e)
@@ -367,20 +377,21 @@ __global__ void __launch_bounds__(256) split_finish_kernel(const SplitArgs a) {
 }
 #endif
 
-// The max/avg modes and one weight channel fit 256 registers: two workgroups per compute unit, one wave's reductions run
-// beside the other's matrix work.  More channels take the whole register file, and a wave reduces one row while it
-// multiplies the next.  Both ways measured at C=256: max/avg, B=2, 55x128 0.149 ms with two workgroups and 0.166 with one;
-// two channels over the four levels of 47x156 0.225 and 0.212.
-__host__ __device__ constexpr bool pipelined(int mode, int kc) { return mode == SPLIT_WEIGHTED && kc > 1; }
+// The max/avg modes and one weight channel fit 256 registers, and so do two channels where a pixel's halves take few (C <= 64):
+// two workgroups per compute unit, one wave's reductions run beside the other's matrix work.  More channels take the whole
+// register file, and a wave reduces one row while it multiplies the next.  Both ways measured (two workgroups / one): C=256
+// max/avg, B=2, 55x128 0.149 / 0.166 ms, two channels over the four levels of 47x156 0.225 / 0.212; C=64 two channels B=4, 80x120
+// 0.270 / 0.342, four 0.895 / 0.521; C=100 two channels B=2, 47x61 0.054 / 0.046.
+__host__ __device__ constexpr bool pipelined(int mode, int kc, int nk) { return mode == SPLIT_WEIGHTED && kc > 1 && !(kc == 2 && nk == 4); }
 
 // NK: channel steps of 16 (C <= 16 NK, the rest zeros).  Measured at B=2, 55x128, C=256: max/avg/argmax 0.454 ms with the
 // fp32 sweep, 0.149 ms here (+ 0.013 split_prepare_kernel, 0.032 split_finish_kernel); four weighted sums 0.474 and
 // 0.192 ms (+ 0.013 and 0.034).  The matrix instructions alone take 0.061 ms at 2.4 GHz; what is left is the vector work
 // of the reductions, the reads of the row block from LDS and the beginning and end of every step.
 template <int MODE, int KC, int NK>
-__global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_kernel(const SplitArgs a) {
+__global__ void __launch_bounds__(256, pipelined(MODE, KC, NK) ? 1 : 2) split_sweep_kernel(const SplitArgs a) {
     constexpr bool WT = MODE == SPLIT_WEIGHTED;
-    constexpr bool PIPE = pipelined(MODE, KC);
+    constexpr bool PIPE = pipelined(MODE, KC, NK);
     constexpr int Q = WT ? KC : (MODE == SPLIT_ARGMAX ? 3 : 2);
     constexpr int BLK = block_bytes(NK), BF = BLK / 4, NBUF = PIPE ? 3 : 2;
     // The low halves' products are summed apart, in units of LOW_UNIT.  The max/avg modes have no registers left for a second
@@ -444,7 +455,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
             const __amdgpu_buffer_rsrc_t rw = make_rsrc(L.wv + ((size_t)b * N1 + min((a.pt0 + pt) * TPX, N1 - 1)) * a.KT * W2,
                                                         (unsigned)min(TPX, N1 - (a.pt0 + pt) * TPX) * a.KT * W2 * 4u);
             const unsigned row0 = ((32 * wave + pl) * a.KT + a.k0) * W2;
-            if ((W2 & 3) == 0) {
+            if ((W2 & 3) == 0 || 32 * vc + 32 <= W2) {   // (loads of 16 bytes need 4-byte alignment only)
 #pragma unroll
                 for (int k = 0; k < KC; ++k)
 #pragma unroll
@@ -748,7 +759,7 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC) ? 1 : 2) split_sweep_
 
 template <int MODE, int KC>
 int launch_sweep(const SplitArgs &a, int nk, hipStream_t s) {
-    const size_t lds = (pipelined(MODE, KC) ? 3 : 2) * (size_t)block_bytes(nk) + (MODE == SPLIT_WEIGHTED ? 4 * KC * 128 * sizeof(float) : 0);
+    const size_t lds = (pipelined(MODE, KC, nk) ? 3 : 2) * (size_t)block_bytes(nk) + (MODE == SPLIT_WEIGHTED ? 4 * KC * 128 * sizeof(float) : 0);
     auto k = nk == 4 ? split_sweep_kernel<MODE, KC, 4> : nk == 8 ? split_sweep_kernel<MODE, KC, 8> : split_sweep_kernel<MODE, KC, 16>;
     if (lds > 64 * 1024 &&
         hipFuncSetAttribute(reinterpret_cast<const void *>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
@@ -798,7 +809,7 @@ struct SplitPlan {
     size_t bytes() const { return planes + part + slots; }
 };
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
-int places(int mode, int kc) { return pipelined(mode, kc) ? kPlaces : 2 * kPlaces; }
+int places(int mode, int kc, int nk) { return pipelined(mode, kc, nk) ? kPlaces : 2 * kPlaces; }
 
 SplitPlan plan(int B, int N1, const int *h2, const int *w2, int nlev, int C, int mode, int kc) {
     SplitPlan p = {};
@@ -819,17 +830,22 @@ SplitPlan plan(int B, int N1, const int *h2, const int *w2, int nlev, int C, int
     p.npt_slab = (p.npt + p.slabs - 1) / p.slabs;
     const long steps = blocks * p.npt_slab;
     // The three launches and the hand-over through scratch take 26 us at the least, the fp32 sweep two launches and its
-    // matrix work.  Measured (fp32 sweep / this one, max/average): B=1, 24x64, C=256 37.5 / 33.2 us, B=4, 20x40 37.6 /
-    // 38.6, B=2, 32x64 54 / 39; C=72 24x64 28.0 / 27.8, B=2, 32x64 34.6 / 29.2; C=32 B=2, 32x64 29.8 / 29.0, 47x90 52 / 40:
-    // the line lies where pairs (C + 64) reach 1e9 (3.1 million pairs at C=256, 10 million at C=32).
+    // matrix work.  This sweep's time over the fp32 sweep's, three shapes each, at pairs (C + 64) = 0.4e9, 0.8e9, 1.3e9:
+    // max/average C=32 0.84-1.06, 0.76-0.88, 0.73-0.85; C=128 0.64-0.84, 0.72-0.75, 0.57-0.65; C=256 0.89-1.12, 0.67-0.81,
+    // 0.65-0.75; four channels C=32 0.98-1.08, 0.83-0.92, 0.82-1.01; C=128 0.70-0.84, 0.80-0.86, 0.65-0.76; C=256
+    // 0.97-1.24, 0.76-0.94, 0.81-0.87; four levels are 0.3 to 0.9 from 0.7e9 on.  Above the line, in 402 shapes of up to 64
+    // channels with two to four weight channels the median is 0.66; slower by more than 2 % are three or four channels
+    // of some pyramids (16 of 190, at the most 1.21: B=12, 29x41, C=32, K=3: pieces of few rows) and, on a single level, three
+    // channels at C=32 (0.89 to 1.13, on average 1.0): these stay with the fp32 sweep.
     if (pairs * (C + 64) < 1e9) return p;
+    if (mode == SPLIT_WEIGHTED && kc == 3 && C % 32 == 0 && C < 64 && nlev == 1) return p;
     for (int l = 0; l < nlev; ++l)
         if ((size_t)h2[l] * block_bytes(p.nk) >= (1u << 30)) return p;
     if (steps > (1L << 30) || blocks > (1L << 24)) return p;
     p.planes = align256((size_t)B * ((N1 + 31) / 32) * block_bytes(p.nk));
     for (int l = 0; l < nlev; ++l) p.planes += align256((size_t)B * ((w2[l] + 31) / 32) * h2[l] * block_bytes(p.nk));
     p.part = align256(per_pt * p.npt_slab) + 4 * 256;
-    p.slots = (size_t)2 * places(mode, kc) * p.q * 4096 * sizeof(float);
+    p.slots = (size_t)2 * places(mode, kc, p.nk) * p.q * 4096 * sizeof(float);
     p.ok = true;
     return p;
 }
@@ -876,7 +892,7 @@ int split_sweep(int mode, int kc, SplitArgs a, void *ws, size_t ws_bytes, hipStr
             a.fin_blocks += a.B * 2 * a.npt * ((L.H2 + 31) / 32);
             pp += ((size_t)a.B * L.nvc * L.H2 * p.q * a.npt * TPX + 63) & ~(size_t)63;
         }
-        const int G = places(mode, kc);
+        const int G = places(mode, kc, p.nk);
         a.G = a.steps < G ? a.steps : G;
         int rc;
         if (mode == SPLIT_MAXAVG) rc = split_launch_maxavg(a, p.nk, s);

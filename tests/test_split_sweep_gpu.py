@@ -42,6 +42,20 @@ def test_sizes_take_the_split_sweep(device, dims):
             assert _labels_of(lambda: _max_avg(f1, f2, dims, scratch, argmax)) == {"fwd_maxavg_split"}
 
 
+def test_three_channels_of_32_features_stay_fp32(device):
+    from separableflowthesis_amd import MemorySaver
+    B, H1, W1, H2, W2, C = dims = SHAPES[0]
+    f1, f2 = (torch.randn(B, *hw, C, device=device) for hw in (dims[1:3], dims[3:5]))
+    for K, labels in ((2, {"fwd_weighted_split"}), (3, {"fwd_weighted"}), (4, {"fwd_weighted_split"}), (7, {"fwd_weighted", "fwd_weighted_split"})):
+        a_u, a_v = (torch.randn(B, H1, W1, K, n, device=device) for n in (W2, H2))
+        got = []
+        assert _labels_of(lambda: got.extend(MemorySaver.compression_forward(f1, f2, a_u, a_v))) == labels
+        vol = _volume(f1.double(), f2.double())
+        for k in range(K):
+            assert torch.allclose(got[0][:, :, :, k].double(), (vol * a_u[:, :, :, k, None, :]).sum(4), rtol=1e-4, atol=1e-4)
+            assert torch.allclose(got[1][:, :, :, k].double(), (vol * a_v[:, :, :, k, :, None]).sum(3), rtol=1e-4, atol=1e-4)
+
+
 @pytest.mark.parametrize("mode,label", [("CONTRACT_FP32", "fwd_maxavg"), ("CONTRACT_BF16X3", "fwd_maxavg"), ("CONTRACT_SPLIT", "fwd_maxavg_split")])
 def test_contraction_modes(device, mode, label):
     """fp32 products when they are asked for, also by the planes' mode where the planes do not apply (C = 128)."""
@@ -110,7 +124,7 @@ def test_max_argmax_avg(device, dims):
 
 
 @pytest.mark.parametrize("K", [1, 2, 3, 4, 5])
-@pytest.mark.parametrize("dims", SHAPES[1::2], ids=str)
+@pytest.mark.parametrize("dims", SHAPES[1::2] + [(2, 45, 48, 46, 53, 64), (2, 45, 48, 46, 66, 40)], ids=str)
 def test_weighted(device, dims, K):
     B, H1, W1, H2, W2, C = dims
     f1, f2, g = op_inputs(*dims, seed=6)
