@@ -1,14 +1,18 @@
 """Sweeps dealt out in pieces of tiles against the same sweeps run tile by tile, under memory traffic from a second stream.
 
-With a workspace the forward-type sweeps (and d_f1) cut a pixel tile's rows into pieces that different workgroups take;
-a piece leaves its column state in a slot in device memory, counts itself in, and whichever piece of a tile arrives last
-adds up all pieces in row order.  Without a workspace every workgroup sweeps whole tiles and nothing is handed over.
+With a workspace the fp32 forward-type sweeps (and d_f1) cut a pixel tile's rows into pieces that different workgroups
+take; a piece leaves its column state in a slot in device memory, counts itself in, and whichever piece of a tile arrives
+last adds up all pieces in row order.  Without a workspace every workgroup sweeps whole tiles and nothing is handed over.
+The sweeps on 16-bit halves, which larger sizes run unless fp32 products are asked for, leave their pieces to a kernel of
+their own and take the same scratch from the memory pool when they are given none; the same calls must agree there too.
 Maxima and argmax must come out bit-equal either way (the merge keeps the lower row on ties, as the unsplit sweep does);
 sums differ by the rounding of a different association only.  The hand-over relies on stores and loads that go through
 to device memory and on a device-scope atomic counter; the launches below run it 200 times per size while another
 stream of the same GPU streams a buffer through the memory system, and stop at the first difference.
 Called through the C ABI.
 """
+import ctypes
+
 import pytest
 import torch
 
@@ -20,8 +24,38 @@ pytestmark = pytest.mark.gpu
 LAUNCHES = 200
 
 
-@pytest.mark.parametrize("dims", [(1, 48, 64, 48, 64, 256), (2, 55, 128, 55, 128, 256)], ids=["cfg1", "cfg4"])
-def test_split_and_unsplit_sweeps_agree_under_memory_traffic(device, dims):
+@pytest.fixture(params=["split", "fp32"])
+def contraction(request):
+    """Runs a test with the initial choice of arithmetic and with fp32 products throughout."""
+    from separableflowthesis_amd import MemorySaver
+    previous = MemorySaver.set_contraction(MemorySaver.CONTRACT_FP32 if request.param == "fp32" else MemorySaver.CONTRACT_SPLIT)
+    yield request.param
+    MemorySaver.set_contraction(previous)
+
+
+def _takes_halves(dims):
+    B, H1, W1, H2, W2, C = dims
+    return 32 <= C <= 256 and B * H1 * W1 * H2 * W2 * (C + 64) >= 1e9
+
+
+def _labels_of(fn):
+    lib = _lib.load()
+    lib.sepcorr_profile_enable(1)
+    try:
+        fn()
+        torch.cuda.synchronize()
+    finally:
+        names, ms = ctypes.create_string_buffer(1 << 14), (ctypes.c_float * 256)()
+        n = lib.sepcorr_profile_collect(names, len(names), ms, 256)
+        lib.sepcorr_profile_enable(0)
+    return set(names.value.decode().split("\n")[:n])
+
+
+@pytest.mark.parametrize("dims", [(1, 48, 64, 48, 64, 256), (2, 55, 128, 55, 128, 256), (1, 24, 32, 24, 32, 256), (1, 33, 57, 31, 90, 300)],
+                         ids=["cfg1", "cfg4", "24x32", "C300"])
+def test_split_and_unsplit_sweeps_agree_under_memory_traffic(device, dims, contraction):
+    if contraction == "fp32" and not _takes_halves(dims):
+        pytest.skip("these sizes run fp32 products either way")
     lib = _lib.load()
     B, H1, W1, H2, W2, C = dims
     f1, f2, g = op_inputs(*dims, seed=31)
@@ -47,6 +81,8 @@ def test_split_and_unsplit_sweeps_agree_under_memory_traffic(device, dims):
         _lib.check(lib.sepcorr_compression_forward(P(f1), P(f2), P(a_u), P(a_v), P(cu), P(cv), *dims, K, wptr, n, main.cuda_stream))
         return cu, cv
 
+    suffix = "_split" if contraction == "split" and _takes_halves(dims) else ""
+    assert _labels_of(lambda: (maxavg(P(ws), nws), weighted(P(ws), nws))) == {"fwd_maxavg" + suffix, "fwd_weighted" + suffix}
     # the reference results: whole tiles, no hand-over, idle chip
     rou, rov, rau, rav = maxavg(None, 0)
     rcu, rcv = weighted(None, 0)
@@ -117,9 +153,9 @@ def test_split_d_f1_agrees_with_itself_under_memory_traffic(device):
 
 
 @pytest.mark.parametrize("dims", [(1, 55, 128, 55, 128, 256), (1, 48, 64, 48, 64, 256)], ids=["cfg3", "cfg1"])
-def test_sweep_with_and_without_scratch(device, dims):
-    """The shape of the workgroups depends on whether the steps are dealt out (scratch given: two 4-wave workgroups per
-    CU) or whole tiles are swept (no scratch: 8 waves): same maxima and argmax, sums to rounding.  A buffer smaller
+def test_sweep_with_and_without_scratch(device, dims, contraction):
+    """The shape of the fp32 sweep's workgroups depends on whether the steps are dealt out (scratch given: two 4-wave
+    workgroups per CU) or whole tiles are swept (no scratch: 8 waves): same maxima and argmax, sums to rounding.  A buffer smaller
     than sepcorr_forward_workspace_bytes() is refused, not silently ignored."""
     lib = _lib.load()
     B, H1, W1, H2, W2, C = dims

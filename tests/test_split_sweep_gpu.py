@@ -1,8 +1,8 @@
 """Forward-type sweeps whose operands are split into two 16-bit halves (csrc/split_sweep.hip) against float64.
 
 Sizes at the edges of its tiles: pixels around multiples of 128, columns around multiples of 32, channels around the
-16/64/128/256 its channel steps are padded to, and pixels it cannot split (inf, NaN, magnitudes outside [2^-24, 2^24)),
-which it multiplies in fp32.
+16/64/128/256 its channel steps are padded to, and pixels it cannot split (inf, NaN, magnitudes outside [2^-60, 2^61),
+several channels far below the largest), which it multiplies in fp32.
 """
 import ctypes
 
@@ -10,7 +10,7 @@ import pytest
 import torch
 
 from separableflowthesis_amd import _lib
-from tests._util import op_inputs
+from tests._util import assert_close, op_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -299,3 +299,135 @@ def test_dense_max_avg_backward_on_two_streams(device, dims):
             assert all(torch.equal(a, b) for a, b in zip(call(), serial))
     finally:
         MemorySaver.set_max_avg_backward(previous)
+
+
+@pytest.mark.parametrize("K", [1, 3, 4])
+@pytest.mark.parametrize("dims", [SHAPES[2], SHAPES[6], SHAPES[7], (2, 45, 48, 46, 66, 40)], ids=str)
+def test_softmax_inside(device, dims, K):
+    """Weights from logits and gradients of the logits, rows of odd length and of 2 more than a multiple of 4."""
+    from separableflowthesis_amd import MemorySaver as ms
+    B, H1, W1, H2, W2, C = dims
+    f1, f2, g = op_inputs(*dims, seed=14)
+    z_u, z_v = 3 * torch.randn(B, H1, W1, K, W2, generator=g), 3 * torch.randn(B, H1, W1, K, H2, generator=g)
+    g_cu, g_cv = torch.randn(B, H1, W1, K, H2, generator=g), torch.randn(B, H1, W1, K, W2, generator=g)
+    f1, f2, z_u, z_v, g_cu, g_cv = (t.to(device) for t in (f1, f2, z_u, z_v, g_cu, g_cv))
+    labels = _labels_of(lambda: ms.compression_forward_from_logits(f1, f2, z_u, z_v))
+    assert "fwd_weighted_split" in labels
+    cu, cv, st_u, st_v = ms.compression_forward_from_logits(f1, f2, z_u, z_v)
+    dz_u, dz_v = ms.compression_backward_from_logits(f1, f2, z_u, z_v, st_u, st_v, cu, cv, g_cu, g_cv, need_features=False)[2:]
+    vol = _volume(f1.double(), f2.double())
+    a_u, a_v = z_u.double().softmax(-1), z_v.double().softmax(-1)
+    over_v = lambda w: torch.stack([(vol * w[:, :, :, k, None, :]).sum(4) for k in range(K)], 3)
+    over_u = lambda w: torch.stack([(vol * w[:, :, :, k, :, None]).sum(3) for k in range(K)], 3)
+    assert_close(cu.cpu(), over_v(a_u).cpu(), "compression_output_u")
+    assert_close(cv.cpu(), over_u(a_v).cpu(), "compression_output_v")
+    for got, a, d, name in ((dz_u, a_u, over_u(g_cu.double()), "d_logits_u"), (dz_v, a_v, over_v(g_cv.double()), "d_logits_v")):
+        assert_close(got.cpu(), (a * (d - (a * d).sum(-1, keepdim=True))).cpu(), name, scale_atol=True)
+
+
+def test_levels_with_pixels_without_halves(device):
+    """Every level of a pyramid in one launch, pixels of image 1 and of each level that are multiplied in fp32."""
+    from separableflowthesis_amd import MemorySaver as ms
+    B, H, W, C = 2, 41, 67, 72
+    f1, f2, _ = op_inputs(B, H, W, H, W, C, seed=15)
+    levels = [f2[:, :H >> l, :W >> l].contiguous() for l in range(4)]
+    f1[1, 20, 33, 5], f1[0, 40, 66, 71] = float("nan"), 2.0 ** 70
+    for l, value in enumerate((float("inf"), 2.0 ** 64, float("nan"), 2.0 ** -70)):
+        levels[l][l % 2, (H >> l) - 1, (W >> l) - 1] *= 2.0 ** -60 if value < 1 else 1.0
+        levels[l][l % 2, (H >> l) - 1, (W >> l) - 1, 9] = value
+    on_gpu = [t.to(device) for t in levels]
+    got = []
+    assert _labels_of(lambda: got.extend(ms.max_argmax_avg_forward_levels(f1.to(device), on_gpu))) == {"fwd_maxavg_levels_split"}
+    for outs, f in zip(got, levels):
+        _check_max_avg([t.cpu() for t in outs], f1, f)
+
+
+@pytest.mark.parametrize("K", [0, 1, 2, 4])
+def test_pixel_range_in_slabs(device, K):
+    """With argmax and with four channels there is more of out_u's parts than one launch may leave in scratch (96 MiB): the
+    pixel range is cut into two slabs (checked in float64 on the GPU)."""
+    dims = (1, 199, 201, 61, 99, 32)
+    B, H1, W1, H2, W2, C = dims
+    f1, f2 = (torch.randn(B, *hw, C, device=device) for hw in (dims[1:3], dims[3:5]))
+    if K:
+        a_u, a_v = (torch.randn(B, H1, W1, K, n, device=device) for n in (W2, H2))
+        outs = [torch.empty(B, H1, W1, K, n, device=device) for n in (H2, W2)]
+        _call("sepcorr_compression_forward", outs, [f1, f2, a_u, a_v], dims, True, (K,), K)
+    else:
+        outs = _max_avg(f1, f2, dims)
+    for rows in torch.arange(H1, device=device).split(25):
+        vol = _volume(f1[:, rows].double(), f2.double())
+        if K:
+            for k in range(K):
+                for out, w, d in ((outs[0], a_u[:, rows, :, k, None, :], 4), (outs[1], a_v[:, rows, :, k, :, None], 3)):
+                    want = (vol * w).sum(d)
+                    assert ((out[:, rows, :, k] - want).norm() <= 1e-6 * want.norm()).item()
+        else:
+            for out, am, d in ((outs[0], outs[2], 4), (outs[1], outs[3], 3)):
+                assert ((out[:, rows, :, 0] - vol.amax(d)).norm() <= 1e-6 * vol.amax(d).norm()).item()
+                assert ((out[:, rows, :, 1] - vol.mean(d)).norm() <= 1e-6 * vol.mean(d).norm()).item()
+                at = vol.gather(d, am[:, rows, :, 0].long().unsqueeze(d)).squeeze(d)
+                assert (vol.amax(d) - at <= 1e-5 * vol.amax(d)).all()
+
+
+def _shifted(t):
+    """A contiguous copy whose first element lies 4 bytes past a 256-byte boundary."""
+    view = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)[1:].view(t.shape)
+    view.copy_(t)
+    assert view.data_ptr() % 8 == 4
+    return view
+
+
+@pytest.mark.parametrize("dims", [SHAPES[2], SHAPES[4], (2, 45, 48, 46, 64, 40), SHAPES[6]], ids=str)
+def test_tensors_aligned_to_4_bytes(device, dims):
+    B, H1, W1, H2, W2, C = dims
+    f1, f2 = (torch.randn(B, *hw, C, device=device) for hw in (dims[1:3], dims[3:5]))
+    e = lambda *s, **k: torch.empty(*s, device=device, **k)
+    max_avg = [e(B, H1, W1, 2, H2), e(B, H1, W1, 2, W2), e(B, H1, W1, 1, H2, dtype=torch.int32), e(B, H1, W1, 1, W2, dtype=torch.int32)]
+    calls = [("sepcorr_max_argmax_avg_forward", max_avg, [f1, f2], (), 2)]
+    for K in (1, 2, 4):
+        a_u, a_v = (torch.randn(B, H1, W1, K, n, device=device) for n in (W2, H2))
+        calls.append(("sepcorr_compression_forward", [e(B, H1, W1, K, H2), e(B, H1, W1, K, W2)], [f1, f2, a_u, a_v], (K,), K))
+    for name, outs, ins, extra, K in calls:
+        _call(name, outs, ins, dims, True, extra, K)
+        shifted = [_shifted(t) for t in outs]
+        for t in shifted:
+            t.fill_(7)
+        _call(name, shifted, [_shifted(t) for t in ins], dims, True, extra, K)
+        assert all(torch.equal(a, b) for a, b in zip(outs, shifted)), name
+
+
+@pytest.mark.parametrize("dims", [SHAPES[1], SHAPES[5], SHAPES[7], (4, 48, 64, 48, 64, 256)], ids=str)
+def test_workspaces_of_exactly_the_quoted_size(device, dims):
+    """What each query gives is enough and nothing behind it is written."""
+    from separableflowthesis_amd import MemorySaver
+    lib, stream = _lib.load(), torch.cuda.current_stream().cuda_stream
+    B, H1, W1, H2, W2, C = dims
+    f1, f2 = (torch.randn(B, *hw, C, device=device) for hw in (dims[1:3], dims[3:5]))
+    e = lambda *s, **k: torch.empty(*s, device=device, **k)
+    P = lambda t: t.data_ptr()
+
+    def guarded(n, call):
+        ws = torch.full((n + 4096,), 0x5A, dtype=torch.uint8, device=device)
+        _lib.check(call(P(ws), n))
+        assert (ws[n:] == 0x5A).all()
+
+    outs = [e(B, H1, W1, 2, H2), e(B, H1, W1, 2, W2), e(B, H1, W1, 1, H2, dtype=torch.int32), e(B, H1, W1, 1, W2, dtype=torch.int32)]
+    n = lib.sepcorr_forward_workspace_bytes(*dims, 2)
+    assert n > 0
+    guarded(n, lambda ws, n: lib.sepcorr_max_avg_forward(P(f1), P(f2), P(outs[0]), P(outs[1]), *dims, ws, n, stream))
+    guarded(n, lambda ws, n: lib.sepcorr_max_argmax_avg_forward(P(f1), P(f2), *(P(t) for t in outs), *dims, ws, n, stream))
+    for K in (3, 7):
+        a_u, a_v = (torch.randn(B, H1, W1, K, m, device=device) for m in (W2, H2))
+        g_cu, g_cv = torch.randn_like(a_v), torch.randn_like(a_u)
+        c_u, c_v, d_u, d_v, st_u, st_v = (torch.empty_like(t) for t in (a_v, a_u, a_u, a_v, a_u[..., :2], a_v[..., :2]))
+        d_f1, d_f2 = torch.empty_like(f1), torch.empty_like(f2)
+        guarded(lib.sepcorr_forward_workspace_bytes(*dims, K), lambda ws, n: lib.sepcorr_compression_forward_from_logits(
+            P(f1), P(f2), P(a_u), P(a_v), P(c_u), P(c_v), P(st_u), P(st_v), 0, *dims, K, ws, n, stream))
+        for feat in (0, 1):
+            guarded(lib.sepcorr_compression_backward_from_logits_workspace_bytes(*dims, K, feat),
+                    lambda ws, n: lib.sepcorr_compression_backward_from_logits(
+                        P(f1), P(f2), P(a_u), P(a_v), P(st_u), P(st_v), P(c_u), P(c_v), P(g_cu), P(g_cv), P(d_f1) if feat else None,
+                        P(d_f2) if feat else None, P(d_u), P(d_v), *dims, K, ws, n, stream))
+        guarded(lib.sepcorr_backward_workspace_bytes(*dims), lambda ws, n: lib.sepcorr_compression_backward(
+            P(f1), P(f2), P(a_u), P(a_v), P(g_cu), P(g_cv), P(d_f1), P(d_f2), P(d_u), P(d_v), *dims, K, ws, n, stream))
