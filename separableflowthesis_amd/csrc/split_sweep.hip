@@ -5,19 +5,18 @@
 //
 // Contraction.  A pixel's channels are scaled by a power of two that brings the largest of them into [2^14, 2^15) and
 // each is written as h + 2^-11 l, h = fp16(x), l = fp16(2^11 (x - h)): 22 significant bits down to 2^-28 of the pixel's
-// largest channel (both halves of a smaller one are subnormal), 2^-50 of it below.  Pixels with more than a few
-// channels that are smaller still but not zero are marked (below).  A product is h h + 2^-11 (h l + l h): three
-// v_mfma_f32_32x32x16_f16, which accumulate in fp32, in place of eight v_mfma_f32_32x32x2_f32 of twice the length.
+// largest channel (both halves of a smaller one are subnormal), 2^-50 of it below.  A product is h h + 2^-11 (h l + l h):
+// three v_mfma_f32_32x32x16_f16, which accumulate in fp32, in place of eight v_mfma_f32_32x32x2_f32 of twice the length.
 // What is left out (l l) and what the halves do not hold are below the rounding of the fp32 sum, and a sum of 256
-// products is rounded 48 times instead of 128.
+// products is rounded 16 times instead of 128 (the sum of the cross terms, 2^-11 of it, 32 times).
 // Scaling by powers of two is exact and taken back in fp32.  A pixel that has no such form (a channel that is inf or
-// NaN, whose largest channel lies outside [2^-60, 2^61), or max(2, C / 32) channels below 2^-28 of that) is marked, and 32x32 blocks with a marked pixel are
-// multiplied with fp32 MFMAs straight from the inputs.
+// NaN, a largest channel outside [2^-60, 2^61), max(2, C / 32) channels below 2^-28 of it that are not zero) is marked,
+// and 32x32 blocks with a marked pixel are multiplied with fp32 MFMAs straight from the inputs.
 //
 // Work split.  A step = 128 pixels p x 32 columns v of one row u: the workgroup's four waves own 32 pixels each, whose
 // halves stay in registers for the whole sweep (128 registers at C = 256), and share the row block of fmap2 (33 KB at
 // C = 256), which is DMA'd into LDS while the step before is multiplied.  Per step and compute unit that is 33 KB from
-// the L2 and 132 KB from LDS for 1536 cycles of matrix work of each wave.  The steps of all tiles (levels, images,
+// the L2 and 132 KB from LDS (198 where the high halves are read twice) for 1536 cycles of matrix work of each wave.  The steps of all tiles (levels, images,
 // column chunks, pixel tiles, rows) are dealt out evenly.  Results of the other chunks and of other pieces of a tile
 // are left in scratch and put together by split_finish_kernel in a fixed order.
 #include "split_sweep.h"
@@ -377,17 +376,18 @@ __global__ void __launch_bounds__(256) split_finish_kernel(const SplitArgs a) {
 }
 #endif
 
-// The max/avg modes and one weight channel fit 256 registers, and so do two channels where a pixel's halves take few (C <= 64):
-// two workgroups per compute unit, one wave's reductions run beside the other's matrix work.  More channels take the whole
-// register file, and a wave reduces one row while it multiplies the next.  Both ways measured (two workgroups / one): C=256
-// max/avg, B=2, 55x128 0.149 / 0.166 ms, two channels over the four levels of 47x156 0.225 / 0.212; C=64 two channels B=4, 80x120
-// 0.270 / 0.342, four 0.895 / 0.521; C=100 two channels B=2, 47x61 0.054 / 0.046.
+// The max/avg modes and one weight channel fit 256 registers, and so do two channels where a pixel's halves take few
+// (C <= 64): two workgroups per compute unit, one wave's reductions run beside the other's matrix work.  More channels
+// take the whole register file, and a wave reduces one row while it multiplies the next.  Both ways measured (two
+// workgroups / one): C=256 max/avg, B=2, 55x128 0.149 / 0.166 ms, two channels over the four levels of 47x156 0.225 / 0.212;
+// C=64 two channels B=4, 80x120 0.270 / 0.342, four 0.895 / 0.521; C=100 two channels B=2, 47x61 0.054 / 0.046.
 __host__ __device__ constexpr bool pipelined(int mode, int kc, int nk) { return mode == SPLIT_WEIGHTED && kc > 1 && !(kc == 2 && nk == 4); }
 
 // NK: channel steps of 16 (C <= 16 NK, the rest zeros).  Measured at B=2, 55x128, C=256: max/avg/argmax 0.454 ms with the
-// fp32 sweep, 0.149 ms here (+ 0.013 split_prepare_kernel, 0.032 split_finish_kernel); four weighted sums 0.474 and
-// 0.192 ms (+ 0.013 and 0.034).  The matrix instructions alone take 0.061 ms at 2.4 GHz; what is left is the vector work
-// of the reductions, the reads of the row block from LDS and the beginning and end of every step.
+// fp32 sweep, 0.158 ms here (+ 0.014 split_prepare_kernel, 0.033 split_finish_kernel); four weighted sums 0.474 and
+// 0.203 ms (+ 0.014 and 0.034).  The matrix instructions alone take 0.061 ms at 2.4 GHz; the clock falls to 1.5 to 1.7 GHz
+// under them (matrix units 53 and 34 % busy), the rest is the vector work of the reductions, the reads of the row block
+// from LDS and the beginning and end of every step.
 template <int MODE, int KC, int NK>
 __global__ void __launch_bounds__(256, pipelined(MODE, KC, NK) ? 1 : 2) split_sweep_kernel(const SplitArgs a) {
     constexpr bool WT = MODE == SPLIT_WEIGHTED;
@@ -633,9 +633,9 @@ __global__ void __launch_bounds__(256, pipelined(MODE, KC, NK) ? 1 : 2) split_sw
         // The products of a row block; `beside(s)` is what the vector units do beside the matrix work of channel step s.
         // Operands are read two channel steps before they are used.  The order is fixed here: left to itself the
         // compiler either reads everything at once (and spills) or waits for every read, and puts the vector work last.
-        // Row `next` is requested into row block nbuf a KB at a time between the matrix instructions (all requests at once hold the wave up
-        // for 700 cycles; behind a piece's last row they fetch what follows it in the scratch, which is not used).  The factors that scale
-        // row u back are in `fac` at the end and the block's mark in `mark`.
+        // Row `next` is requested into row block nbuf a KB at a time between the matrix instructions (all requests at once
+        // hold the wave up for 700 cycles; behind a piece's last row they fetch what follows it in the scratch, which is
+        // not used).  The factors that scale row u back are in `fac` at the end and the block's mark in `mark`.
         v4f fac[4];
         int mark = 0;
         auto multiply = [&](int next, int buf, int nbuf, auto beside) {
