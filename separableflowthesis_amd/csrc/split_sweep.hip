@@ -16,9 +16,9 @@
 // Work split.  A step = 128 pixels p x 32 columns v of one row u: the workgroup's four waves own 32 pixels each, whose
 // halves stay in registers for the whole sweep (128 registers at C = 256), and share the row block of fmap2 (33 KB at
 // C = 256), which is DMA'd into LDS while the step before is multiplied.  Per step and compute unit that is 33 KB from
-// the L2 and 132 KB from LDS (198 where the high halves are read twice) for 1536 cycles of matrix work of each wave.  The steps of all tiles (levels, images,
-// column chunks, pixel tiles, rows) are dealt out evenly.  Results of the other chunks and of other pieces of a tile
-// are left in scratch and put together by split_finish_kernel in a fixed order.
+// the L2 and 132 KB from LDS (198 where the high halves are read twice) for 1536 cycles of matrix work of each wave.
+// The steps of all tiles (levels, images, column chunks, pixel tiles, rows) are dealt out evenly.  Results of the other
+// chunks and of other pieces of a tile are left in scratch and put together by split_finish_kernel in a fixed order.
 #include "split_sweep.h"
 
 #include <math.h>
@@ -81,7 +81,8 @@ __device__ __forceinline__ bool pixel_scale(unsigned m, float &fwd, float &back)
     back = __uint_as_float((e - 14u) << 23);
     return true;
 }
-constexpr float LOW_UNIT = 1.f / 2048.f;   // low halves are held times 2^11: they are as far from the subnormals as high ones
+// low halves are held times 2^11: they are as far from the subnormals as high ones
+constexpr float LOW_UNIT = 1.f / 2048.f;
 // (a marked pixel has factor 0 and may hold inf: its halves are zeros, not NaN)
 __device__ __forceinline__ void split8(const float (&x)[8], float f, v8h &h, v8h &l) {
 #pragma unroll
@@ -111,8 +112,9 @@ __device__ __forceinline__ void load8(__amdgpu_buffer_rsrc_t r, unsigned off, in
 __device__ __forceinline__ unsigned magnitude(float x) { return __float_as_uint(x) & 0x7fffffffu; }
 
 // A block with a marked pixel: fp32 products straight from the inputs, this lane's pixel of image 1 at byte o1 of n1, of
-// fmap2 at byte o2 of n2 (OOB: none), the first `cols` columns of this lane's half.  16 channels a turn; a lane's eight are contiguous, and the next turn's are on their
-// way.  A function of its own: its registers would otherwise be taken from the sweep's.
+// fmap2 at byte o2 of n2 (OOB: none), the first `cols` columns of this lane's half.  16 channels a turn; a lane's eight are
+// contiguous, and the next turn's are on their way.  A function of its own: its registers would otherwise be taken from
+// the sweep's.
 // B=2, 55x128, max/average: 0.18 ms without a marked pixel, 0.44 with one in image 1, 0.86 with all of them marked; with one
 // channel a turn 0.88 and 2.78 ms, the fp32 sweep 0.44.
 __device__ __attribute__((noinline)) v16f products_fp32(const float *f1, unsigned n1, unsigned o1, const float *f2, unsigned n2, unsigned o2,
