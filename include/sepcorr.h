@@ -71,8 +71,10 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap);
  * Arithmetic of the contractions of the forward sweeps (max/avg, max/argmax/avg, compression forward and the
  * attention-gradient pass of the compression backward) and of d_f1; no counterpart in the reference.
  *   SEPCORR_CONTRACT_SPLIT   forward sweeps of 32 <= C <= 256 channels and at least 1e9 of B H1 W1 H2 W2 (C + 64) with every
- *                            fp32 operand as two 16-bit halves (the note on scratch memory above), fp32 MFMA
- *                            elsewhere (the initial choice).
+ *                            fp32 operand as two 16-bit halves (the note on scratch memory above), and so the
+ *                            feature gradients of the compression from 5e8 on, of the combined backward from
+ *                            2.5e8 on, where the workspace is what the query gives; fp32 MFMA elsewhere (the
+ *                            initial choice).
  *   SEPCORR_CONTRACT_FP32    fp32 MFMA throughout.
  *   SEPCORR_CONTRACT_BF16X3  every fp32 operand is written exactly as the sum of three bf16 numbers and the
  *                            product taken as the six largest of the nine plane products, with bf16 MFMA
@@ -148,7 +150,9 @@ int sepcorr_compression_forward(const float *f1, const float *f2, const float *a
                                 int B, int H1, int W1, int H2, int W2, int C, int K,
                                 void *workspace, size_t workspace_bytes, void *stream);
 
-/* Scratch bytes needed by any of the three backward entry points for these sizes (0 is possible). */
+/* Scratch bytes for any of the three backward entry points at these sizes (0 is possible).  (Part of it is for the feature
+ * gradients' contractions with operands in two 16-bit halves; a call that gets less, but as much as its fp32 kernels need,
+ * runs those.) */
 size_t sepcorr_backward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C);
 
 /*

@@ -38,6 +38,7 @@
 
 #include "sepcorr.h"
 #include "sepcorr_internal.h"
+#include "split_grad.h"
 #include "split_sweep.h"
 
 // This file is compiled once per part (see the Makefile) so that its many kernel instantiations build in parallel:
@@ -3665,10 +3666,12 @@ Df1Shape df1_shape(const Dims &d) {
 // after the other, and the regions of different kernels share the same memory; so too where the sweep runs on 16-bit halves,
 // which always takes scratch.  (Whole tiles, d_f1 and d_f2 beside each other / after each other: compression backward B=4,
 // 64x64, C=256 783 / 746 us, C=128 512 / 474; fused backward 759 / 702 and 536 / 450; at no measured size worse.)
+// total: what a call needs.  full: with what the contractions of split_grad.hip take, from the same memory.
 struct BwdWs {
     bool aliased;
     size_t off_uwt, off_df1sk, fwd_bytes, own_total, total;   // own_total: without the weight-gradient sweep
     size_t off_vtable;                                        // (B,W2,C) table of the combined d_f2 (Df2Plan::noavgv)
+    size_t full;
 };
 BwdWs bwd_ws(const Dims &d) {
     BwdWs w;
@@ -3691,6 +3694,7 @@ BwdWs bwd_ws(const Dims &d) {
     }
     w.off_vtable = w.total;
     if (df2_plan(d, true).noavgv) w.total += ((size_t)d.B * d.W2 * d.C * sizeof(float) + 255) & ~(size_t)255;
+    w.full = std::max(w.total, split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C));
     return w;
 }
 
@@ -4019,7 +4023,7 @@ int static_scratch(void **out) {
 #endif
 
 int check_workspace(const Dims &d, void *ws, size_t ws_bytes) {
-    const size_t need = sepcorr_backward_workspace_bytes(d.B, d.H1, d.W1, d.H2, d.W2, d.C);
+    const size_t need = bwd_ws(d).total;   // (the rest of what sepcorr_backward_workspace_bytes() gives is for split_gradients())
     if (need > 0 && (ws == nullptr || ws_bytes < need))
         return fail(SEPCORR_EWORKSPACE, "sepcorr: backward needs %zu bytes of workspace, got %zu", need, ws ? ws_bytes : (size_t)0);
     if (need > 0 && (reinterpret_cast<uintptr_t>(ws) & 255))
@@ -4085,6 +4089,61 @@ int maxavg_backward(const Dims &d, bool gather, const float *f1, const float *f2
     a.d1 = d_f1; a.d2 = d_f2;
     a.B = d.B; a.N1 = d.H1 * d.W1; a.H2 = d.H2; a.W2 = d.W2; a.C = d.C; a.KT = 1;
     return launch_bwd<GMODE_MAXAVG, 1>(a, d, ws, s1, s);
+}
+
+// Whether the feature gradients of a call with this workspace come from the contractions of split_grad.hip.
+bool split_gradients(const Dims &d, const BwdWs &lay, bool both, size_t ws_bytes) {
+    const double size = (double)d.B * d.H1 * d.W1 * d.H2 * d.W2 * (d.C + 64);
+    return split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C) > 0 && size >= (both ? SPLIT_GRAD_LINE : SPLIT_GRAD_LINE_ALONE) &&
+           ws_bytes >= lay.full && g_contraction.load(std::memory_order_relaxed) == SEPCORR_CONTRACT_SPLIT;
+}
+
+// d_f1 and d_f2 of the compression (`both`: with the max/average terms) of K weight channels, the tensors as `a` names
+// them: d_f1 on stream s1, d_f2 on s (split: one stream).
+int feature_gradients(const Dims &d, BwdArgs a, bool both, int K, bool split, void *ws, size_t ws_bytes, hipStream_t s1, hipStream_t s) {
+    a.KT = K;
+    for (int k0 = 0; split && k0 < K; k0 += KCH) {
+        GradArgs g;
+        memset(&g, 0, sizeof(g));
+        g.f1 = a.f1; g.f2 = a.f2; g.a_u = a.a_u; g.a_v = a.a_v; g.g_cu = a.g_cu; g.g_cv = a.g_cv;
+        g.am_u = a.am_u; g.am_v = a.am_v; g.g_u = a.g_u; g.g_v = a.g_v;
+        g.d1 = a.d1; g.d2 = a.d2;
+        g.B = d.B; g.N1 = a.N1; g.H2 = d.H2; g.W2 = d.W2; g.C = d.C; g.KT = K; g.k0 = k0;
+        g.add1 = a.add_d1 || k0 > 0;
+        g.add2 = k0 > 0;
+        const int rc = split_grad(both && k0 == 0, std::min(K - k0, KCH), g, ws, ws_bytes, s);
+        if (rc == 1 && k0 == 0) split = false;   // (weights at odd addresses take more scratch)
+        else if (rc) return rc < 0 ? rc : fail(SEPCORR_EWORKSPACE, "sepcorr: feature gradients: scratch does not suffice");
+    }
+    if (split) return SEPCORR_OK;
+    int rc = SEPCORR_OK;
+    const int kch = d.W2 > 128 ? 2 : KCH;   // wide workgroups have half the registers per lane
+    const int kc0 = std::min(K, kch);
+    // The first chunk of weight channels carries the max/avg terms of G along (built for 2 and 4 channels);
+    // otherwise they follow as one more accumulating launch.
+    const bool first_carries = both && (kc0 == 2 || kc0 == 4);
+    // channel chunks accumulate into d_f1 / d_f2: each output keeps its own stream, so chunks stay ordered
+    for (int k0 = 0; k0 < K && rc == SEPCORR_OK; k0 += kch) {
+        a.k0 = k0;
+        a.accumulate = k0 > 0;
+        const int kc = std::min(K - k0, kch);
+        if (k0 == 0 && first_carries) {
+            rc = kc == 2 ? launch_bwd<GMODE_BOTH, 2>(a, d, ws, s1, s) : launch_bwd<GMODE_BOTH, 4>(a, d, ws, s1, s);
+            continue;
+        }
+        switch (kc) {
+            case 1: rc = launch_bwd<GMODE_COMP, 1>(a, d, ws, s1, s); break;
+            case 2: rc = launch_bwd<GMODE_COMP, 2>(a, d, ws, s1, s); break;
+            case 3: rc = launch_bwd<GMODE_COMP, 3>(a, d, ws, s1, s); break;
+            default: rc = launch_bwd<GMODE_COMP, 4>(a, d, ws, s1, s); break;
+        }
+    }
+    if (both && !first_carries && rc == SEPCORR_OK) {
+        a.k0 = 0; a.KT = 1;
+        a.accumulate = 1;
+        rc = launch_bwd<GMODE_MAXAVG, 1>(a, d, ws, s1, s);
+    }
+    return rc;
 }
 
 #define REQUIRE_PTR(p) \
@@ -4210,7 +4269,7 @@ int sepcorr_compression_forward(const float *f1, const float *f2, const float *a
 size_t sepcorr_backward_workspace_bytes(int B, int H1, int W1, int H2, int W2, int C) {
     if (B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1) return 0;
     const Dims d = {B, H1, W1, H2, W2, C};
-    return bwd_ws(d).total;
+    return bwd_ws(d).full;
 }
 
 int sepcorr_max_argmax_avg_backward(const float *f1, const float *f2, const int32_t *argmax_u, const int32_t *argmax_v,
@@ -4275,7 +4334,8 @@ int sepcorr_compression_backward(const float *f1, const float *f2, const float *
     }
     if (int rc = check_workspace(d, workspace, workspace_bytes)) return rc;
     const BwdWs lay = bwd_ws(d);
-    ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased);
+    const bool split = split_gradients(d, lay, false, workspace_bytes);
+    ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased && !split);
     // d_a_v[k,u] = sum_v S g_cv[k,v];  d_a_u[k,v] = sum_u S g_cu[k,u]: the forward's weighted sums
     int rc = weighted_forward(d, f1, f2, g_cv, g_cu, d_a_v, d_a_u, K, lay.fwd_bytes ? workspace : nullptr, lay.fwd_bytes, fj.user);
     BwdArgs a;
@@ -4283,20 +4343,8 @@ int sepcorr_compression_backward(const float *f1, const float *f2, const float *
     a.xcd_order = xcd_order_enabled();
     a.f1 = f1; a.f2 = f2; a.a_u = a_u; a.a_v = a_v; a.g_cu = g_cu; a.g_cv = g_cv;
     a.d1 = d_f1; a.d2 = d_f2;
-    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C; a.KT = K;
-    const int kch = W2 > 128 ? 2 : KCH;  // wide workgroups have half the registers per lane
-    // channel chunks accumulate into d_f1 / d_f2: each output keeps its own stream, so chunks stay ordered
-    for (int k0 = 0; k0 < K && rc == SEPCORR_OK; k0 += kch) {
-        a.k0 = k0;
-        a.accumulate = k0 > 0;
-        const int kc = K - k0 < kch ? K - k0 : kch;
-        switch (kc) {
-            case 1: rc = launch_bwd<GMODE_COMP, 1>(a, d, workspace, fj.sa, fj.sb); break;
-            case 2: rc = launch_bwd<GMODE_COMP, 2>(a, d, workspace, fj.sa, fj.sb); break;
-            case 3: rc = launch_bwd<GMODE_COMP, 3>(a, d, workspace, fj.sa, fj.sb); break;
-            default: rc = launch_bwd<GMODE_COMP, 4>(a, d, workspace, fj.sa, fj.sb); break;
-        }
-    }
+    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
+    if (rc == SEPCORR_OK) rc = feature_gradients(d, a, false, K, split, workspace, workspace_bytes, fj.sa, fj.sb);
     const int rj = fj.join();
     return rc ? rc : rj;
 }
@@ -4348,7 +4396,7 @@ size_t sepcorr_compression_backward_from_logits_workspace_bytes(int B, int H1, i
     const size_t dots = 2 * ((rows * sizeof(float) + 255) & ~(size_t)255);
     if (!with_features) return ((sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255) + dots;
     const size_t a_bytes = ((rows * W2 * sizeof(float) + 255) & ~(size_t)255) + ((rows * H2 * sizeof(float) + 255) & ~(size_t)255);
-    return bwd_ws(d).total + dots + a_bytes;
+    return bwd_ws(d).full + dots + a_bytes;
 }
 
 int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, const float *logits_u, const float *logits_v,
@@ -4363,7 +4411,9 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     if (int rc = check_dims(d, K)) return rc;
     if ((d_f1 == nullptr) != (d_f2 == nullptr))
         return fail(SEPCORR_EINVAL, "sepcorr: d_f1 and d_f2 must be given together or both be NULL");
-    const size_t need = sepcorr_compression_backward_from_logits_workspace_bytes(B, H1, W1, H2, W2, C, K, d_f1 != nullptr);
+    const BwdWs lay = bwd_ws(d);
+    const size_t best = sepcorr_compression_backward_from_logits_workspace_bytes(B, H1, W1, H2, W2, C, K, d_f1 != nullptr);
+    const size_t need = best - (d_f1 ? lay.full - lay.total : 0);   // (the rest is for split_gradients())
     if (workspace == nullptr || workspace_bytes < need)
         return fail(SEPCORR_EWORKSPACE, "sepcorr: backward from logits needs %zu bytes of workspace, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
@@ -4371,7 +4421,7 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     hipStream_t s = static_cast<hipStream_t>(stream);
     const size_t rows = (size_t)B * H1 * W1 * K;
     const size_t dot_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
-    const size_t own_bytes = d_f1 ? bwd_ws(d).total : (sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255;
+    const size_t own_bytes = d_f1 ? (workspace_bytes >= best ? lay.full : lay.total) : (sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255;
     char *base = static_cast<char *>(workspace);
     float *dot_u = reinterpret_cast<float *>(base + own_bytes);               // sum_u g_cu * comp_u = sum_v a_u * d_a_u
     float *dot_v = reinterpret_cast<float *>(base + own_bytes + dot_bytes);   // sum_v g_cv * comp_v = sum_u a_v * d_a_v
@@ -4402,26 +4452,15 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
         hipLaunchKernelGGL(softmax_apply_kernel, grid, block, 0, s, logits_v, stats_v, a_v, (long)rows, H2, (int)(rows_vec4(logits_v, H2) && rows_vec4(a_v, H2)));
         if (int rc2 = check_launch("softmax from statistics")) return rc2;
     }
-    const BwdWs lay = bwd_ws(d);
-    ForkJoin fj(s, !lay.aliased);
+    const bool split = split_gradients(d, lay, false, own_bytes);
+    ForkJoin fj(s, !lay.aliased && !split);
     BwdArgs a;
     memset(&a, 0, sizeof(a));
     a.xcd_order = xcd_order_enabled();
     a.f1 = f1; a.f2 = f2; a.a_u = a_u; a.a_v = a_v; a.g_cu = g_cu; a.g_cv = g_cv;
     a.d1 = d_f1; a.d2 = d_f2;
-    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C; a.KT = K;
-    const int kch = W2 > 128 ? 2 : KCH;
-    for (int k0 = 0; k0 < K && rc == SEPCORR_OK; k0 += kch) {
-        a.k0 = k0;
-        a.accumulate = k0 > 0;
-        const int kc = K - k0 < kch ? K - k0 : kch;
-        switch (kc) {
-            case 1: rc = launch_bwd<GMODE_COMP, 1>(a, d, workspace, fj.sa, fj.sb); break;
-            case 2: rc = launch_bwd<GMODE_COMP, 2>(a, d, workspace, fj.sa, fj.sb); break;
-            case 3: rc = launch_bwd<GMODE_COMP, 3>(a, d, workspace, fj.sa, fj.sb); break;
-            default: rc = launch_bwd<GMODE_COMP, 4>(a, d, workspace, fj.sa, fj.sb); break;
-        }
-    }
+    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
+    rc = feature_gradients(d, a, false, K, split, workspace, own_bytes, fj.sa, fj.sb);
     const int rj = fj.join();
     return rc ? rc : rj;
 }
@@ -4632,35 +4671,11 @@ static int fused_backward(const float *f1, const float *f2, const int32_t *argma
     a.a_u = a_u; a.a_v = a_v; a.g_cu = g_cu; a.g_cv = g_cv;
     a.d1 = d_f1; a.d2 = d_f2;
     a.add_d1 = add_d_f1 != 0;
-    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C; a.KT = K;
-    ForkJoin fj(static_cast<hipStream_t>(stream), !bwd_ws(d).aliased);
-    const int kch = W2 > 128 ? 2 : KCH;
-    const int kc0 = K < kch ? K : kch;
-    // The first chunk of weight channels carries the max/avg terms of G along (built for 2 and 4 channels);
-    // otherwise they follow as one more accumulating launch.
-    const bool first_carries = kc0 == 2 || kc0 == 4;
-    int rc = SEPCORR_OK;
-    for (int k0 = 0; k0 < K && rc == SEPCORR_OK; k0 += kch) {
-        a.k0 = k0;
-        a.accumulate = k0 > 0;
-        const int kc = K - k0 < kch ? K - k0 : kch;
-        if (k0 == 0 && first_carries) {
-            rc = kc == 2 ? launch_bwd<GMODE_BOTH, 2>(a, d, workspace, fj.sa, fj.user)
-                         : launch_bwd<GMODE_BOTH, 4>(a, d, workspace, fj.sa, fj.user);
-            continue;
-        }
-        switch (kc) {
-            case 1: rc = launch_bwd<GMODE_COMP, 1>(a, d, workspace, fj.sa, fj.user); break;
-            case 2: rc = launch_bwd<GMODE_COMP, 2>(a, d, workspace, fj.sa, fj.user); break;
-            case 3: rc = launch_bwd<GMODE_COMP, 3>(a, d, workspace, fj.sa, fj.user); break;
-            default: rc = launch_bwd<GMODE_COMP, 4>(a, d, workspace, fj.sa, fj.user); break;
-        }
-    }
-    if (!first_carries && rc == SEPCORR_OK) {
-        a.k0 = 0; a.KT = 1;
-        a.accumulate = 1;
-        rc = launch_bwd<GMODE_MAXAVG, 1>(a, d, workspace, fj.sa, fj.user);
-    }
+    a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
+    const BwdWs lay = bwd_ws(d);
+    const bool split = split_gradients(d, lay, true, workspace_bytes);
+    ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased && !split);
+    const int rc = feature_gradients(d, a, true, K, split, workspace, workspace_bytes, fj.sa, fj.user);
     const int rj = fj.join();
     return rc ? rc : rj;
 }

@@ -1,0 +1,53 @@
+// Feature gradients (d_f1, d_f2) of the compression and of the combined backward with every fp32 operand split into two
+// 16-bit halves (split_grad.hip): what sepcorr.hip hands over.  Internal to libsepcorr.
+#ifndef SEPCORR_SPLIT_GRAD_H
+#define SEPCORR_SPLIT_GRAD_H
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+struct VField {
+    const float *src;      // a tensor of `rows` rows of W2 per pixel of image 1
+    int rows, row;         // the field's among them
+};
+struct GradArgs {
+    const float *f1, *f2;
+    const float *a_u, *a_v, *g_cu, *g_cv;     // (B,N1,KT,W2), (B,N1,KT,H2), (B,N1,KT,H2), (B,N1,KT,W2)
+    const int *am_u, *am_v;                   // with the max/average terms: (B,N1,H2), (B,N1,W2)
+    const float *g_u, *g_v;                   //                             (B,N1,2,H2), (B,N1,2,W2)
+    float *d1, *d2;                           // (B,N1,C), (B,H2 W2,C)
+    int B, N1, H2, W2, C;
+    int KT, k0;                               // weight channels in all, first one of this launch
+    int add1, add2;                           // add to d1 / d2 instead of overwriting
+    // filled by split_grad()
+    int ncb, nvc;                             // channel blocks of 32 (2, 4, 8), column chunks of 32
+    int H2p, N1p;                             // rows padded to 8, pixels padded to 128
+    int npx;                                  // pixel tiles of 16 that hold pixels
+    int direct;                               // the v-indexed weights are read where they are, not from pv
+    float *pv;                                // [B][nvc][N1p / 16][field][8 groups of columns][16 pixels][4 columns]
+    float *pu;                                // [B][H2p][N1p][u-indexed fields]
+    float *back;                              // [B][N1p] what takes a pixel's factor back, 0 where G is zero
+    float *block_back, *top_back;             // the largest of 16 pixels, negative if one has no factor; of an image
+    unsigned *pmax;                           // [2][B][slab][256] largest |f1|, |f2| of a channel
+    float *cback;                             // [2][B][256] what takes a channel's factor back
+    unsigned *count;                          // small values of f1, of f2; whether anything else is unsuitable
+    char *f1h, *f2h;                          // halves of f1 [B][npx], of f2 [B][nvc][H2]
+    VField vfield[11];                        // the v-indexed weights
+    GradArgs *self;                           // these arguments, on the device
+    float *slots;
+    int G1, G2;                               // workgroups of the two contractions
+};
+
+// Below this many pairs of pixels times (channels + 64) split_grad() takes nothing, and below the other one it does not pay
+// for the compression alone.  Five or six launches, three of them over the operands, against two to five: time over that of
+// the fp32 kernels in 70 shapes of 1e8 to 6e9, 32 <= C <= 256, 1 to 4 weight channels: with the max/average terms 1.0 to 2.1
+// below 1.4e8, 0.38 to 1.01 from 2.5e8 on (the fp32 kernels make two passes for one or three weight channels); without
+// them 0.76 to 1.34 up to 5e8, 0.65 to 1.09 up to 1e9; above 1e9 0.28 to 0.80, on average 0.49.
+#define SPLIT_GRAD_LINE 2.5e8
+#define SPLIT_GRAD_LINE_ALONE 5e8
+// Scratch split_grad() wants for these sizes, whatever the number of channels, 0 where it does not take them.
+size_t split_grad_bytes(int B, int N1, int H2, int W2, int C);
+// Runs both contractions, with the max/average terms if `both`, when the sizes suit it and ws_bytes suffice; returns 1 without
+// launching anything otherwise, a negative SEPCORR_ code on error.  kc: 1 to 4 weight channels.
+int split_grad(int both, int kc, GradArgs a, void *ws, size_t ws_bytes, hipStream_t s);
+#endif
