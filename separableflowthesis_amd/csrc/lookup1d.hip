@@ -8,7 +8,7 @@
 // For its first volume the reference clamps the sampling positions to [-1, 1] before sampling
 // (core/corr.py:593); `clamp_unit` reproduces that.
 //
-// The pyramid is not stored: entry m of level l is the mean of level-0 entries [m*2^l, (m+1)*2^l).  One thread per (b, d, i, j): neighbouring threads are
+// The pyramid is not stored: entry m of level l is the mean of level-0 entries [m*2^l, (m+1)*2^l).  Neighbouring threads are
 // neighbouring image-1 pixels, whose reads of corr[b,d,w,i,j] sit side by side whenever their w agree (smooth flow).
 // HBM/L2-bound gather, no matrix work.  The backward pass is its exact adjoint in gather form: one thread per entry
 // of d_corr collects what the samples around it passed on, so there are no atomics and the order of the sums is fixed.
@@ -47,7 +47,48 @@ __device__ __forceinline__ void sample_pos(float x, int k, int r, bool clamp_uni
     if (!(f >= 0.f && f <= 1.f)) f = pos - pos;     // NaN for infinite positions, as in the sampler
 }
 
-// grid.x covers (b, d, pixel), grid.y = pyramid level
+// entry m of level SH, its loads in flight together
+template <int SH>
+__device__ __forceinline__ float pooled(const float *col, size_t plane, int m) {
+    float x[1 << SH], s = 0.f;
+#pragma unroll
+    for (int t = 0; t < (1 << SH); ++t) x[t] = col[(size_t)((m << SH) + t) * plane];
+#pragma unroll
+    for (int t = 0; t < (1 << SH); ++t) s += x[t];
+    return s / (float)(1 << SH);
+}
+
+// grid.x covers (b, d, pixel), grid.y = pyramid level and sample.  Bound by latency: a thread reads the 2^l entries under
+// both neighbours of one sample, all of them at once.  (55x128, 4 levels, radius 4, one channel: 7.4 us, which is what a launch
+// takes, against 13.5 with a thread for all samples of a level; the two forms give the same bits.)
+__global__ void __launch_bounds__(256) lookup1d_forward_samples_kernel(const L1dArgs a) {
+    const size_t plane = (size_t)a.H1 * a.W1;
+    const size_t total = (size_t)a.B * a.dim * plane;
+    const size_t e = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= total) return;
+    const int n = 2 * a.r + 1, l = blockIdx.y / n, k = blockIdx.y - l * n, Ll = a.L >> l;
+    const size_t pix = e % plane;
+    const int d = (int)((e / plane) % a.dim), b = (int)(e / (plane * a.dim));
+    const float xl = a.coords[((size_t)b * 2 + a.coord_channel) * plane + pix] / (float)(1 << l);
+    const float *col = a.corr + ((size_t)b * a.dim + d) * a.L * plane + pix;
+    int p0;
+    float f, v0, v1;
+    sample_pos(xl, k, a.r, a.clamp_unit != 0, p0, f);
+    const int m0 = min(max(p0, 0), Ll - 1), m1 = min(max(p0 + 1, 0), Ll - 1);   // (read in any case, dropped where there is none)
+    switch (l) {
+        case 0: v0 = pooled<0>(col, plane, m0); v1 = pooled<0>(col, plane, m1); break;
+        case 1: v0 = pooled<1>(col, plane, m0); v1 = pooled<1>(col, plane, m1); break;
+        case 2: v0 = pooled<2>(col, plane, m0); v1 = pooled<2>(col, plane, m1); break;
+        case 3: v0 = pooled<3>(col, plane, m0); v1 = pooled<3>(col, plane, m1); break;
+        default: v0 = pooled_any(col, plane, m0, l); v1 = pooled_any(col, plane, m1, l); break;
+    }
+    if (p0 != m0) v0 = 0.f;
+    if (p0 + 1 != m1) v1 = 0.f;
+    a.out[((size_t)b * a.levels * a.dim + (size_t)l * a.dim + d) * n * plane + (size_t)k * plane + pix] = fmaf(f, v1, (1.f - f) * v0);
+}
+
+// One thread for all samples of a level, each entry formed once: half the reads, one entry after the other.  grid.x covers
+// (b, d, pixel), grid.y = pyramid level
 __global__ void __launch_bounds__(256) lookup1d_forward_kernel(const L1dArgs a) {
     const size_t plane = (size_t)a.H1 * a.W1;
     const size_t total = (size_t)a.B * a.dim * plane;
@@ -180,6 +221,11 @@ int run(bool backward, const float *corr, const float *coords, const float *gout
         else
             hipLaunchKernelGGL(lookup1d_backward_columns_kernel, dim3((unsigned)((total + 255) / 256)), block, 0, s, a);
     }
+    // by samples up to where the columns alone keep the chip busy; measured, 4 levels, radius 4, by columns / by samples:
+    // 55x128 1 channel 13.5 / 7.4 us, B=2 with 8 channels (112 640 columns) 35.9 / 35.5, 24 channels (337 920) 200 / 191, B=12
+    // with 8 channels (675 840) 455 / 505
+    else if (total < (size_t)384 * 1024 && levels * n <= 65535)
+        hipLaunchKernelGGL(lookup1d_forward_samples_kernel, dim3((unsigned)((total + 255) / 256), levels * n), block, 0, s, a);
     else hipLaunchKernelGGL(lookup1d_forward_kernel, dim3((unsigned)((total + 255) / 256), levels), block, 0, s, a);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) {

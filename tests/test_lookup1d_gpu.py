@@ -54,6 +54,21 @@ def test_without_the_clamp_both_volumes_follow_the_plain_definition(device):
     assert_close(q1, ref, "out1 without clamp")
 
 
+@pytest.mark.parametrize("shape,levels,radius", [((1, 2, 70, 5, 77), 6, 16),      # levels of 16 and 32 entries, windows wider than the volume
+                                                 ((2, 1, 9, 3, 85), 4, 4),        # one entry at the last level
+                                                 ((1, 63, 8, 78, 80), 3, 2),      # 393 120 columns: a thread per sample
+                                                 ((1, 64, 8, 77, 80), 3, 2)])     # 394 240: a thread per column
+@pytest.mark.parametrize("clamp", [False, True])
+def test_forward_forms_against_the_definition(device, shape, levels, radius, clamp):
+    from separableflowthesis_amd import MemorySaver
+    B, dim, L, H, W = shape
+    g = torch.Generator().manual_seed(L)
+    corr = torch.randn(shape, generator=g)
+    coords = (torch.randn(B, 2, H, W, generator=g) * L).contiguous()
+    got = MemorySaver.lookup1d_forward(corr.to(device), coords.to(device), 1, clamp, levels, radius)
+    assert_close(got, O.lookup1d_direct(corr.double(), coords[:, 1].double(), levels, radius, clamp_unit=clamp), "out")
+
+
 def test_consumes_the_volumes_of_separate_and_checks_arguments(device):
     from separableflowthesis_amd import AlternateCorrBlockSepflow, CorrBlock1D, MemorySaver
     g = torch.Generator().manual_seed(3)
