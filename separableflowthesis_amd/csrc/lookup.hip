@@ -314,7 +314,8 @@ __global__ void __launch_bounds__(256) lookup_forward_group_kernel(const LookupA
 
 constexpr int TQX = 8, TQY = 4;                     // fmap2 positions per d_f2 wave: the 32 rows of one MFMA tile
 constexpr int NCH = 128;                            // channels per d_f2 wave
-constexpr int NPR = 2;                              // pixel pairs fetched before their MFMAs are issued
+constexpr int NPR = 2;                              // pixel pairs of a step
+constexpr int CHUNK = 512;                          // pixels that a d_f2 wave looks through at a time
 static_assert(TQX * TQY == 32, "one tile position per MFMA row");
 
 struct LookupBwdArgs {
@@ -497,15 +498,22 @@ __global__ void __launch_bounds__(256) lookup_df1_group_kernel(const LookupBwdAr
 
 // One wave = (tile of TQY x TQX positions of one level, slice of the pixel range, block of NCH channels).  For the
 // tile, d_f2[pos, ch] = sum over pixels of W[pos, pixel] * f1[pixel, ch] is a small matrix product whose inner index
-// runs over the pixels whose window touches the tile.  The wave scans its pixels 64 at a time (origins stay in the
-// lanes' registers), takes the touching ones in ascending order, two per v_mfma_f32_32x32x2_f32: operand A = the two
-// pixels' window entries at the tile's positions (zero outside the window), operand B = their f1 channels, fetched as
-// contiguous runs.  Four pixels are fetched before their MFMAs are issued (measured: 2 pixels 0.147, 4 0.137, 8 0.142 ms).
-// No LDS, no barrier, no atomics.
+// runs over the pixels whose window touches the tile.  The wave lists those of CHUNK pixels at a time in LDS, in ascending
+// order (the origins of the next ones on their way), and takes them from there two per v_mfma_f32_32x32x2_f32: operand
+// A = the two pixels' window entries at the tile's positions (zero outside the window), operand B = their f1 channels.
+// What bounds it is how long a window entry is on its way (W, 22 MB at B=2, 55x128, is too large for the L2s) against the
+// 512 cycles of the 2 NPR pixels of a step, so a step's fetches are under way while the step before is multiplied.
+// Measured at C=256, 4 levels, r=4, the whole backward (d_f1 runs beside this): B=2, 55x128 300 us with pixels taken 64 at a
+// time and fetched when needed, 267 like this; B=1 189 and 157; B=12, 40x56 458 and 420; one or four pairs a step, lists of
+// 256 pixels: 269, 271, 271.
+// VEC: a lane holds channels c0 + 4 l32 + cb and fetches them as one float4 (C a multiple of 4, f1 aligned); otherwise
+// c0 + 32 cb + l32.  No barrier, no atomics.
 typedef float lk_v16f __attribute__((ext_vector_type(16)));
 
+template <bool VEC>
 __global__ void __launch_bounds__(64) lookup_df2_kernel(const LookupBwdArgs a) {
     constexpr int NB = NCH / 32;                               // operand-B registers (32 channels each) per pixel pair
+    __shared__ int2 list[CHUNK];                               // pixel; its origin relative to the tile's, y << 16 | x
     const int G = 2 * a.r + 2, GG = G * G, C = a.C;
     const int lane = threadIdx.x, half = lane >> 5, l32 = lane & 31;
     int l = 0;
@@ -520,11 +528,17 @@ __global__ void __launch_bounds__(64) lookup_df2_kernel(const LookupBwdArgs a) {
     const int P = a.H1 * a.W1;
     const int per = (P + S - 1) / S, p_begin = slice * per, p_end = min(P, p_begin + per);
     const size_t pl0 = ((size_t)b * a.L + l) * P;
-    const int *__restrict__ org = a.org + pl0 * 2;
+    const int2 *__restrict__ org = reinterpret_cast<const int2 *>(a.org) + pl0;
     const float *__restrict__ wg = a.wg + pl0 * GG;
     const float *__restrict__ f1 = a.f1 + (size_t)b * P * C;
-    // operand A row of this lane: tile position l32; operand B columns: channels c0 + 32*cb + l32
-    const int qy = ty0 + l32 / TQX, qx = tx0 + l32 % TQX;
+    // operand A row of this lane: tile position l32; operand B columns: see above, those past C repeat a channel (not stored)
+    const int qy = l32 / TQX, qx = l32 % TQX;
+    int ch[NB];
+#pragma unroll
+    for (int cb = 0; cb < NB; ++cb) {
+        const int c = c0 + (VEC ? 4 * l32 + cb : 32 * cb + l32);
+        ch[cb] = c < C ? c : VEC ? cb : 0;
+    }
 
     lk_v16f acc[NB];
 #pragma unroll
@@ -532,54 +546,72 @@ __global__ void __launch_bounds__(64) lookup_df2_kernel(const LookupBwdArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[cb][v] = 0.f;
 
-    // origins of the next 64 pixels are fetched while the current ones are worked on
-    int2 nxt = make_int2(0, 0);
-    if (p_begin + lane < p_end) nxt = *reinterpret_cast<const int2 *>(org + (size_t)(p_begin + lane) * 2);
-    for (int pc = p_begin; pc < p_end; pc += 64) {
-        const int p = pc + lane;
-        const int ox = nxt.x, oy = nxt.y;
-        if (p + 64 < p_end) nxt = *reinterpret_cast<const int2 *>(org + (size_t)(p + 64) * 2);
-        const bool hit = p < p_end && ox < tx0 + TQX && ox + G > tx0 && oy < ty0 + TQY && oy + G > ty0;
-        unsigned long long m = __ballot(hit);
-        while (m) {
+    int2 nxt[CHUNK / 64];
+    auto origins = [&](int pc) {
+#pragma unroll
+        for (int k = 0; k < CHUNK / 64; ++k) nxt[k] = org[min(pc + 64 * k + lane, P - 1)];
+    };
+    origins(p_begin);
+    for (int pc = p_begin; pc < p_end; pc += CHUNK) {
+        int count = 0;
+#pragma unroll
+        for (int k = 0; k < CHUNK / 64; ++k) {
+            const int p = pc + 64 * k + lane, ox = nxt[k].x - tx0, oy = nxt[k].y - ty0;
+            const bool hit = p < p_end && ox < TQX && ox + G > 0 && oy < TQY && oy + G > 0;
+            const unsigned long long m = __ballot(hit);
+            if (hit) list[count + __builtin_popcountll(m & ((1ull << lane) - 1))] = make_int2(p, oy * 65536 + (ox & 65535));
+            count += __builtin_popcountll(m);
+        }
+        if (pc + CHUNK < p_end) origins(pc + CHUNK);
+        if (count == 0) continue;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        struct Step {
             float wa[NPR], fb[NPR][NB];
-            bool any[NPR];
+        };
+        // the step's pixels past the list repeat its last one, with weight 0
+        auto fetch = [&](int at, Step &s) __attribute__((always_inline)) {
 #pragma unroll
             for (int pr = 0; pr < NPR; ++pr) {
-                any[pr] = m != 0;                              // wave-uniform
-                if (!any[pr]) {                                // nothing left in these 64 pixels: skip the slot
-                    wa[pr] = 0.f;
+                const int k = at + 2 * pr + half;
+                const int2 e = list[min(k, count - 1)];
+                const int gx = qx - (int)(short)e.y, gy = qy - (e.y >> 16);
+                const bool in = k < count && gx >= 0 && gx < G && gy >= 0 && gy < G;
+                const float w = wg[(size_t)e.x * GG + (in ? gy * G + gx : 0)];
+                s.wa[pr] = in ? w : 0.f;
+                const float *src = f1 + (size_t)e.x * C;
+                if constexpr (VEC) {
+                    const float4 v = *reinterpret_cast<const float4 *>(src + ch[0]);
+                    s.fb[pr][0] = v.x, s.fb[pr][1] = v.y, s.fb[pr][2] = v.z, s.fb[pr][3] = v.w;
+                } else {
 #pragma unroll
-                    for (int cb = 0; cb < NB; ++cb) fb[pr][cb] = 0.f;
-                    continue;
-                }
-                const int cn0 = m ? __builtin_ctzll(m) : 0;
-                m &= m - 1;
-                const bool two = m != 0;
-                const int cn1 = two ? __builtin_ctzll(m) : cn0;
-                m &= m - 1;
-                const bool mine = any[pr] && (half == 0 || two);
-                const int cn = half ? cn1 : cn0;
-                const int oxc = __shfl(ox, cn), oyc = __shfl(oy, cn);
-                const size_t pp = (size_t)(pc + cn);
-                const int gx = qx - oxc, gy = qy - oyc;
-                wa[pr] = mine && gx >= 0 && gx < G && gy >= 0 && gy < G ? wg[pp * GG + gy * G + gx] : 0.f;
-#pragma unroll
-                for (int cb = 0; cb < NB; ++cb) {
-                    const int c = c0 + 32 * cb + l32;
-                    fb[pr][cb] = mine && c < C ? f1[pp * C + c] : 0.f;
+                    for (int cb = 0; cb < NB; ++cb) s.fb[pr][cb] = src[ch[cb]];
                 }
             }
+        };
+        auto multiply = [&](int at, const Step &s) __attribute__((always_inline)) {
 #pragma unroll
             for (int pr = 0; pr < NPR; ++pr)
-                if (any[pr]) {
+                if (at + 2 * pr < count) {
 #pragma unroll
-                    for (int cb = 0; cb < NB; ++cb)
-                        acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(wa[pr], fb[pr][cb], acc[cb], 0, 0, 0);
+                    for (int cb = 0; cb < NB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.wa[pr], s.fb[pr][cb], acc[cb], 0, 0, 0);
                 }
+        };
+        Step s0, s1;
+        fetch(0, s0);
+        for (int at = 0; at < count; at += 4 * NPR) {
+            fetch(at + 2 * NPR, s1);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(at, s0);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(at + 4 * NPR, s0);
+            __builtin_amdgcn_sched_barrier(0);
+            multiply(at + 2 * NPR, s1);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        __builtin_amdgcn_wave_barrier();
     }
-    // register v of lane (half, l32) holds tile position 8*(v/4) + 4*half + v%4, channel c0 + 32*cb + l32
+    // register v of lane (half, l32) holds tile position 8*(v/4) + 4*half + v%4
     const size_t lvl_elems = (size_t)a.B * H2 * W2 * C;
     float *dst = (S == 1 ? a.d_f2[l] : a.part[l] + (size_t)slice * lvl_elems) + (size_t)b * H2 * W2 * C;
 #pragma unroll
@@ -588,10 +620,14 @@ __global__ void __launch_bounds__(64) lookup_df2_kernel(const LookupBwdArgs a) {
         const int y = ty0 + pos / TQX, x = tx0 + pos % TQX;
         if (y < H2 && x < W2) {
             float *d = dst + ((size_t)y * W2 + x) * C;
+            if constexpr (VEC) {
+                if (c0 + 4 * l32 < C) *reinterpret_cast<float4 *>(d + c0 + 4 * l32) = make_float4(acc[0][v], acc[1][v], acc[2][v], acc[3][v]);
+            } else {
 #pragma unroll
-            for (int cb = 0; cb < NB; ++cb) {
-                const int c = c0 + 32 * cb + l32;
-                if (c < C) d[c] = acc[cb][v];
+                for (int cb = 0; cb < NB; ++cb) {
+                    const int c = c0 + 32 * cb + l32;
+                    if (c < C) d[c] = acc[cb][v];
+                }
             }
         }
     }
@@ -778,7 +814,10 @@ int sepcorr_lookup_backward(const float *f1, const float *const *f2_levels, cons
     else hipLaunchKernelGGL(lookup_df1_kernel, dim3((unsigned)((size_t)B * H1 * W1)), dim3(256), 0, sa, a);
     int rl = launch_error("lookup d_f1 kernel");
     if (rl == SEPCORR_OK) {
-        hipLaunchKernelGGL(lookup_df2_kernel, dim3((unsigned)tiles, (C + NCH - 1) / NCH, B), dim3(64), 0, sb, a);
+        const dim3 grid((unsigned)tiles, (C + NCH - 1) / NCH, B);
+        // (the slices' results lie in the workspace, aligned; a level is always cut into two at least)
+        if (C % 4 == 0 && (uintptr_t)f1 % 16 == 0) hipLaunchKernelGGL(lookup_df2_kernel<true>, grid, dim3(64), 0, sb, a);
+        else hipLaunchKernelGGL(lookup_df2_kernel<false>, grid, dim3(64), 0, sb, a);
         rl = launch_error("lookup d_f2 kernel");
     }
     if (rl == SEPCORR_OK) {

@@ -119,6 +119,39 @@ def test_lookup_gradients_match_autograd_through_the_oracle(device, B, C, H, W, 
     assert_close(g1.grad, 2 * r1.grad, "d_fmap1 accumulated", scale_atol=True)
 
 
+@pytest.mark.parametrize("H,W,C,r,same,shift", [
+    (32, 32, 132, 4, True, 0),      # two slices of 512 pixels, all of them on one place: a full list
+    (2, 513, 132, 4, True, 0),      # 513: one pixel in a second list
+    (2, 511, 130, 4, True, 0),      # 511, an odd number of pixels; channels one by one
+    (1, 2, 8, 1, False, 0),         # a list of one pixel
+    (3, 700, 64, 3, False, 0),      # lists in the middle of a row, some of them empty
+    (5, 205, 132, 8, False, 1),     # feature map not aligned to 16 bytes
+])
+def test_feature_gradient_at_the_edges_of_the_pixel_lists(device, H, W, C, r, same, shift):
+    """d_f2 is a sum over pixels of window gradient times channel, the window gradient one of at most four products and a
+    factor: with P pixels every term meets at most P + 8 roundings, so the error is at most (P + 16) 2^-24 of the sum of the
+    terms' magnitudes (same operands without signs)."""
+    from separableflowthesis_amd import MemorySaver
+    g = torch.Generator().manual_seed(H * W + C)
+    f1, f2 = torch.randn(1, C, H, W, generator=g), torch.randn(1, C, H, W, generator=g)
+    coords = _coords(1, H, W, g, 3.0)
+    if same:
+        coords = torch.tensor([W / 2 + 0.3, H / 2 - 0.4])[None, :, None, None].expand(1, 2, H, W).contiguous()
+    up = torch.randn(1, (2 * r + 1) ** 2, H, W, generator=g)
+
+    def exact(x1, u):
+        x2 = f2.double().requires_grad_()
+        (O.lookup_direct(x1.double(), x2, coords.double(), 1, r) * u.double()).sum().backward()
+        return x2.grad.permute(0, 2, 3, 1)
+
+    nhwc = f1.permute(0, 2, 3, 1).contiguous().to(device)
+    x1 = torch.empty(nhwc.numel() + shift, device=device)[shift:].view_as(nhwc).copy_(nhwc)
+    _, (d_f2,) = MemorySaver.lookup_backward(x1, [f2.permute(0, 2, 3, 1).contiguous().to(device)], coords.to(device), up.to(device), r,
+                                             C ** -0.5)
+    bound = (H * W + 16) * 2.0 ** -24 * exact(f1.abs(), up.abs())
+    assert ((d_f2.cpu().double() - exact(f1, up)).abs() <= bound).all()
+
+
 def test_lookup_backward_is_deterministic_and_checks_its_workspace(device):
     import ctypes
     from separableflowthesis_amd import MemorySaver, _lib
