@@ -409,9 +409,12 @@ __global__ void __launch_bounds__(256) lookup_df1_kernel(const LookupBwdArgs a) 
 // d_f1 for C a multiple of 4: a wave takes NPX consecutive pixels and, level by level, walks the bounding box of their
 // windows once.  Lane = 4 channels (float4 fetch of a whole fmap2 row per wave and box point); the NPX weights of a box
 // point (zero outside a pixel's own window or outside the level) sit in a per-wave LDS table and arrive as one
-// broadcast read.  Scattered windows (box above BOXMAX points) are walked pixel by pixel with the same code.
+// broadcast read, and so does the point's place in fmap2: worked out on the way it took as many vector instructions as the
+// sums (whole backward, C=256, 4 levels, B=2, 55x128: 267 -> 247 us; B=12, 40x56: 420 -> 394; eight points a trip, or the
+// place as a scalar: 281).  Scattered windows (box above BOXMAX points) are walked pixel by pixel with the same code.
 __global__ void __launch_bounds__(256) lookup_df1_group_kernel(const LookupBwdArgs a) {
     __shared__ __attribute__((aligned(16))) float wtab[4][BOXMAX][NPX];
+    __shared__ int otab[4][BOXMAX];
     const int G = 2 * a.r + 2, GG = G * G, C = a.C;
     // (the wave index stays a vector value here: with it as a scalar the walk measured slower, 0.137 against 0.127 ms)
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -419,6 +422,7 @@ __global__ void __launch_bounds__(256) lookup_df1_group_kernel(const LookupBwdAr
     if (j0 >= a.W1) return;                                 // whole wave; the kernel has no workgroup barrier
     const size_t plane = (size_t)a.H1 * a.W1;
     float (*wt)[NPX] = wtab[wave];
+    int *ot = otab[wave];
     for (int c0 = 0; c0 < C; c0 += 256) {
         const int ch = c0 + lane * 4;
         const int chl = ch < C ? ch : 0;                    // idle lanes re-read channel 0 and store nothing
@@ -466,14 +470,13 @@ __global__ void __launch_bounds__(256) lookup_df1_group_kernel(const LookupBwdAr
                         w[e] = use ? a.wg[pl[e] * GG + gy * G + gx] : 0.f;
                     }
                     *reinterpret_cast<float4 *>(wt[bp]) = make_float4(w[0], w[1], w[2], w[3]);
+                    ot[bp] = (min(max(yy, 0), H2 - 1) * W2 + min(max(xx, 0), W2 - 1)) * C;
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
-                int bx = 0, by = 0;
 #pragma unroll 4
                 for (int bp = 0; bp < npts; ++bp) {
-                    const int yc = min(max(qy0 + by, 0), H2 - 1), xc = min(max(qx0 + bx, 0), W2 - 1);
-                    const float4 v = *reinterpret_cast<const float4 *>(f2 + ((size_t)yc * W2 + xc) * C);
+                    const float4 v = *reinterpret_cast<const float4 *>(f2 + ot[bp]);
                     const float4 w = *reinterpret_cast<const float4 *>(wt[bp]);
                     const float ws[NPX] = {w.x, w.y, w.z, w.w};
 #pragma unroll
@@ -483,7 +486,6 @@ __global__ void __launch_bounds__(256) lookup_df1_group_kernel(const LookupBwdAr
                         acc[e].z = fmaf(ws[e], v.z, acc[e].z);
                         acc[e].w = fmaf(ws[e], v.w, acc[e].w);
                     }
-                    if (++bx == BW) { bx = 0; ++by; }
                 }
             }
         }
