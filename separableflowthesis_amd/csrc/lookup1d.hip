@@ -222,9 +222,10 @@ int run(bool backward, const float *corr, const float *coords, const float *gout
             hipLaunchKernelGGL(lookup1d_backward_columns_kernel, dim3((unsigned)((total + 255) / 256)), block, 0, s, a);
     }
     // by samples up to where the columns alone keep the chip busy; measured, 4 levels, radius 4, by columns / by samples:
-    // 55x128 1 channel 13.5 / 7.4 us, B=2 with 8 channels (112 640 columns) 35.9 / 35.5, 24 channels (337 920) 200 / 191, B=12
-    // with 8 channels (675 840) 455 / 505
-    else if (total < (size_t)384 * 1024 && levels * n <= 65535)
+    // 55x128 1 channel 13.5 / 7.4 us; both volumes of a block, the first clamped and not: B=2 with 4 channels (56 320 columns)
+    // 44 / 35 and 52 / 35, 8 channels (112 640) 54 / 44 and 60 / 59, 40x56 with 24 (107 520) 52 / 45 and 59 / 63, 55x128 with 24
+    // (168 960) 70 / 67 and 116 / 138, B=2 with 24 (337 920) 114 / 121 and 267 / 261
+    else if (total < (size_t)64 * 1024 && levels * n <= 65535)
         hipLaunchKernelGGL(lookup1d_forward_samples_kernel, dim3((unsigned)((total + 255) / 256), levels * n), block, 0, s, a);
     else hipLaunchKernelGGL(lookup1d_forward_kernel, dim3((unsigned)((total + 255) / 256), levels), block, 0, s, a);
     const hipError_t e = hipGetLastError();

@@ -56,8 +56,8 @@ def test_without_the_clamp_both_volumes_follow_the_plain_definition(device):
 
 @pytest.mark.parametrize("shape,levels,radius", [((1, 2, 70, 5, 77), 6, 16),      # levels of 16 and 32 entries, windows wider than the volume
                                                  ((2, 1, 9, 3, 85), 4, 4),        # one entry at the last level
-                                                 ((1, 63, 8, 78, 80), 3, 2),      # 393 120 columns: a thread per sample
-                                                 ((1, 64, 8, 77, 80), 3, 2)])     # 394 240: a thread per column
+                                                 ((1, 13, 8, 71, 71), 3, 2),      # 65 533 columns: a thread per sample
+                                                 ((1, 16, 8, 64, 64), 3, 2)])     # 65 536: a thread per column
 @pytest.mark.parametrize("clamp", [False, True])
 def test_forward_forms_against_the_definition(device, shape, levels, radius, clamp):
     from separableflowthesis_amd import MemorySaver
