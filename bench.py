@@ -42,7 +42,8 @@ WORKLOADS = {
 OPS_TEXT = "(f=max/argmax/avg fwd, c=compression fwd, C=compression bwd, F=max/avg bwd)"
 PASSES = {"f": 1, "c": 1, "C": 3, "F": 2}
 # kernels that execute one contraction pass (W = 2*B*N1*N2*C flops) per launch
-SWEEP_KERNELS = ("fwd_maxavg", "fwd_weighted", "fwd_maxavg_split", "fwd_weighted_split", "df1_comp", "df2_comp", "df1_maxavg", "df2_maxavg", "df1_both", "df2_both")
+SWEEP_KERNELS = ("fwd_maxavg", "fwd_weighted", "fwd_maxavg_split", "fwd_weighted_split", "df1_comp", "df2_comp", "df1_maxavg", "df2_maxavg", "df1_both", "df2_both",
+                 "df1_comp_split", "df2_comp_split", "df1_both_split", "df2_both_split")
 _MIB = 2 ** 20
 
 

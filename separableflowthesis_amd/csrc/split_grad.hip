@@ -1062,7 +1062,7 @@ int launch_all(const GradArgs &a, hipStream_t s) {
         if (rc) return rc;
     }
     for (int first = 1; first >= 0; --first) {
-        void *prof = sepcorr_prof_begin(first ? "df1_split" : "df2_split", s);
+        void *prof = sepcorr_prof_begin(first ? (BOTH ? "df1_both_split" : "df1_comp_split") : (BOTH ? "df2_both_split" : "df2_comp_split"), s);
         const int rc = a.ncb == 2 ? launch_contraction<BOTH, KC, 2>(a, s, first)
                      : a.ncb == 4 ? launch_contraction<BOTH, KC, 4>(a, s, first) : launch_contraction<BOTH, KC, 8>(a, s, first);
         if (first) hipLaunchKernelGGL((grad_finish_kernel<true, BOTH, KC>), dim3(a.B * (a.N1p / TPX) * a.ncb), dim3(256), 0, s, a);

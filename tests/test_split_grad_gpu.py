@@ -91,7 +91,8 @@ def _labels_of(fn):
 def test_against_float64(device, dims, K, both):
     x = _tensors(device, dims, K, seed=K)
     got = []
-    assert {"df1_split", "df2_split"} <= _labels_of(lambda: got.extend(_run(x, both)))
+    kind = "both" if both else "comp"
+    assert {f"df1_{kind}_split", f"df2_{kind}_split"} <= _labels_of(lambda: got.extend(_run(x, both)))
     ref = _exact(x, both)
     # An operand's halves hold 22 bits (an error of 2^-23 of it at the most, 0.7e-7 in the mean), dL/dS itself is a sum of up to 15
     # fp32 terms, and at most 96 sums follow one another before they are put apart: 1.3e-7 to 1.9e-7 for d_f1 and up to
