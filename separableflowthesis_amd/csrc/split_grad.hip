@@ -36,6 +36,7 @@
 
 #include "sepcorr.h"
 #include "sepcorr_internal.h"
+#include "split_grad_deal.h"
 
 #ifndef GRAD_PART
 #define GRAD_PART (-1)
@@ -53,9 +54,6 @@ typedef unsigned v4u __attribute__((ext_vector_type(4)));
 constexpr int TPX = 128;      // pixels of a d_f1 tile
 constexpr int ROWS = 8;       // rows of fmap2 of a d_f2 tile
 constexpr unsigned OOB = 0x80000000u;   // a byte offset above every buffer size used here: reads as zero
-// Steps whose sums the registers take before they are added to the piece's slot.  d_f1 / d_f2 at B=2, 55x128: 24 steps 1.69e-7
-// / 2.5e-7, 813 us a backward call; 48 1.86e-7 / 3.2e-7, 740 us; 96 2.14e-7 / 4.3e-7 (before the signs of block_sign()).
-constexpr int FLUSH = 48;
 // One feature in so many may be below 2^-17 of its channel's largest.  (Of normal ones one in 37 000 is; beside a single one
 // of 2^17 times the rest a whole channel, one in 256 at the most.)
 constexpr unsigned SMALL_SHARE = 2048;
@@ -111,20 +109,6 @@ __device__ __forceinline__ bool unsuitable(const GradArgs &a) {
     return a.count[2] != 0 || a.count[0] > (unsigned)((size_t)a.B * a.N1 * a.C / SMALL_SHARE) ||
            a.count[1] > (unsigned)((size_t)a.B * a.H2 * a.W2 * a.C / SMALL_SHARE);
 }
-
-// The workgroups that hold the steps [t0, t1) when T steps are dealt out evenly to G workgroups.
-__device__ __forceinline__ void pieces_of(long t0, long t1, int G, long T, int &w0, int &w1) {
-    w0 = (int)((t0 * G) / T);
-    while (w0 > 0 && ((long)w0 * T) / G > t0) --w0;
-    while (((long)(w0 + 1) * T) / G <= t0) ++w0;
-    w1 = w0;
-    while (((long)(w1 + 1) * T) / G < t1) ++w1;
-}
-// Slot of the piece that workgroup wg has of a tile (it is not its first step there if `inside`).
-__host__ __device__ __forceinline__ int slot_of(int wg, int tile, bool inside, int tiles, int G) {
-    return tiles < G ? wg + tile : 2 * wg + (inside ? 0 : 1);
-}
-__host__ __device__ __forceinline__ long slots_of(long tiles, int G) { return tiles < G ? G + tiles : 2L * G; }
 
 // Four consecutive columns from v on of a row of W2, zeros beyond it.
 __device__ __forceinline__ v4f columns4(const float *row, int v, int W2, bool ok) {
@@ -512,7 +496,7 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
     const long T = (long)tiles * spt, t0 = (long)tile * spt;
     int w0, w1;
     pieces_of(t0, t0 + spt, G, T, w0, w1);
-    if (w0 == w1 && spt <= FLUSH) return;   // (its workgroup has written it)
+    if (w0 == w1) return;   // (its workgroup has written it)
     const int ug = tile % nug, bv = tile / nug, u = ROWS * ug + row;   // (d_f2)
     if (!FIRST && u >= a.H2) return;
     const size_t slot = (size_t)per * 1024;
@@ -523,7 +507,7 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int w = min(wb + i, w1);
-            const v4f *src = reinterpret_cast<const v4f *>(a.slots + slot_of(w, tile, (long)w * T / G > t0, tiles, G) * slot + sub * 1024) + lane;
+            const v4f *src = reinterpret_cast<const v4f *>(a.slots + slot_of(w, tile, first_step(w, G, T) > t0, tiles, G) * slot + sub * 1024) + lane;
 #pragma unroll
             for (int q = 0; q < 4; ++q) y[i][q] = src[q * 64];
         }
@@ -547,19 +531,19 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
 // result (d_f1 at 136x240, error against 64 bits: 2.66e-7 as products of one sign).
 __device__ __forceinline__ float block_sign(int odd) { return odd & 1 ? -1.f : 1.f; }
 
-// What a lane leaves of its block in a piece's slot; a later flush of the same piece adds to it.
-__device__ __forceinline__ void put_block(float *slot, int sub, bool first, const v16f &x, float sign) {
-    v4f *d = reinterpret_cast<v4f *>(slot + sub * 1024) + (threadIdx.x & 63);
+// A piece's sums of a lane's block: what earlier flushes left of it in its slot (none if `first`), and x.
+__device__ __forceinline__ void sums_of_piece(const v4f *slot, bool first, const v16f &x, float sign, float (&y)[16]) {
     v4f old[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) old[q] = first ? v4f{0.f, 0.f, 0.f, 0.f} : d[q * 64];
+    for (int q = 0; q < 4; ++q) old[q] = first ? v4f{0.f, 0.f, 0.f, 0.f} : slot[q * 64];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        v4f y;
+    for (int r = 0; r < 16; ++r) y[r] = fmaf(sign, x[r], old[r >> 2][r & 3]);
+}
+__device__ __forceinline__ v4f *block_of(float *slot, int sub) { return reinterpret_cast<v4f *>(slot + sub * 1024) + (threadIdx.x & 63); }
+// Leaves them in the slot; a later flush of the same piece adds to it.
+__device__ __forceinline__ void put_block(v4f *slot, const float (&y)[16]) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y[e] = fmaf(sign, x[4 * q + e], old[q][e]);
-        d[q * 64] = y;
-    }
+    for (int q = 0; q < 4; ++q) slot[q * 64] = v4f{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
 }
 
 // dL/dS, scaled, of one column at the pixel whose u-indexed weights are wu; wv(f): its v-indexed weights, the max/average
@@ -606,7 +590,7 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
     const int wg = xcd_contiguous(blockIdx.x, gridDim.x), npt = a.N1p / TPX, H2 = a.H2;
     const int spt = a.nvc * H2, tiles = a.B * npt;
     const long T = (long)tiles * spt;
-    const int g0 = (int)(wg * T / a.G1), g1 = (int)((wg + 1) * T / a.G1);
+    const int g0 = (int)first_step(wg, a.G1, T), g1 = (int)first_step(wg + 1, a.G1, T);
     v16f acc[MP][MC];
     int held = 0;              // steps in acc
     bool first = true;         // nothing of this piece is in its slot yet
@@ -614,7 +598,7 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
         const int tile = g / spt, r0 = g - tile * spt, vc = r0 / H2, ua = r0 - vc * H2;
         const int b = tile / npt, pt = tile - b * npt;
         const int ub = min(min(H2, ua + g1 - g), ua + FLUSH - held);
-        const int pstart = max(0, g0 - tile * spt);                       // first step of this piece
+        const Piece piece = piece_of(tile, g0, g1, spt);
         g += ub - ua;
         const __amdgpu_buffer_rsrc_t rs = make_rsrc(a.f2h + (size_t)(b * a.nvc + vc) * H2 * BLK, (unsigned)H2 * BLK);
         auto dma = [&](int u, int buf) __attribute__((always_inline)) {
@@ -788,25 +772,20 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (what was requested past the last row, before the buffers are used again)
         held += ub - ua;
         const int rend = r0 + ub - ua;
-        const bool ends = g == g1 || rend == spt;
+        const bool ends = rend == piece.end;
         if (!ends && held < FLUSH) continue;
-        if (rend == spt && pstart == 0 && spt <= FLUSH) {
+        float *slot = a.slots + (size_t)slot_of(wg, tile, piece.begin > 0, tiles, a.G1) * 4 * NCB * 1024;
+        const bool out = ends && piece.whole(spt);
 #pragma unroll
-            for (int i = 0; i < MP; ++i)
+        for (int i = 0; i < MP; ++i)
 #pragma unroll
-                for (int j = 0; j < MC; ++j) {
-                    float z[16];
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) z[r] = acc[i][j][r];
-                    store_block<true, true>(a, b, 0, TPX * pt + 32 * (mp0 + i), 32 * (mc0 + j), z);
-                }
-        } else {
-            float *slot = a.slots + (size_t)slot_of(wg, tile, pstart > 0, tiles, a.G1) * 4 * NCB * 1024;
-#pragma unroll
-            for (int i = 0; i < MP; ++i)
-#pragma unroll
-                for (int j = 0; j < MC; ++j) put_block(slot, (mp0 + i) * NCB + mc0 + j, first, acc[i][j], 1.f);
-        }
+            for (int j = 0; j < MC; ++j) {
+                float y[16];
+                v4f *block = block_of(slot, (mp0 + i) * NCB + mc0 + j);
+                sums_of_piece(block, first, acc[i][j], 1.f, y);
+                if (out) store_block<true, true>(a, b, 0, TPX * pt + 32 * (mp0 + i), 32 * (mc0 + j), y);
+                else put_block(block, y);
+            }
         held = 0;
         first = ends;
     }
@@ -839,14 +818,14 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
     const int rp = wave & 3, half = wave >> 2;                           // rows 2 rp, 2 rp + 1; columns 16 half.. / channels
     const int wg = xcd_contiguous(blockIdx.x, gridDim.x), nug = a.H2p / ROWS, spt = a.npx, tiles = a.B * nug * a.nvc;
     const long T = (long)tiles * spt;
-    const int g0 = (int)(wg * T / a.G2), g1 = (int)((wg + 1) * T / a.G2);
+    const int g0 = (int)first_step(wg, a.G2, T), g1 = (int)first_step(wg + 1, a.G2, T);
     const float inv_h2 = 1.f / (float)a.H2;
     bool first = true;
     for (int g = g0; g < g1;) {
         const int tile = g / spt, ta = g - tile * spt, tb = min(min(spt, ta + g1 - g), (ta / FLUSH + 1) * FLUSH);
         // (row groups of one column chunk follow each other: the workgroups of an XCD then read the same weights)
         const int ug = tile % nug, bv = tile / nug, vc = bv % a.nvc, b = bv / a.nvc;
-        const int pstart = max(0, g0 - tile * spt);
+        const Piece piece = piece_of(tile, g0, g1, spt);
         g += tb - ta;
         // A step's requests: f1 of that step and the weights of the one after it, whose dL/dS is formed during it.  This
         // wave's i-th one is KB 8 i + wave of the two together; every wave makes the same number of them.
@@ -1004,26 +983,19 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
         }
         if (wave < 4) phase_end();
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (what was requested past the last step, before the buffers are used again)
-        const bool ends = g == g1 || tb == spt;
-        if (tb == spt && pstart == 0 && spt <= FLUSH) {
+        const bool ends = tb == piece.end;
+        float *slot = a.slots + (size_t)slot_of(wg, tile, piece.begin > 0, tiles, a.G2) * ROWS * NCB * 1024;
+        const bool out = ends && piece.whole(spt);
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                if (u0 + r >= a.H2) continue;
+        for (int r = 0; r < 2; ++r)
 #pragma unroll
-                for (int j = 0; j < MC; ++j) {
-                    float z[16];
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) z[e] = acc[r][j][e];
-                    store_block<false, true>(a, b, u0 + r, 32 * vc, 32 * (half * MC + j), z);
-                }
+            for (int j = 0; j < MC; ++j) {
+                float y[16];
+                v4f *block = block_of(slot, (2 * rp + r) * NCB + half * MC + j);
+                sums_of_piece(block, first, acc[r][j], block_sign(ta / FLUSH), y);
+                if (!out) put_block(block, y);
+                else if (u0 + r < a.H2) store_block<false, true>(a, b, u0 + r, 32 * vc, 32 * (half * MC + j), y);
             }
-        } else {
-            float *slot = a.slots + (size_t)slot_of(wg, tile, pstart > 0, tiles, a.G2) * ROWS * NCB * 1024;
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int j = 0; j < MC; ++j) put_block(slot, (2 * rp + r) * NCB + half * MC + j, first, acc[r][j], block_sign(ta / FLUSH));
-        }
         first = ends;
     }
 }

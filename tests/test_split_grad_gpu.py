@@ -2,7 +2,7 @@
 
 Sizes at the edges of its tiles: pixels around multiples of 16 and 128, rows around multiples of 8, columns around
 multiples of 32 and rows that are no multiple of 4 long (their weights are laid out anew), channels around the 64/128/256
-they are padded to; and operands that have no halves, which it multiplies in fp32.
+they are padded to, tiles around the number of workgroups; and operands that have no halves, which it multiplies in fp32.
 """
 import ctypes
 
@@ -18,6 +18,17 @@ pytestmark = pytest.mark.gpu
 SHAPES = [((1, 30, 82, 74, 35, 32), 1), ((2, 31, 64, 61, 36, 33), 4), ((1, 63, 65, 33, 65, 64), 3), ((1, 41, 91, 62, 32, 65), 2),
           ((1, 36, 64, 33, 68, 128), 4), ((3, 21, 43, 55, 36, 130), 1), ((1, 47, 48, 42, 36, 255), 3), ((2, 24, 49, 27, 97, 256), 2),
           ((1, 16, 8, 136, 240, 256), 4), ((1, 72, 120, 8, 24, 256), 4), ((1, 33, 47, 17, 100, 256), 6)]
+
+
+# More tiles than workgroups (256), or as many: tiles of d_f1 x their steps, tiles of d_f2 x theirs.  Up to 48 steps a tile's
+# sums stay in registers, above that what a workgroup has of it passes through its slot.
+MANY_TILES = [((33, 32, 32, 64, 32, 32), 1),     # 264 x 64, 264 x 64
+              ((32, 32, 32, 49, 32, 32), 2),     # 256 x 49, 224 x 64
+              ((33, 24, 32, 64, 32, 64), 1),     # 198 x 64, 264 x 48
+              ((33, 32, 32, 24, 64, 40), 1),     # 264 x 48, 198 x 64
+              ((12, 64, 128, 49, 8, 33), 1),     # 768 x 49, 84 x 512: three tiles a workgroup
+              ((12, 28, 28, 128, 128, 32), 1),   # 84 x 512, 768 x 49
+              ((7, 61, 83, 51, 37, 100), 3)]     # 280 x 102, 98 x 317
 
 
 def _tensors(device, dims, K, seed=0):
@@ -87,7 +98,7 @@ def _labels_of(fn):
 
 
 @pytest.mark.parametrize("both", [False, True], ids=["compression", "combined"])
-@pytest.mark.parametrize("dims,K", SHAPES, ids=str)
+@pytest.mark.parametrize("dims,K", SHAPES + MANY_TILES, ids=str)
 def test_against_float64(device, dims, K, both):
     x = _tensors(device, dims, K, seed=K)
     got = []
