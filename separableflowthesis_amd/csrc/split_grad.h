@@ -26,10 +26,11 @@ struct GradArgs {
     int direct;                               // the v-indexed weights are read where they are, not from pv
     float *pv;                                // [B][nvc][N1p / 16][field][8 groups of columns][16 pixels][4 columns]
     float *pu;                                // [B][H2p][N1p][u-indexed fields]
-    float *back;                              // [B][N1p] what takes a pixel's factor back, 0 where G is zero
-    float *block_back, *top_back;             // the largest of 16 pixels, negative if one has no factor; of an image
+    float *pscale;                            // [B][N1p] power of two that dL/dS of a pixel is multiplied by in d_f1
+    int *block_bad;                           // whether one of 16 pixels has none
+    float *bound_v, *bound_u;                 // [B][nvc][N1p / 16][bounds][32], [B][N1p / 16][bounds][H2p]: see grad_prepare_kernel
     unsigned *pmax;                           // [2][B][slab][256] largest |f1|, |f2| of a channel
-    float *cback;                             // [2][B][256] what takes a channel's factor back
+    int *cback;                               // [2][B][256] the power of two that takes a channel's factor back
     unsigned *count;                          // small values of f1, of f2; whether anything else is unsuitable
     char *f1h, *f2h;                          // halves of f1 [B][npx], of f2 [B][nvc][H2]
     VField vfield[11];                        // the v-indexed weights

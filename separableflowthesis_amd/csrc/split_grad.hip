@@ -8,14 +8,19 @@
 // Halves.  Both operands of a product are written as h + l, h = fp16(x), l = fp16(x - h), and multiplied as h h + h l + l h
 // with v_mfma_f32_32x32x16_f16, accumulated in fp32.  The contraction runs over pixels, so a scale may depend on anything
 // that is not summed over, or be split between the two factors:
-//   features   a power of two per image and channel, largest value into [2^14, 2^15), taken back at the end;
-//   G          a power of two per pixel p from a bound of |G[p,:]|; d_f1 takes it back at the end, in d_f2 image 1 carries it.
+//   features   a power of two per image and channel, largest value into [2^14, 2^15);
+//   G, d_f1    a power of two per pixel p from a bound of |G[p,:]|;
+//   G, d_f2    a power of two per position q of image 2 and FLUSH steps of pixels, from bounds of |G[p,q]| over 16 pixels each
+//              (grad_prepare_kernel): a row of d_f2 that all attention avoids, or that only pixels of small gradients reach,
+//              has its own.  (Summed over p with one factor per pixel, rows 2^-17, 2^-23, 2^-29 of the largest were off by
+//              2e-6, 2e-4, 8e-3.)
 // 22 bits are held down to 2^-17 of the largest value a scale stands for, 2^-39 of that below.  Operands without such a form
-// (inf, NaN, a largest value outside [2^-60, 2^61), more than one feature in 2048 below 2^-17 of its channel's largest)
-// are found on the way, and the contractions then run in fp32 from the inputs instead (contract_fp32).
+// (inf, NaN, more than one feature in 2048 below 2^-17 of its channel's largest) are found on the way, and the contractions
+// then run in fp32 from the inputs instead (contract_fp32).
 // Relative error against 64 bits, d_f1 / d_f2, fp32 kernels -> halves: B=2, 55x128, K=4 2.2e-7 / 6.9e-7 -> 1.7e-7 / 3.0e-7;
-// 40x56 1.9e-7 / 2.1e-7 -> 1.4e-7 / 1.7e-7; 136x240 2.4e-7 / 9.0e-7 -> 1.8e-7 / 3.3e-7; B=2, 47x61, C=100, K=2 2.1e-7 /
-// 3.5e-7 -> 1.3e-7 / 2.0e-7.
+// 40x56 1.9e-7 / 2.1e-7 -> 1.3e-7 / 1.5e-7, of single rows at the most 2.6e-7 / 3.1e-7 -> 1.6e-7 / 3.2e-7, also with attention
+// that avoids half of image 2 by 40 in the logits or with gradients of 2^-40..1; 136x240 2.4e-7 / 9.0e-7 -> 1.8e-7 / 3.3e-7;
+// B=2, 47x61, C=100, K=2 2.1e-7 / 3.5e-7 -> 1.3e-7 / 2.0e-7.
 //
 // Work split.  A workgroup of eight waves, one per compute unit, owns 128 pixels x all channels of d_f1, or 8 rows x 32
 // columns x all channels of d_f2 (64 or 128 accumulator registers a lane), and takes a step at a time: 32 columns of a row of
@@ -62,8 +67,10 @@ constexpr int SLABS = 16;     // blocks per image and tensor that look for the l
 
 // Fields of the v-indexed weights of a pixel and column: a_u[k], g_cv[k] (, g_v[max], g_v[avg], argmax_v), as they are.
 __host__ __device__ constexpr int vfields(bool both, int kc) { return 2 * kc + (both ? 3 : 0); }
-// Of the u-indexed ones, times the pixel's factor s: s g_cu[k], s a_v[k] (, s (g_u[max] + g_u[avg] / W2), s g_u[avg] / W2, argmax_u, s).
-__host__ __device__ constexpr int ufields(bool both, int kc) { return (2 * kc + (both ? 4 : 0) + 3) & ~3; }
+// Of the u-indexed ones: g_cu[k], a_v[k] (, g_u[max] + g_u[avg] / W2, g_u[avg] / W2, argmax_u).
+__host__ __device__ constexpr int ufields(bool both, int kc) { return (2 * kc + (both ? 3 : 0) + 3) & ~3; }
+// Bounds of a block of 16 pixels, by columns and by rows (grad_prepare_kernel).
+__host__ __device__ constexpr int nbounds(bool both) { return both ? 3 : 2; }
 
 // floats between the u-indexed rows of a pixel in LDS (16 bytes aligned, banks apart)
 __host__ __device__ __forceinline__ int u_row(int H2) { return (H2 + ROWS - 1) / ROWS * ROWS + 4; }
@@ -85,22 +92,33 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *p, unsig
 __device__ __forceinline__ void dma16(__amdgpu_buffer_rsrc_t rs, void *lds, unsigned lane_off, unsigned off) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void *)lds, 16, lane_off, off, 0, 0);
 }
-// largest magnitude (its bits) -> factor into [2^14, 2^15) and the factor back; false: no such form
-__device__ __forceinline__ bool scale_of(unsigned m, float &fwd, float &back) {
-    const unsigned e = m >> 23;
-    fwd = back = 1.f;
-    if (m == 0) return true;
-    if (e < 67 || e > 187) return false;
-    fwd = __uint_as_float((268u - e) << 23);
-    back = __uint_as_float((e - 14u) << 23);
-    return true;
+// largest magnitude -> the power of two that brings it into [2^14, 2^15), at most 2^126 (below 2^-112 it stays smaller: a bit
+// of the halves is then one of the smallest numbers there are)
+__device__ __forceinline__ int scale_exponent(float m) { return 141 - (int)max(magnitude(m) >> 23, 15u); }
+__device__ __forceinline__ float power(int e) { return __uint_as_float((unsigned)(e + 127) << 23); }
+__device__ __forceinline__ int exponent_of(float p) { return (int)(__float_as_uint(p) >> 23) - 127; }
+// the largest of 16 lanes in a row, for all of them
+__device__ __forceinline__ unsigned max16(unsigned x) {
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x128, 0xf, 0xf, true));   // (row_ror)
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x124, 0xf, 0xf, true));
+    x = max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x122, 0xf, 0xf, true));
+    return max(x, (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x121, 0xf, 0xf, true));
 }
+__device__ __forceinline__ float max16(float x) { return __uint_as_float(max16(__float_as_uint(x))); }   // (none negative)
 // x, y -> their high halves in one register, their low halves in another: x - h is exact and rounded once
 __device__ __forceinline__ void split2(float x, float y, unsigned &h, unsigned &l) {
     asm("v_cvt_pk_f16_f32 %0, %2, %3\n\t"
         "v_fma_mixlo_f16 %1, %0, -1.0, %2 op_sel_hi:[1,0,0]\n\t"
         "v_fma_mixhi_f16 %1, %0, -1.0, %3 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
         : "=&v"(h), "=&v"(l) : "v"(x), "v"(y));
+}
+// the same of x s, y t, s and t powers of two
+__device__ __forceinline__ void split2(float x, float y, float s, float t, unsigned &h, unsigned &l) {
+    asm("v_fma_mixlo_f16 %0, %2, %4, 0\n\t"
+        "v_fma_mixhi_f16 %0, %3, %5, 0\n\t"
+        "v_fma_mixlo_f16 %1, %2, %4, -%0 op_sel_hi:[0,0,1]\n\t"
+        "v_fma_mixhi_f16 %1, %3, %5, -%0 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+        : "=&v"(h), "=&v"(l) : "v"(x), "v"(y), "v"(s), "v"(t));
 }
 __device__ __forceinline__ void phase_end() { asm volatile("s_barrier" ::: "memory"); }
 __device__ __forceinline__ v16f mfma(v8h a, v8h b, v16f c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
@@ -134,13 +152,17 @@ __device__ __forceinline__ const float *vrow(const GradArgs &a, int f, size_t bp
 // What both contractions need beforehand, bound by its traffic: 82 MB read and 29 written in 32 us at B=2, 55x128, K=4 (46 with
 // the channels' blocks behind the others and one channel a lane; 59 more with atomics for the channels' maxima).
 // Blocks [0, 2 B SLABS): the largest magnitude of every channel of a slab of f1 or f2.
-// The blocks behind them: the weights of 16 pixels and their factor.  |G[p,:]| <= beta = sum_k max|a_u| max|g_cu| + max|a_v|
-// max|g_cv| (+ the largest max/average gradients); the factor brings beta into [2^14, 2^15).  It goes into the u-indexed
-// weights (and the max/average terms), which makes it a factor of G.
+// The blocks behind them: the weights of 16 pixels, and what bounds |G| there,
+//   |G[p,u,v]| <= sum_k |a_u[k,v] g_cu[k,u]| + sum_k |a_v[k,u] g_cv[k,v]| (+ the max/average gradients):
+//   the pixel's factor (d_f1) brings beta = sum_k max|a_u| max|g_cu| + max|a_v| max|g_cv| (+ ..) into [2^14, 2^15);
+//   the factors of d_f2 go by positions of image 2 (split_d2_kernel) and need, of the 16 pixels together, for every column
+//     X = max_p sum_k |a_u[k,v]| max_u |g_cu[k]|,  X' = max_p sum_k |g_cv[k,v]| max_u |a_v[k]|  (, |g_v[max]| + |g_v[avg]| / H2),
+//   for every row Y and Y' likewise (, |g_u[max]| + |g_u[avg]| / W2): |G| <= min(X, Y) + min(X', Y') (+ both others).
 template <bool BOTH, int KC>
 __global__ void __launch_bounds__(256) grad_prepare_kernel(const GradArgs a) {
-    constexpr int NF = vfields(BOTH, KC), NU = ufields(BOTH, KC), NR = 2 * KC + (BOTH ? 3 : 0);
-    __shared__ float sfwd[16], sback[16];
+    constexpr int NF = vfields(BOTH, KC), NU = ufields(BOTH, KC), NR = 2 * KC + (BOTH ? 3 : 0), NX = nbounds(BOTH);
+    constexpr int NM = 2 * KC + (BOTH ? 2 : 0);
+    __shared__ unsigned smv[NM][16], smu[NM][16];   // [field][pixel]: the largest magnitude of a row
     extern __shared__ float sh[];   // [pixel][row of u-indexed weights][urow]
     const int urow = u_row(a.H2);
     const int ntile = a.N1p / 16;
@@ -180,100 +202,114 @@ __global__ void __launch_bounds__(256) grad_prepare_kernel(const GradArgs a) {
     const int b = blk / ntile, t16 = blk - b * ntile;
     const float inv_w2 = 1.f / (float)W2, inv_h2 = 1.f / (float)H2;
     if (blk == 0 && threadIdx.x < 3) a.count[threadIdx.x] = 0;
-    {
+    if ((int)threadIdx.x < NM * 16) smv[threadIdx.x / 16][threadIdx.x % 16] = 0;
+    {   // u-indexed rows: their largest magnitudes; they stay in LDS
         const int i = threadIdx.x >> 4, j = threadIdx.x & 15, pix = 16 * t16 + i;
         const bool ok = pix < N1;
         const size_t bp = (size_t)b * N1 + (ok ? pix : N1 - 1);
-        // the largest magnitude of every row, all rows' loads in flight together; the u-indexed rows stay in LDS
-        constexpr int NM = 2 * KC + (BOTH ? 2 : 0);
-        const float *vr[NM], *ur[NR];
-#pragma unroll
-        for (int f = 0; f < NM; ++f) vr[f] = vrow<KC>(a, f, bp);
+        const float *ur[NR];
 #pragma unroll
         for (int f = 0; f < NR; ++f)
             ur[f] = f < KC ? a.g_cu + (bp * a.KT + a.k0 + f) * H2 : f < 2 * KC ? a.a_v + (bp * a.KT + a.k0 + f - KC) * H2
                   : f < 2 * KC + 2 ? a.g_u + (2 * bp + f - 2 * KC) * H2 : reinterpret_cast<const float *>(a.am_u) + bp * H2;
-        unsigned mv[NM] = {}, mu[NM] = {};
-        for (int x = 4 * j; x < max(W2, a.H2p); x += 64) {
-            v4f y[NM], z[NR];
-#pragma unroll
-            for (int f = 0; f < NM; ++f) y[f] = columns4(vr[f], x, W2, x < W2);
+        unsigned mu[NM] = {};
+        for (int x = 4 * j; x < a.H2p; x += 64) {
+            v4f z[NR];
 #pragma unroll
             for (int f = 0; f < NR; ++f) z[f] = columns4(ur[f], x, H2, x < H2 && ok);
-            if (x < a.H2p) {
 #pragma unroll
-                for (int f = 0; f < NR; ++f) *reinterpret_cast<v4f *>(sh + (i * NR + f) * urow + x) = z[f];
-            }
+            for (int f = 0; f < NR; ++f) *reinterpret_cast<v4f *>(sh + (i * NR + f) * urow + x) = z[f];
 #pragma unroll
             for (int f = 0; f < NM; ++f)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    mv[f] = max(mv[f], magnitude(y[f][e]));
-                    mu[f] = max(mu[f], magnitude(z[f][e]));
-                }
+                for (int e = 0; e < 4; ++e) mu[f] = max(mu[f], magnitude(z[f][e]));
         }
-        unsigned top = 0;
 #pragma unroll
         for (int f = 0; f < NM; ++f) {
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1) {
-                mv[f] = max(mv[f], (unsigned)__shfl_xor((int)mv[f], d));
-                mu[f] = max(mu[f], (unsigned)__shfl_xor((int)mu[f], d));
-            }
-            top = max(top, max(mv[f], mu[f]));
-        }
-        float beta = 0.f;
-#pragma unroll
-        for (int f = 0; f < 2 * KC; ++f) beta += __uint_as_float(mv[f]) * __uint_as_float(mu[f]);
-        if constexpr (BOTH) {
-            beta += __uint_as_float(mu[2 * KC]) + __uint_as_float(mu[2 * KC + 1]) * inv_w2;
-            beta += __uint_as_float(mv[2 * KC]) + __uint_as_float(mv[2 * KC + 1]) * inv_h2;
-        }
-        float fwd, back;
-        const bool good = scale_of(magnitude(beta), fwd, back) && top < (188u << 23);
-        if (!ok || !good) fwd = 0.f;
-        if (!ok || !good || beta == 0.f) back = 0.f;
-        if (j == 0) {
-            sfwd[i] = fwd;
-            sback[i] = back;
-            a.back[(size_t)b * a.N1p + pix] = back;
-        }
-        const int bad = __syncthreads_or(ok && !good);
-        if (threadIdx.x < 16) {
-            float m = sback[threadIdx.x];
-#pragma unroll
-            for (int d = 1; d < 16; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-            if (threadIdx.x == 0) a.block_back[blk] = bad ? -1.f : m;
+            mu[f] = max16(mu[f]);
+            if (j == f) smu[f][i] = mu[f];
         }
     }
-    if (!a.direct) {   // v-indexed weights: 64 lanes write the four columns each of 16 pixels, 1 KB
-        const int i = threadIdx.x & 15, pix = 16 * t16 + i;
-        const bool ok = pix < N1;
+    __syncthreads();
+    const int i = threadIdx.x & 15, pix = 16 * t16 + i;
+    const bool ok = pix < N1;
+    {   // v-indexed rows: 64 lanes have the four columns each of 16 pixels
         const size_t bp = (size_t)b * N1 + (ok ? pix : N1 - 1);
+        unsigned mv[NM] = {};
+        float wu[2 * KC];
+#pragma unroll
+        for (int f = 0; f < 2 * KC; ++f) wu[f] = __uint_as_float(smu[f][i]);
         for (int vg = threadIdx.x >> 4; vg < 8 * a.nvc; vg += 16) {
-            float *dst = a.pv + (((size_t)b * a.nvc + (vg >> 3)) * ntile + t16) * NF * 512 + ((vg & 7) * 16 + i) * 4;
-            v4f y[NF];
+            v4f y[NF], x[NX] = {};
+            if (a.direct) {   // (argmax_v is only copied)
 #pragma unroll
-            for (int f = 0; f < NF; ++f) y[f] = columns4(vrow<KC>(a, f, bp), 4 * vg, W2, ok);
+                for (int f = 0; f < NM; ++f) y[f] = columns4(vrow<KC>(a, f, bp), 4 * vg, W2, ok);
+            } else {
 #pragma unroll
-            for (int f = 0; f < NF; ++f) *reinterpret_cast<v4f *>(dst + f * 512) = y[f];
+                for (int f = 0; f < NF; ++f) y[f] = columns4(vrow<KC>(a, f, bp), 4 * vg, W2, ok);
+                float *dst = a.pv + (((size_t)b * a.nvc + (vg >> 3)) * ntile + t16) * NF * 512 + ((vg & 7) * 16 + i) * 4;   // (1 KB a wave)
+#pragma unroll
+                for (int f = 0; f < NF; ++f) *reinterpret_cast<v4f *>(dst + f * 512) = y[f];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+#pragma unroll
+                for (int f = 0; f < NM; ++f) mv[f] = max(mv[f], magnitude(y[f][e]));
+#pragma unroll
+                for (int f = 0; f < 2 * KC; ++f) x[f / KC][e] = fmaf(fabsf(y[f][e]), wu[f], x[f / KC][e]);
+                if constexpr (BOTH) x[NX - 1][e] = fmaf(fabsf(y[2 * KC + 1][e]), inv_h2, fabsf(y[2 * KC][e]));
+            }
+#pragma unroll
+            for (int n = 0; n < NX; ++n) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[n][e] = max16(x[n][e]);
+                if (i == n) *reinterpret_cast<v4f *>(a.bound_v + (((size_t)b * a.nvc + (vg >> 3)) * ntile + t16) * NX * 32 + n * 32 + 4 * (vg & 7)) = x[n];
+            }
+        }
+#pragma unroll
+        for (int f = 0; f < NM; ++f) atomicMax(&smv[f][i], mv[f]);
+    }
+    __syncthreads();
+    float wv[2 * KC];
+#pragma unroll
+    for (int f = 0; f < 2 * KC; ++f) wv[f] = __uint_as_float(smv[f][i]);
+    if (threadIdx.x < 64) {
+        float beta = 0.f;
+#pragma unroll
+        for (int f = 0; f < 2 * KC; ++f) beta += wv[f] * __uint_as_float(smu[f][i]);
+        if constexpr (BOTH) {
+            beta += __uint_as_float(smu[2 * KC][i]) + __uint_as_float(smu[2 * KC + 1][i]) * inv_w2;
+            beta += __uint_as_float(smv[2 * KC][i]) + __uint_as_float(smv[2 * KC + 1][i]) * inv_h2;
+        }
+        const bool good = beta < 0x1p126f;   // (not where an operand is inf or NaN)
+        if (threadIdx.x < 16) a.pscale[(size_t)b * a.N1p + pix] = good ? power(scale_exponent(beta)) : 1.f;
+        const unsigned long long bad = __ballot(ok && !good);
+        if (threadIdx.x == 0) a.block_bad[blk] = bad != 0;
+    }
+    for (int u = threadIdx.x >> 4; u < a.H2p; u += 16) {
+        const float *r = sh + i * NR * urow + u;
+        float y[NX] = {};
+#pragma unroll
+        for (int f = 0; f < 2 * KC; ++f) y[f / KC] = fmaf(fabsf(r[f * urow]), wv[f], y[f / KC]);
+        if constexpr (BOTH) y[NX - 1] = fmaf(fabsf(r[(2 * KC + 1) * urow]), inv_w2, fabsf(r[2 * KC * urow]));
+#pragma unroll
+        for (int n = 0; n < NX; ++n) {
+            y[n] = max16(y[n]);
+            if (i == n) a.bound_u[((size_t)b * ntile + t16) * NX * a.H2p + n * a.H2p + u] = y[n];
         }
     }
     // u-indexed weights: a pixel's fields of a row together
     for (int n = threadIdx.x; n < a.H2p * 16 * (NU / 4); n += 256) {
         const int f4 = 4 * (n % (NU / 4)), pi = n / (NU / 4) % 16, u = n / (16 * (NU / 4));
         const float *r = sh + pi * NR * urow + u;
-        const float s = sfwd[pi];
         v4f y;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int f = f4 + e;
-            if (f < 2 * KC) y[e] = r[f * urow] * s;
-            else if (!BOTH || f > 2 * KC + 3) y[e] = 0.f;
-            else if (f == 2 * KC) y[e] = (r[f * urow] + r[(f + 1) * urow] * inv_w2) * s;
-            else if (f == 2 * KC + 1) y[e] = r[f * urow] * inv_w2 * s;
-            else if (f == 2 * KC + 2) y[e] = r[f * urow];
-            else y[e] = s;
+            if (f < 2 * KC) y[e] = r[f * urow];
+            else if (!BOTH || f > 2 * KC + 2) y[e] = 0.f;
+            else if (f == 2 * KC) y[e] = r[f * urow] + r[(f + 1) * urow] * inv_w2;
+            else y[e] = f == 2 * KC + 1 ? r[f * urow] * inv_w2 : r[f * urow];
         }
         *reinterpret_cast<v4f *>(a.pu + (((size_t)b * a.H2p + u) * a.N1p + 16 * t16 + pi) * NU + f4) = y;
     }
@@ -282,18 +318,15 @@ __global__ void __launch_bounds__(256) grad_prepare_kernel(const GradArgs a) {
 #if GRAD_IN_PART(0)
 // Halves of 32 pixels of a row of fmap2, or of 16 pixels of image 1, in operand order: one KB per (16 pixels, 32 channels,
 // half) holding the 16 bytes of each lane in lane order (lane 32 g + i: channel i, pixels 8 g + 0..7).  A channel is scaled
-// by a power of two that brings the largest of the image into [2^14, 2^15); image 1 also by what takes the factor of its
-// pixel's G back, over the largest such one of the image.
+// by a power of two that brings the largest of the image into [2^14, 2^15).
 template <int NCB>
 __global__ void __launch_bounds__(256) grad_split_kernel(const GradArgs a) {
     constexpr int CP = 32 * NCB;
-    __shared__ float sback[4];
     const bool second = (int)blockIdx.x < a.B * a.nvc * a.H2;
     int b, n, p0;
-    const float *src, *back = nullptr;
+    const float *src;
     char *dst;
     bool leads;   // the block that writes down the scales of its image
-    float inv = 1.f;
     bool bad = false;
     if (second) {
         const int u = blockIdx.x % a.H2, bc = blockIdx.x / a.H2, vc = bc % a.nvc;
@@ -310,21 +343,9 @@ __global__ void __launch_bounds__(256) grad_split_kernel(const GradArgs a) {
         p0 = 16 * (blk - b * a.npx);
         leads = p0 == 0;
         src = a.f1 + (size_t)b * a.N1 * a.C;
-        back = a.back + (size_t)b * a.N1p;
         dst = a.f1h + (size_t)blk * NCB * 2048;
-        float m = 0.f;
-        for (int i = threadIdx.x; i < ntile; i += 256) {
-            const float x = a.block_back[b * ntile + i];
-            bad |= x < 0.f;
-            m = fmaxf(m, x);
-        }
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d));
-        if ((threadIdx.x & 63) == 0) sback[threadIdx.x >> 6] = m;
-        __syncthreads();
-        m = fmaxf(fmaxf(sback[0], sback[1]), fmaxf(sback[2], sback[3]));
-        inv = m > 0.f ? 1.f / m : 0.f;   // (a power of two)
-        if (leads && threadIdx.x == 0) a.top_back[b] = m;
+        if (leads)
+            for (int i = threadIdx.x; i < ntile; i += 256) bad |= a.block_bad[b * ntile + i] != 0;
     }
     if (blockIdx.x == 0) {   // (from where they are: an assignment would move them to the stack)
         const unsigned *args = (const unsigned *)__builtin_amdgcn_kernarg_segment_ptr();
@@ -337,9 +358,10 @@ __global__ void __launch_bounds__(256) grad_split_kernel(const GradArgs a) {
 #pragma unroll
         for (int i = 0; i < SLABS; ++i) top = max(top, pm[i * 256]);
     }
-    float fwd, bk;
-    bad |= !scale_of(top, fwd, bk);
-    if (leads && (int)threadIdx.x < CP) a.cback[((second ? a.B : 0) + b) * 256 + c] = bk;
+    bad |= top >= 0x7f800000u;
+    const int fe = scale_exponent(__uint_as_float(top));
+    float fwd = power(fe);
+    if (leads && (int)threadIdx.x < CP) a.cback[((second ? a.B : 0) + b) * 256 + c] = -fe;
     if (second ? (blockIdx.x % a.H2) & 1 : (p0 / 16 / FLUSH) & 1) fwd = -fwd;   // (see block_sign)
     const unsigned least = top > (17u << 23) ? (top & 0x7f800000u) - (17u << 23) : 0;
     unsigned small = 0;
@@ -354,7 +376,7 @@ __global__ void __launch_bounds__(256) grad_split_kernel(const GradArgs a) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             small += magnitude(x[e]) - 1u < least - 1u && least > 0;
-            x[e] *= second ? fwd : back[p0 + 8 * g + e] * inv * fwd;
+            x[e] *= fwd;
         }
         v4u h, l;
 #pragma unroll
@@ -376,11 +398,12 @@ __global__ void __launch_bounds__(256) grad_split_kernel(const GradArgs a) {
 #endif
 
 // Finished 32 x 32 block of d_f1 (rows: pixels of image b) or d_f2 (rows: columns of row u of fmap2), accumulator layout.
+// (d_f1 may still carry the factors of its channel and pixels: SCALED)
 template <bool FIRST, bool SCALED>
 __device__ __forceinline__ void store_block(const GradArgs &a, int b, int u, int p0, int c0, const float (&x)[16]) {
     const int lane = threadIdx.x & 63, c = c0 + (lane & 31), h = lane >> 5;
     if (c >= a.C) return;
-    const float bk = SCALED ? a.cback[((FIRST ? a.B : 0) + b) * 256 + c] : 1.f;
+    const int ce = SCALED ? a.cback[(a.B + b) * 256 + c] : 0;
     const int n = FIRST ? a.N1 : a.W2, add = FIRST ? a.add1 : a.add2;
     float *dst = (FIRST ? a.d1 + (size_t)b * a.N1 * a.C : a.d2 + ((size_t)b * a.H2 + u) * a.W2 * a.C) + c;
     float old[16];
@@ -393,7 +416,7 @@ __device__ __forceinline__ void store_block(const GradArgs &a, int b, int u, int
     for (int r = 0; r < 16; ++r) {
         const int p = p0 + vmap(r, h);
         float y = x[r];
-        if constexpr (SCALED) y = y * bk * (FIRST ? a.back[(size_t)b * a.N1p + p] : a.top_back[b]);
+        if constexpr (SCALED) y = ldexpf(y, ce - exponent_of(a.pscale[(size_t)b * a.N1p + p]));
         if (p < n) dst[(size_t)p * a.C] = add ? old[r] + y : y;
     }
 }
@@ -522,7 +545,7 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) z[r] = x[r >> 2][r & 3];
     if constexpr (FIRST) store_block<true, true>(a, tile / npt, 0, TPX * (tile % npt) + 32 * row, 32 * cb, z);
-    else store_block<false, true>(a, bv / a.nvc, u, 32 * (bv % a.nvc), 32 * cb, z);
+    else store_block<false, false>(a, bv / a.nvc, u, 32 * (bv % a.nvc), 32 * cb, z);
 }
 
 // The 16-bit matrix instructions round their sums down, not to nearest: with every product of one sign convention the
@@ -532,12 +555,12 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
 __device__ __forceinline__ float block_sign(int odd) { return odd & 1 ? -1.f : 1.f; }
 
 // A piece's sums of a lane's block: what earlier flushes left of it in its slot (none if `first`), and x.
-__device__ __forceinline__ void sums_of_piece(const v4f *slot, bool first, const v16f &x, float sign, float (&y)[16]) {
+__device__ __forceinline__ void sums_of_piece(const v4f *slot, bool first, const float (&x)[16], float (&y)[16]) {
     v4f old[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) old[q] = first ? v4f{0.f, 0.f, 0.f, 0.f} : slot[q * 64];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) y[r] = fmaf(sign, x[r], old[r >> 2][r & 3]);
+    for (int r = 0; r < 16; ++r) y[r] = old[r >> 2][r & 3] + x[r];
 }
 __device__ __forceinline__ v4f *block_of(float *slot, int sub) { return reinterpret_cast<v4f *>(slot + sub * 1024) + (threadIdx.x & 63); }
 // Leaves them in the slot; a later flush of the same piece adds to it.
@@ -546,8 +569,8 @@ __device__ __forceinline__ void put_block(v4f *slot, const float (&y)[16]) {
     for (int q = 0; q < 4; ++q) slot[q * 64] = v4f{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
 }
 
-// dL/dS, scaled, of one column at the pixel whose u-indexed weights are wu; wv(f): its v-indexed weights, the max/average
-// ones scaled and as ma = max + average, mean = average.
+// dL/dS of one column at the pixel whose u-indexed weights are wu; wv(f): its v-indexed weights, the max/average ones as
+// ma = max + average, mean = average.
 template <bool BOTH, int KC, typename WV>
 __device__ __forceinline__ float gval(const float *wu, WV wv, int amu_rel, int col, int u, float ma, float mean, int amv) {
     float g = 0.f;
@@ -622,6 +645,7 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
         if (NB == 3) dma(ua + 1, 1);
         load_pu(ua);
         const int col0 = 32 * vc + 16 * sh + 8 * h;
+        const float sc = a.pscale[(size_t)b * a.N1p + pix];
         float wv[2 * KC][8];
         {
             v4f y[NF][2];
@@ -647,15 +671,15 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) wv[f][e] = y[f][e / 4][e % 4];
             if constexpr (BOTH) {   // kept in LDS: each thread reads its own again
-                const float sc = pn[(2 * KC + 3) / 4][(2 * KC + 3) % 4], inv_h2 = 1.f / (float)H2;
+                const float inv_h2 = 1.f / (float)H2;
 #pragma unroll
                 for (int q = 0; q < 2; ++q) {
                     v4f ma, mean;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
                         const float m = y[2 * KC + 1][q][e] * inv_h2;
-                        mean[e] = m * sc;
-                        ma[e] = (m + y[2 * KC][q][e]) * sc;
+                        mean[e] = m;
+                        ma[e] = m + y[2 * KC][q][e];
                     }
                     char *d = gbuf + 32768 + q * 24576 + tid * 16;
                     *reinterpret_cast<v4f *>(d) = ma;
@@ -687,7 +711,7 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     unsigned hh, ll;
-                    split2(x[2 * e], x[2 * e + 1], hh, ll);
+                    split2(x[2 * e], x[2 * e + 1], sc, sc, hh, ll);
                     hi[2 * q + e] = hh;
                     lo[2 * q + e] = ll;
                 }
@@ -780,9 +804,11 @@ __global__ void __launch_bounds__(512) split_d1_kernel(const GradArgs a) {
         for (int i = 0; i < MP; ++i)
 #pragma unroll
             for (int j = 0; j < MC; ++j) {
-                float y[16];
+                float x[16], y[16];
                 v4f *block = block_of(slot, (mp0 + i) * NCB + mc0 + j);
-                sums_of_piece(block, first, acc[i][j], 1.f, y);
+#pragma unroll
+                for (int r = 0; r < 16; ++r) x[r] = acc[i][j][r];
+                sums_of_piece(block, first, x, y);
                 if (out) store_block<true, true>(a, b, 0, TPX * pt + 32 * (mp0 + i), 32 * (mc0 + j), y);
                 else put_block(block, y);
             }
@@ -796,7 +822,7 @@ struct D2Shape {
     static constexpr int MC = NCB / 2;                                   // channel blocks of a wave (and two rows)
     static constexpr int FB = NCB * 2048, VB = vfields(BOTH, KC) * 2048; // a step's f1 and v-indexed weights
     static constexpr int RS = 72, GB = ROWS * 2 * 16 * RS;               // dL/dS: [row][half][16 pixels][32 columns]
-    static constexpr size_t LDS = 3 * (size_t)(FB + VB) + 2 * GB;
+    static constexpr size_t LDS = 3 * (size_t)(FB + VB) + 2 * GB + ROWS * 32 * 4;
 };
 
 // DIRECT: the v-indexed weights come into LDS from the tensors themselves (rows of a multiple of 4 floats, 16-byte aligned),
@@ -806,9 +832,10 @@ struct D2Shape {
 template <bool BOTH, int KC, int NCB, bool DIRECT>
 __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
     typedef D2Shape<BOTH, KC, NCB> S;
-    constexpr int NU = ufields(BOTH, KC), NF = vfields(BOTH, KC), MC = S::MC, FB = S::FB, VB = S::VB, RS = S::RS, GB = S::GB;
+    constexpr int NU = ufields(BOTH, KC), NF = vfields(BOTH, KC), NX = nbounds(BOTH), MC = S::MC, FB = S::FB, VB = S::VB, RS = S::RS, GB = S::GB;
     extern __shared__ char smem[];
     char *gbuf = smem + 3 * (FB + VB);
+    float *tq = reinterpret_cast<float *>(gbuf + 2 * GB);                // factors of the tile's positions, [row][column]
     if (unsuitable(a)) {
         contract_fp32<false, BOTH, KC>(a.self, reinterpret_cast<float *>(smem));
         return;
@@ -865,7 +892,8 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
             for (int i = 0; i < ND; ++i) {
                 const int kb = 8 * i + wave < 2 * (NCB + NF) ? 8 * i + wave : 2 * (NCB + NF) - 2 + (wave & 1);
                 const int at = max(0, min(kb < 2 * NCB ? t : t + 1, spt - 1));   // (past either end: not used, but read)
-                dma16(make_rsrc(reinterpret_cast<const void *>(src[i]), bytes[i]), smem + buf * (FB + VB) + kb * 1024, lane_off[i], off[i] + at * step[i]);
+                dma16(make_rsrc(reinterpret_cast<const void *>(src[i]), bytes[i]), smem + buf * (FB + VB) + kb * 1024, lane_off[i],
+                      __builtin_amdgcn_readfirstlane(off[i] + at * step[i]));
             }
         };
         const int p16 = lane & 15, vg = 4 * half + (lane >> 4), u0 = ROWS * ug + 2 * rp;
@@ -879,33 +907,41 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
                     pn[r][i] = *reinterpret_cast<const v4f *>(pu + ((size_t)r * a.N1p + 16 * min(t, spt - 1)) * NU + 4 * i);
         };
         // halves of dL/dS of this lane's pixel, four columns and two rows, from weight block buf into buffer gi
-        auto make_g = [&](int buf, int gi) __attribute__((always_inline)) {
+        auto load_tr = [&](v4f (&tr)[2]) __attribute__((always_inline)) {   // the factors of its positions
+#pragma unroll
+            for (int r = 0; r < 2; ++r) tr[r] = *reinterpret_cast<const v4f *>(tq + (2 * rp + r) * 32 + 4 * vg);
+        };
+        // (tr: its factors, read first: the compiler waits for everything else before it when it is read where it is needed)
+        auto make_g = [&](int buf, int gi, const v4f (&tr)[2]) __attribute__((always_inline)) {
             const char *wb = smem + buf * (FB + VB) + FB + (vg * 16 + p16) * 16;
             v4f m[NF], ma = {0.f, 0.f, 0.f, 0.f}, mean = ma, am = ma;
 #pragma unroll
             for (int f = 0; f < NF; ++f) m[f] = *reinterpret_cast<const v4f *>(wb + f * 2048);
             if constexpr (BOTH) {
-                const float sc = pn[0][(2 * KC + 3) / 4][(2 * KC + 3) % 4], si = sc * inv_h2;
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    mean[e] = m[2 * KC + 1][e] * si;
-                    ma[e] = fmaf(m[2 * KC][e], sc, mean[e]);
+                    mean[e] = m[2 * KC + 1][e] * inv_h2;
+                    ma[e] = m[2 * KC][e] + mean[e];
                 }
                 am = m[2 * KC + 2];
             }
+            float x[2][4];
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
-                float wu[NU], x[4];
+                float wu[NU];
 #pragma unroll
                 for (int i = 0; i < NU; ++i) wu[i] = pn[r][i / 4][i % 4];
                 const int rel = BOTH ? __float_as_int(wu[BOTH ? 2 * KC + 2 : 0]) - (32 * vc + 4 * vg) : 0;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) x[e] = gval<BOTH, KC>(wu, [&](int f) { return m[f][e]; }, rel, e, u0 + r, ma[e], mean[e], __float_as_int(am[e]));
+                for (int e = 0; e < 4; ++e) x[r][e] = gval<BOTH, KC>(wu, [&](int f) { return m[f][e]; }, rel, e, u0 + r, ma[e], mean[e], __float_as_int(am[e]));
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
                 v2u hi, lo;
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     unsigned hh, ll;
-                    split2(x[2 * e], x[2 * e + 1], hh, ll);
+                    split2(x[r][2 * e], x[r][2 * e + 1], tr[r][2 * e], tr[r][2 * e + 1], hh, ll);
                     hi[e] = hh;
                     lo[e] = ll;
                 }
@@ -925,8 +961,43 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
         dma(ta - 1, 2);   // (for the weights; of f1 the step before, or nothing)
         dma(ta, 0);
         dma(ta + 1, 1);
+        {   // factors of the tile's positions for these steps: eight waves take every eighth block of 16 pixels
+            const float *bx = a.bound_v + ((size_t)b * a.nvc + vc) * (a.N1p / 16) * NX * 32 + 4 * (lane & 7);
+            const float *by = a.bound_u + (size_t)b * (a.N1p / 16) * NX * a.H2p + ROWS * ug + (lane >> 3);
+            v4f top = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < FLUSH / 8; ++i) {
+                const int t = min(ta + 8 * i + wave, tb - 1);
+                v4f x[NX];
+                float y[NX];
+#pragma unroll
+                for (int n = 0; n < NX; ++n) {
+                    x[n] = *reinterpret_cast<const v4f *>(bx + ((size_t)t * NX + n) * 32);
+                    y[n] = by[((size_t)t * NX + n) * a.H2p];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float m = fminf(x[0][e], y[0]) + fminf(x[1][e], y[1]);
+                    if constexpr (BOTH) m += x[NX - 1][e] + y[NX - 1];
+                    top[e] = fmaxf(top[e], m);
+                }
+            }
+            float *red = reinterpret_cast<float *>(gbuf);   // [wave][row][column]
+            *reinterpret_cast<v4f *>(red + wave * 256 + lane * 4) = top;
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            if (tid < 256) {
+                float m = 0.f;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) m = fmaxf(m, red[i * 256 + tid]);
+                tq[tid] = power(scale_exponent(m));
+            }
+        }
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * ND) : "memory");
-        make_g(2, 0);
+        {
+            v4f tr[2];
+            load_tr(tr);
+            make_g(2, 0, tr);
+        }
         load_pu(ta + 1);
         // (the builtin: the compiler then knows that nothing is outstanding, and waits for no requests in the loop)
         __builtin_amdgcn_s_waitcnt(0x0F70);
@@ -936,16 +1007,19 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
         for (int t = ta; t < tb; ++t) {
             const int gi = (t - ta) & 1, far = buf == 0 ? 2 : buf - 1;
             const char *fb = smem + buf * (FB + VB) + half * MC * 2048 + lane * 16;
-            v8h F[MC][2];
+            v4f tr[2];
+            load_tr(tr);
+            __builtin_amdgcn_sched_barrier(0);
+            make_g(buf, gi ^ 1, tr);
+            load_pu(t + 2);
+            __builtin_amdgcn_sched_barrier(0);
+            dma(t + 2, far);
+            __builtin_amdgcn_sched_barrier(0);
+            v8h F[MC][2];   // (not before: there are not the registers to have them while dL/dS is formed)
 #pragma unroll
             for (int j = 0; j < MC; ++j)
 #pragma unroll
                 for (int q = 0; q < 2; ++q) F[j][q] = *reinterpret_cast<const v8h *>(fb + j * 2048 + q * 1024);
-            __builtin_amdgcn_sched_barrier(0);
-            make_g(buf, gi ^ 1);
-            load_pu(t + 2);
-            __builtin_amdgcn_sched_barrier(0);
-            dma(t + 2, far);
             __builtin_amdgcn_sched_barrier(0);
             // lane 16 (2 h + w) + 4 r + q asks for columns 16 w + 4 q.. of pixel 8 h + r and gets column 16 w + 4 r + q of four pixels
             const char *gb = gbuf + gi * GB + (8 * h + ((lane >> 2) & 3)) * RS + ((lane >> 4) & 1) * 32 + (lane & 3) * 8 + 2 * rp * 2 * 16 * RS;
@@ -990,11 +1064,18 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
         for (int r = 0; r < 2; ++r)
 #pragma unroll
             for (int j = 0; j < MC; ++j) {
-                float y[16];
+                float x[16], y[16];
                 v4f *block = block_of(slot, (2 * rp + r) * NCB + half * MC + j);
-                sums_of_piece(block, first, acc[r][j], block_sign(ta / FLUSH), y);
+                const int ce = a.cback[b * 256 + 32 * (half * MC + j) + (lane & 31)];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const v4f t = *reinterpret_cast<const v4f *>(tq + (2 * rp + r) * 32 + 8 * q + 4 * h);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[4 * q + e] = ldexpf(block_sign(ta / FLUSH) * acc[r][j][4 * q + e], ce - exponent_of(t[e]));
+                }
+                sums_of_piece(block, first, x, y);
                 if (!out) put_block(block, y);
-                else if (u0 + r < a.H2) store_block<false, true>(a, b, u0 + r, 32 * vc, 32 * (half * MC + j), y);
+                else if (u0 + r < a.H2) store_block<false, false>(a, b, u0 + r, 32 * vc, 32 * (half * MC + j), y);
             }
         first = ends;
     }
@@ -1075,8 +1156,8 @@ constexpr int kPlaces = 256;   // compute units
 struct GradPlan {
     bool ok, direct;
     int ncb, nvc, H2p, N1p, npx, G1, G2;
-    size_t pv, pu, back, block_back, top_back, pmax, cback, f1h, f2h, slots;
-    size_t bytes() const { return pv + pu + back + block_back + top_back + pmax + cback + f1h + f2h + slots + 1024; }
+    size_t pv, pu, pscale, block_bad, bound_v, bound_u, pmax, cback, f1h, f2h, slots;
+    size_t bytes() const { return pv + pu + pscale + block_bad + bound_v + bound_u + pmax + cback + f1h + f2h + slots + 1024; }
 };
 size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 
@@ -1100,9 +1181,10 @@ GradPlan plan(int B, int N1, int H2, int W2, int C, int both, int kc, int KT, bo
     p.G2 = (int)(T2 < kPlaces ? T2 : kPlaces);
     p.pv = p.direct ? 0 : align256((size_t)B * p.nvc * (p.N1p / 16) * nf * 2048);
     p.pu = align256((size_t)B * p.H2p * p.N1p * ufields(both, kc) * 4);
-    p.back = align256((size_t)B * p.N1p * 4);
-    p.block_back = align256((size_t)B * (p.N1p / 16) * 4);
-    p.top_back = align256((size_t)B * 4);
+    p.pscale = align256((size_t)B * p.N1p * 4);
+    p.block_bad = align256((size_t)B * (p.N1p / 16) * 4);
+    p.bound_v = align256((size_t)B * p.nvc * (p.N1p / 16) * nbounds(both) * 128);
+    p.bound_u = align256((size_t)B * (p.N1p / 16) * nbounds(both) * p.H2p * 4);
     p.pmax = align256((size_t)2 * B * SLABS * 256 * 4);
     p.cback = align256((size_t)2 * B * 256 * 4);
     p.f1h = align256((size_t)B * p.npx * p.ncb * 2048);
@@ -1137,11 +1219,12 @@ int split_grad(int both, int kc, GradArgs a, void *ws, size_t ws_bytes, hipStrea
     a.slots = reinterpret_cast<float *>(take(p.slots));
     a.pv = reinterpret_cast<float *>(take(p.pv));
     a.pu = reinterpret_cast<float *>(take(p.pu));
-    a.back = reinterpret_cast<float *>(take(p.back));
-    a.block_back = reinterpret_cast<float *>(take(p.block_back));
-    a.top_back = reinterpret_cast<float *>(take(p.top_back));
+    a.pscale = reinterpret_cast<float *>(take(p.pscale));
+    a.block_bad = reinterpret_cast<int *>(take(p.block_bad));
+    a.bound_v = reinterpret_cast<float *>(take(p.bound_v));
+    a.bound_u = reinterpret_cast<float *>(take(p.bound_u));
     a.pmax = reinterpret_cast<unsigned *>(take(p.pmax));
-    a.cback = reinterpret_cast<float *>(take(p.cback));
+    a.cback = reinterpret_cast<int *>(take(p.cback));
     a.f1h = take(p.f1h);
     a.f2h = take(p.f2h);
     a.count = reinterpret_cast<unsigned *>(take(256));

@@ -118,6 +118,47 @@ def test_against_float64(device, dims, K, both):
         assert torch.equal(added, base + got[0]) if K <= 4 else _rel(added, base.double() + got[0]) < 1e-6
 
 
+@pytest.mark.parametrize("both", [False, True], ids=["compression", "combined"])
+@pytest.mark.parametrize("what", ["avoided 12", "avoided 40", "one loud pixel", "small at random", "peaks", "masked", "tiny"])
+def test_every_row_by_itself(device, what, both):
+    """Rows of d_f2 that all attention avoids, or that only pixels with small gradients reach, and rows of d_f1 of such pixels."""
+    B, H1, W1, H2, W2, C = dims = (1, 40, 53, 37, 56, 128)
+    x = _tensors(device, dims, 3, seed=5)
+    g = torch.Generator(device=device).manual_seed(6)
+    zu, zv = (torch.randn(x[k].shape, generator=g, device=device) for k in ("a_u", "a_v"))
+    size = torch.ones(B, H1, W1, 1, 1, device=device)
+    if "avoided" in what:   # the last columns and rows
+        zu[..., W2 // 2 + 1:] -= float(what.split()[1])
+        zv[..., H2 // 2 + 1:] -= float(what.split()[1])
+    else:                   # every pixel looks at its own place
+        j, v = torch.arange(W1, device=device), torch.arange(W2, device=device)
+        i, u = torch.arange(H1, device=device), torch.arange(H2, device=device)
+        zu -= 5 * (v - j.clamp(max=W2 - 1)[:, None]).abs().clamp(max=4).view(1, 1, W1, 1, W2)
+        zv -= 5 * (u - i.clamp(max=H2 - 1)[:, None]).abs().clamp(max=4).view(1, H1, 1, 1, H2)
+    if what == "one loud pixel":   # (one product of dL/dS: a sum of several may cancel, and rows that have this pixel's alone show it)
+        size[0, 11, 17] = 2.0 ** 40
+        x["g_cu"][0, 11, 17, 1:] = 0
+        x["g_cv"][0, 11, 17] = 0
+    if what == "small at random": size = torch.exp2(-torch.randint(0, 41, size.shape, generator=g, device=device))
+    if what == "masked":
+        size[:, :13] = 0
+        size[:, 20:, 9] = 2.0 ** -30
+    if what == "tiny":
+        size *= 2.0 ** -80
+        x["f1"] *= 2.0 ** -20
+    x["a_u"], x["a_v"] = zu.softmax(-1), zv.softmax(-1)
+    for k in ("g_cu", "g_cv"): x[k] *= size
+    for k in ("g_u", "g_v"): x[k] *= size * 2.0 ** -60   # (the rest of dL/dS is not to be covered by the averages)
+    got = []
+    kind = "both" if both else "comp"
+    assert {f"df1_{kind}_split", f"df2_{kind}_split"} <= _labels_of(lambda: got.extend(_run(x, both)))
+    ref = _exact(x, both)
+    for a, r in zip(got, ref):
+        # Halves hold 22 bits, the products of two low ones are left out: 3 2^-23 of a product at the most, 0.7e-7 in the mean, and
+        # fp32 sums on top; up to 2.5e-7 of a row's length were seen, up to 3.1e-7 from the fp32 kernels.
+        assert bool(((a.double() - r).norm(dim=-1) <= 6e-7 * r.norm(dim=-1)).all())
+
+
 def test_sums_are_not_biased(device):
     """The 16-bit matrix instructions round down; the signs turned in every other row keep that out of the mean."""
     x = _tensors(device, (1, 16, 64, 136, 240, 256), 2)
