@@ -421,96 +421,9 @@ __device__ __forceinline__ void store_block(const GradArgs &a, int b, int u, int
     }
 }
 
-// The contraction in fp32 straight from the inputs, for operands that have no halves.  A workgroup of
-// eight waves owns 32 pixels (FIRST), or 32 columns of a row, with all channels; dL/dS is formed 32 x 32 at a time in LDS, a register sum takes 128 products.
-// (A function of its own, its arguments in memory: with a copy on the stack the kernels don't keep theirs in registers.)
-template <bool FIRST, bool BOTH, int KC>
-__device__ __attribute__((noinline)) void contract_fp32(const GradArgs *args, float *lds) {
-    const GradArgs a = *args;
-    constexpr int NF = vfields(BOTH, KC);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, pl = lane & 31, h = lane >> 5;
-    const int gp = tid >> 3 & 31, gv = 4 * (tid & 7), cb = wave;          // dL/dS: this thread's pixel and four columns
-    const int N1 = a.N1, H2 = a.H2, W2 = a.W2, C = a.C, nb = (N1 + 31) / 32;
-    const float inv_w2 = 1.f / (float)W2, inv_h2 = 1.f / (float)H2;
-    const int tasks = FIRST ? a.B * nb : a.B * a.nvc * H2;
-    for (int task = blockIdx.x; task < tasks; task += gridDim.x) {
-        const int b = FIRST ? task / nb : task / (a.nvc * H2), pb = FIRST ? task - b * nb : 0;
-        const int vc0 = FIRST ? 0 : task / H2 % a.nvc, u0 = FIRST ? 0 : task % H2;
-        v16f sum = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-        const int c = 32 * cb + pl;
-        const int outer = FIRST ? a.nvc : 1, inner = FIRST ? H2 : nb;
-        for (int o = 0; o < outer; ++o) {
-            const int vc = FIRST ? o : vc0;
-            v4f w[NF];
-            v16f acc = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            for (int i = 0; i < inner; ++i) {
-                const int u = FIRST ? i : u0, p = 32 * (FIRST ? pb : i) + gp;
-                const bool pok = p < N1;
-                const size_t bp = (size_t)b * N1 + (pok ? p : 0);
-                if (!FIRST || i == 0) {
-#pragma unroll
-                    for (int f = 0; f < NF; ++f) w[f] = columns4(vrow<KC>(a, f, bp), 32 * vc + gv, W2, pok);
-                }
-                float gu[KC], av[KC], mx = 0.f, mean = 0.f;
-                int am = -1;
-#pragma unroll
-                for (int k = 0; k < KC; ++k) {
-                    gu[k] = a.g_cu[(bp * a.KT + a.k0 + k) * H2 + u];
-                    av[k] = a.a_v[(bp * a.KT + a.k0 + k) * H2 + u];
-                }
-                if constexpr (BOTH) {
-                    mean = a.g_u[(2 * bp + 1) * H2 + u] * inv_w2;
-                    mx = a.g_u[2 * bp * H2 + u] + mean;
-                    am = a.am_u[bp * H2 + u];
-                }
-                float *g = lds + (i & 1) * 32 * 36;                   // [pixel][36]
-                v4f x;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    float y = 0.f;
-                    if constexpr (BOTH) {
-                        const float m = w[2 * KC + 1][e] * inv_h2;
-                        y = (am == 32 * vc + gv + e ? mx : mean) + (__float_as_int(w[2 * KC + 2][e]) == u ? m + w[2 * KC][e] : m);
-                    }
-#pragma unroll
-                    for (int k = 0; k < KC; ++k) {
-                        y = fmaf(w[k][e], gu[k], y);
-                        y = fmaf(av[k], w[KC + k][e], y);
-                    }
-                    x[e] = pok && 32 * vc + gv + e < W2 ? y : 0.f;
-                }
-                if (tid < 256) *reinterpret_cast<v4f *>(g + gp * 36 + gv) = x;
-                __syncthreads();
-                if (cb < a.ncb) {
-                    const int n = FIRST ? W2 - 32 * vc : N1 - 32 * i;   // rows of the other operand there are
-                    const float *src = FIRST ? a.f2 + (((size_t)b * H2 + u) * W2 + 32 * vc) * C : a.f1 + ((size_t)b * N1 + 32 * i) * C;
-                    float f[16];
-#pragma unroll
-                    for (int s = 0; s < 16; ++s) f[s] = c < C && 2 * s + h < n ? src[(size_t)(2 * s + h) * C + c] : 0.f;
-#pragma unroll
-                    for (int s = 0; s < 16; ++s)
-                        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(FIRST ? g[pl * 36 + 2 * s + h] : g[(2 * s + h) * 36 + pl], f[s], acc, 0, 0, 0);
-                    if ((i & 3) == 3 || i == inner - 1) {
-                        sum += acc;
-                        acc = v16f{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-                    }
-                }
-            }
-            __syncthreads();
-        }
-        if (cb < a.ncb) {
-            float z[16];
-#pragma unroll
-            for (int r = 0; r < 16; ++r) z[r] = sum[r];
-            store_block<FIRST, false>(a, b, u0, FIRST ? 32 * pb : 32 * vc0, 32 * cb, z);
-        }
-    }
-}
-
 // Adds up what the pieces of a tile left in their slots, in the order of their steps.  One wave per 32 x 32 block.
 template <bool FIRST, bool BOTH, int KC>
 __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
-    if (unsuitable(a)) return;   // (the contraction has written the results)
     const int ncb = a.ncb, per = (FIRST ? 4 : ROWS) * ncb, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
     const int unit = blockIdx.x * 4 + wave, tile = unit / per, sub = unit - tile * per, cb = sub % ncb, row = sub / ncb;
     const int nug = a.H2p / ROWS, npt = a.N1p / TPX;
@@ -544,7 +457,9 @@ __global__ void __launch_bounds__(256) grad_finish_kernel(const GradArgs a) {
     float z[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) z[r] = x[r >> 2][r & 3];
-    if constexpr (FIRST) store_block<true, true>(a, tile / npt, 0, TPX * (tile % npt) + 32 * row, 32 * cb, z);
+    const bool scaled = FIRST && !unsuitable(a);
+    if (scaled) store_block<true, true>(a, tile / npt, 0, TPX * (tile % npt) + 32 * row, 32 * cb, z);
+    else if (FIRST) store_block<true, false>(a, tile / npt, 0, TPX * (tile % npt) + 32 * row, 32 * cb, z);
     else store_block<false, false>(a, bv / a.nvc, u, 32 * (bv % a.nvc), 32 * cb, z);
 }
 
@@ -567,6 +482,157 @@ __device__ __forceinline__ v4f *block_of(float *slot, int sub) { return reinterp
 __device__ __forceinline__ void put_block(v4f *slot, const float (&y)[16]) {
 #pragma unroll
     for (int q = 0; q < 4; ++q) slot[q * 64] = v4f{y[4 * q], y[4 * q + 1], y[4 * q + 2], y[4 * q + 3]};
+}
+
+// The contraction in fp32 straight from the inputs, for operands that have no halves: the same tiles, pieces and slots.  A
+// workgroup goes through its steps of a tile for 64 of the pixels (FIRST) or two of the rows at a time: a wave has both
+// blocks of 32 of them for 32 channels, or, with 128 channels and fewer, one.  dL/dS is formed in LDS, 32 columns and pixels
+// of each block, while the features and weights of the next step are on their way; a register sum takes 128 products.
+// Call of the compression's backward with one NaN in it, the fp32 kernels of sepcorr.hip -> here: B=2, 55x128, C=256, K=4 1172 -> 1693
+// us; B=4, 48x64 503 -> 708; B=2, 47x61, C=100, K=2 221 -> 275; 55x128 on 27x64 234 -> 347.  (Tasks of 32 pixels or columns of a
+// workgroup's own, nothing on its way: 3414, 1472, 430, 1263; half of the waves forming the next dL/dS while the others multiply: 1628,
+// 706, 300, 351; four rows at a time: 1722, 733, 265, 353, the combined call 1.2 times as long.)
+// (A function of its own, its arguments in memory: with a copy on the stack the kernels don't keep theirs in registers.)
+template <bool FIRST, bool BOTH, int KC>
+__device__ __attribute__((noinline)) void contract_fp32(const GradArgs *args, float *lds) {
+    // (the arguments of a function are a lane's own, and what is loaded through them may lie anywhere: told here that they are not)
+    typedef const __attribute__((address_space(1))) float *Floats;
+    typedef v4f __attribute__((aligned(4))) u4f;
+    GradArgs a;
+    {
+        const uint64_t at = reinterpret_cast<uint64_t>(args);
+        const uint64_t lo = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)at), hi = (unsigned)__builtin_amdgcn_readfirstlane((int)(unsigned)(at >> 32));
+        const __attribute__((address_space(4))) unsigned *words = reinterpret_cast<const __attribute__((address_space(4))) unsigned *>((hi << 32) | lo);
+        unsigned copy[sizeof(a) / 4];
+#pragma unroll
+        for (int i = 0; i < (int)(sizeof(a) / 4); ++i) copy[i] = words[i];
+        __builtin_memcpy(&a, copy, sizeof(a));
+    }
+    constexpr int NF = vfields(BOTH, KC), GP = 36, GBLK = 32 * GP;        // floats of a pixel's row of dL/dS, of a block of it
+    const int tid = threadIdx.x, lane = tid & 63, pl = lane & 31, h = lane >> 5, ncb = a.ncb;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), cb = wave % ncb, part = wave / ncb;
+    const int gb = tid >> 8, gp = tid >> 3 & 31, gv = 4 * (tid & 7);      // dL/dS: this thread's block, pixel and four columns
+    const int N1 = a.N1, H2 = a.H2, W2 = a.W2, C = a.C;
+    const unsigned lane_off = 32 * cb + pl < C ? (unsigned)(16 * h * C + 32 * cb + pl) * 4 : OOB;
+    const int npt = a.N1p / TPX, nug = a.H2p / ROWS, tiles = FIRST ? a.B * npt : a.B * nug * a.nvc;
+    const int spt = FIRST ? a.nvc * H2 : a.npx, G = FIRST ? a.G1 : a.G2, wg = xcd_contiguous(blockIdx.x, gridDim.x);
+    const long T = (long)tiles * spt;
+    const int g0 = (int)first_step(wg, G, T), g1 = (int)first_step(wg + 1, G, T);
+    const float inv_w2 = 1.f / (float)W2, inv_h2 = 1.f / (float)H2;
+    const v16f zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int g = g0; g < g1;) {
+        const int tile = g / spt, bv = FIRST ? 0 : tile / nug, b = FIRST ? tile / npt : bv / a.nvc;
+        const Piece piece = piece_of(tile, g0, g1, spt);
+        g = tile * spt + piece.end;
+        const int p_end = FIRST ? N1 : min(N1, 16 * piece.end);           // pixels that are not this piece's count as none
+        const int steps = FIRST ? piece.end - piece.begin : (piece.end - piece.begin + 1) / 2;
+        for (int pair = 0; pair < (FIRST ? 2 : 4); ++pair) {              // of the tile's blocks of 32 pixels, or of its rows
+            const int p0 = FIRST ? TPX * (tile % npt) + 64 * pair : 0, u0 = FIRST ? 0 : ROWS * (tile % nug) + 2 * pair;
+            if (FIRST ? p0 >= N1 : u0 >= H2) break;
+            v4f w[NF];
+            float gu[KC], av[KC], mx = 0.f, mean = 0.f, fn[16];
+            int am = -1;
+            // weights of this thread's pixel, and features, of a step: column chunk vc and row u (FIRST), 32 pixels from p on
+            // (those past an end are others', and not used)
+            auto load = [&](int vc, int u, int p, bool all) __attribute__((always_inline)) {
+                const size_t bp = (size_t)b * N1 + min(p + gp, N1 - 1);
+                const int row = min(u, H2 - 1), v = 32 * vc + gv;
+                if (!FIRST || all) {
+                    if (32 * vc + 32 <= W2) {
+#pragma unroll
+                        for (int f = 0; f < NF; ++f) w[f] = *(const __attribute__((address_space(1))) u4f *)((Floats)vrow<KC>(a, f, bp) + v);
+                    } else {
+#pragma unroll
+                        for (int f = 0; f < NF; ++f)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) w[f][e] = ((Floats)vrow<KC>(a, f, bp))[min(v + e, W2 - 1)];
+                    }
+                }
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    gu[k] = ((Floats)a.g_cu)[(bp * a.KT + a.k0 + k) * H2 + row];
+                    av[k] = ((Floats)a.a_v)[(bp * a.KT + a.k0 + k) * H2 + row];
+                }
+                if constexpr (BOTH) {
+                    mean = ((Floats)a.g_u)[(2 * bp + 1) * H2 + row];
+                    mx = ((Floats)a.g_u)[2 * bp * H2 + row];
+                    am = __float_as_int(((Floats)a.am_u)[bp * H2 + row]);
+                }
+                const float *src = FIRST ? a.f2 + (((size_t)b * H2 + u) * W2 + 32 * vc) * C : a.f1 + ((size_t)b * N1 + p) * C;
+                const int n = min(32, FIRST ? W2 - 32 * vc : p_end - p);  // rows of the other operand there are: zeros behind them
+                const __amdgpu_buffer_rsrc_t rs = make_rsrc(src, (unsigned)(n * C) * 4);
+#pragma unroll
+                for (int s = 0; s < 16; ++s) fn[s] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs, lane_off + (unsigned)(s * C * 4), 0, 0));
+            };
+            v16f sum[2] = {zero, zero}, acc[2] = {zero, zero};
+            int vc = FIRST ? piece.begin / H2 : bv % a.nvc, u = FIRST ? piece.begin - vc * H2 : u0 + gb, p = FIRST ? p0 + 32 * gb : 16 * piece.begin;
+            load(vc, u, p, true);
+            for (int i = 0; i < steps; ++i) {
+                float *gl = lds + (i & 1) * 2 * GBLK;                     // [block][pixel][36]
+                float f[16];
+#pragma unroll
+                for (int s = 0; s < 16; ++s) f[s] = fn[s];
+                v4f x;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float y = 0.f;
+                    if constexpr (BOTH) {
+                        const float m = w[2 * KC + 1][e] * inv_h2, mu = mean * inv_w2;
+                        y = (am == 32 * vc + gv + e ? mx + mu : mu) + (__float_as_int(w[2 * KC + 2][e]) == u ? m + w[2 * KC][e] : m);
+                    }
+#pragma unroll
+                    for (int k = 0; k < KC; ++k) {
+                        y = fmaf(w[k][e], gu[k], y);
+                        y = fmaf(av[k], w[KC + k][e], y);
+                    }
+                    x[e] = p + gp < p_end && 32 * vc + gv + e < W2 ? y : 0.f;
+                }
+                *reinterpret_cast<v4f *>(gl + gb * GBLK + gp * GP + gv) = x;
+                __syncthreads();
+                if constexpr (FIRST) {
+                    if (++u == H2) u = 0, ++vc;
+                } else p += 32;
+                if (i + 1 < steps) load(vc, u, p, u == 0);
+                // (the contraction's index runs 16 h + s, so that a lane's part of a pixel's row lies together)
+#pragma unroll
+                for (int m = 0; m < 2; ++m) {
+                    if (ncb == 8 || m == part) {
+                        const float *gm = gl + m * GBLK;
+                        float y[16];
+                        if constexpr (FIRST) {
+#pragma unroll
+                            for (int q = 0; q < 4; ++q) {
+                                const v4f z = *reinterpret_cast<const v4f *>(gm + pl * GP + 16 * h + 4 * q);
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) y[4 * q + e] = z[e];
+                            }
+                        } else {
+#pragma unroll
+                            for (int s = 0; s < 16; ++s) y[s] = gm[(16 * h + s) * GP + pl];
+                        }
+#pragma unroll
+                        for (int s = 0; s < 16; ++s) acc[m] = __builtin_amdgcn_mfma_f32_32x32x2f32(y[s], f[s], acc[m], 0, 0, 0);
+                        if ((i & 3) == 3 || i == steps - 1) {
+                            sum[m] += acc[m];
+                            acc[m] = zero;
+                        }
+                    }
+                }
+            }
+            __syncthreads();
+            float *slot = a.slots + (size_t)slot_of(wg, tile, piece.begin > 0, tiles, G) * (FIRST ? 4 : ROWS) * ncb * 1024;
+#pragma unroll
+            for (int m = 0; m < 2; ++m) {
+                if (ncb == 8 || m == part) {
+                    float z[16];
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) z[r] = sum[m][r];
+                    if (!piece.whole(spt)) put_block(block_of(slot, (2 * pair + m) * ncb + cb), z);
+                    else if (FIRST || u0 + m < H2) store_block<FIRST, false>(a, b, u0 + m, FIRST ? p0 + 32 * m : 32 * (bv % a.nvc), 32 * cb, z);
+                }
+            }
+        }
+    }
 }
 
 // dL/dS of one column at the pixel whose u-indexed weights are wu; wv(f): its v-indexed weights, the max/average ones as

@@ -192,6 +192,21 @@ def test_operands_without_halves(device, what, both):
             assert float((a - b)[fin].double().norm()) <= 2e-6 * float(b[fin].double().norm())
 
 
+@pytest.mark.parametrize("both", [False, True], ids=["compression", "combined"])
+@pytest.mark.parametrize("dims,K", SHAPES + MANY_TILES, ids=str)
+def test_fp32_contraction_against_float64(device, dims, K, both):
+    x = _tensors(device, dims, K, seed=K)
+    x["f2"][..., 0] *= 2.0 ** -20   # (a channel of small values beside one large one: more than one feature in 2048)
+    x["f2"][:, 0, 0, 0] = 1
+    got, ref = _run(x, both), _exact(x, both)
+    # fp32 products, 128 of them in a register sum and up to a hundred such sums in another, dL/dS itself a sum of up to 15 fp32
+    # terms: each rounding is 2^-25 of its sum in the mean, of a random walk of n terms about (n / 3)^0.5 of that in all, 2e-7 for
+    # both sums together; 1.3e-7 to 2.7e-7 were seen
+    assert _rel(got[0], ref[0]) < 4e-7 and _rel(got[1], ref[1]) < 4e-7
+    again = _run(x, both)
+    assert torch.equal(got[0], again[0]) and torch.equal(got[1], again[1])
+
+
 def test_scratch_and_alignment(device):
     """Less scratch than the query gives, and weights at addresses that are no multiple of 16: the same gradients."""
     dims, K = (2, 24, 49, 27, 52, 256), 2
