@@ -60,6 +60,11 @@ SIGNATURES = {
     "sepcorr_lookup1d_backward": (_I, [_P] * 3 + [_I] * 9 + [_P]),
 }
 
+# what this package calls besides (csrc/sepcorr_internal.h)
+INTERNAL = {
+    "sepcorr_backward_workspace_bytes_for": (_SZ, [_I] * 8),
+}
+
 _lib = None
 
 
@@ -72,7 +77,7 @@ def load():
                 f"{LIB_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}` "
                 "(or __graft_entry__.build()); there is no CPU fallback for this operator")
         lib = ctypes.CDLL(LIB_PATH)
-        for name, (res, args) in SIGNATURES.items():
+        for name, (res, args) in {**SIGNATURES, **INTERNAL}.items():
             fn = getattr(lib, name)  # AttributeError if the library does not export it
             fn.restype = res
             fn.argtypes = args

@@ -4091,30 +4091,40 @@ int maxavg_backward(const Dims &d, bool gather, const float *f1, const float *f2
     return launch_bwd<GMODE_MAXAVG, 1>(a, d, ws, s1, s);
 }
 
-// Whether the feature gradients of a call with this workspace come from the contractions of split_grad.hip.
-bool split_gradients(const Dims &d, const BwdWs &lay, bool both, size_t ws_bytes) {
+// Scratch the contractions of split_grad.hip are given in a call with these feature gradients, 0 where they do not run.
+size_t split_gradients_bytes(const Dims &d, bool both) {
     const double size = (double)d.B * d.H1 * d.W1 * d.H2 * d.W2 * (d.C + 64);
-    return split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C) > 0 && size >= (both ? SPLIT_GRAD_LINE : SPLIT_GRAD_LINE_ALONE) &&
-           ws_bytes >= lay.full && g_contraction.load(std::memory_order_relaxed) == SEPCORR_CONTRACT_SPLIT;
+    if (size < (both ? SPLIT_GRAD_LINE : SPLIT_GRAD_LINE_ALONE) || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 0;
+    return split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C);
+}
+
+GradArgs grad_args(const Dims &d, const BwdArgs &a, int K, int k0) {
+    GradArgs g;
+    memset(&g, 0, sizeof(g));
+    g.f1 = a.f1; g.f2 = a.f2; g.a_u = a.a_u; g.a_v = a.a_v; g.g_cu = a.g_cu; g.g_cv = a.g_cv;
+    g.am_u = a.am_u; g.am_v = a.am_v; g.g_u = a.g_u; g.g_v = a.g_v;
+    g.d1 = a.d1; g.d2 = a.d2;
+    g.B = d.B; g.N1 = a.N1; g.H2 = d.H2; g.W2 = d.W2; g.C = d.C; g.KT = K; g.k0 = k0;
+    g.add1 = a.add_d1 || k0 > 0;
+    g.add2 = k0 > 0;
+    return g;
+}
+
+// Whether the feature gradients of a call with this workspace come from them.  (Weights at odd addresses take more scratch.)
+bool split_gradients(const Dims &d, const BwdArgs &a, bool both, int K, size_t ws_bytes) {
+    const size_t n = split_gradients_bytes(d, both);
+    if (n == 0 || ws_bytes < n) return false;
+    for (int k0 = 0; k0 < K; k0 += KCH)
+        if (!split_grad_fits(both && k0 == 0, std::min(K - k0, KCH), grad_args(d, a, K, k0), ws_bytes)) return false;
+    return true;
 }
 
 // d_f1 and d_f2 of the compression (`both`: with the max/average terms) of K weight channels, the tensors as `a` names
 // them: d_f1 on stream s1, d_f2 on s (split: one stream).
 int feature_gradients(const Dims &d, BwdArgs a, bool both, int K, bool split, void *ws, size_t ws_bytes, hipStream_t s1, hipStream_t s) {
     a.KT = K;
-    for (int k0 = 0; split && k0 < K; k0 += KCH) {
-        GradArgs g;
-        memset(&g, 0, sizeof(g));
-        g.f1 = a.f1; g.f2 = a.f2; g.a_u = a.a_u; g.a_v = a.a_v; g.g_cu = a.g_cu; g.g_cv = a.g_cv;
-        g.am_u = a.am_u; g.am_v = a.am_v; g.g_u = a.g_u; g.g_v = a.g_v;
-        g.d1 = a.d1; g.d2 = a.d2;
-        g.B = d.B; g.N1 = a.N1; g.H2 = d.H2; g.W2 = d.W2; g.C = d.C; g.KT = K; g.k0 = k0;
-        g.add1 = a.add_d1 || k0 > 0;
-        g.add2 = k0 > 0;
-        const int rc = split_grad(both && k0 == 0, std::min(K - k0, KCH), g, ws, ws_bytes, s);
-        if (rc == 1 && k0 == 0) split = false;   // (weights at odd addresses take more scratch)
-        else if (rc) return rc < 0 ? rc : fail(SEPCORR_EWORKSPACE, "sepcorr: feature gradients: scratch does not suffice");
-    }
+    for (int k0 = 0; split && k0 < K; k0 += KCH)
+        if (const int rc = split_grad(both && k0 == 0, std::min(K - k0, KCH), grad_args(d, a, K, k0), ws, ws_bytes, s)) return rc;
     if (split) return SEPCORR_OK;
     int rc = SEPCORR_OK;
     const int kch = d.W2 > 128 ? 2 : KCH;   // wide workgroups have half the registers per lane
@@ -4272,6 +4282,13 @@ size_t sepcorr_backward_workspace_bytes(int B, int H1, int W1, int H2, int W2, i
     return bwd_ws(d).full;
 }
 
+size_t sepcorr_backward_workspace_bytes_for(int max_avg, int compression, int B, int H1, int W1, int H2, int W2, int C) {
+    if (B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1) return 0;
+    const Dims d = {B, H1, W1, H2, W2, C};
+    const size_t need = bwd_ws(d).total;
+    return compression ? std::max(need, split_gradients_bytes(d, max_avg != 0)) : need;
+}
+
 int sepcorr_max_argmax_avg_backward(const float *f1, const float *f2, const int32_t *argmax_u, const int32_t *argmax_v,
                                     const float *grad_u, const float *grad_v, float *d_f1, float *d_f2, int B, int H1,
                                     int W1, int H2, int W2, int C, void *workspace, size_t workspace_bytes, void *stream) {
@@ -4334,16 +4351,16 @@ int sepcorr_compression_backward(const float *f1, const float *f2, const float *
     }
     if (int rc = check_workspace(d, workspace, workspace_bytes)) return rc;
     const BwdWs lay = bwd_ws(d);
-    const bool split = split_gradients(d, lay, false, workspace_bytes);
-    ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased && !split);
-    // d_a_v[k,u] = sum_v S g_cv[k,v];  d_a_u[k,v] = sum_u S g_cu[k,u]: the forward's weighted sums
-    int rc = weighted_forward(d, f1, f2, g_cv, g_cu, d_a_v, d_a_u, K, lay.fwd_bytes ? workspace : nullptr, lay.fwd_bytes, fj.user);
     BwdArgs a;
     memset(&a, 0, sizeof(a));
     a.xcd_order = xcd_order_enabled();
     a.f1 = f1; a.f2 = f2; a.a_u = a_u; a.a_v = a_v; a.g_cu = g_cu; a.g_cv = g_cv;
     a.d1 = d_f1; a.d2 = d_f2;
     a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
+    const bool split = split_gradients(d, a, false, K, workspace_bytes);
+    ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased && !split);
+    // d_a_v[k,u] = sum_v S g_cv[k,v];  d_a_u[k,v] = sum_u S g_cu[k,u]: the forward's weighted sums
+    int rc = weighted_forward(d, f1, f2, g_cv, g_cu, d_a_v, d_a_u, K, lay.fwd_bytes ? workspace : nullptr, lay.fwd_bytes, fj.user);
     if (rc == SEPCORR_OK) rc = feature_gradients(d, a, false, K, split, workspace, workspace_bytes, fj.sa, fj.sb);
     const int rj = fj.join();
     return rc ? rc : rj;
@@ -4396,7 +4413,7 @@ size_t sepcorr_compression_backward_from_logits_workspace_bytes(int B, int H1, i
     const size_t dots = 2 * ((rows * sizeof(float) + 255) & ~(size_t)255);
     if (!with_features) return ((sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255) + dots;
     const size_t a_bytes = ((rows * W2 * sizeof(float) + 255) & ~(size_t)255) + ((rows * H2 * sizeof(float) + 255) & ~(size_t)255);
-    return bwd_ws(d).full + dots + a_bytes;
+    return std::max(bwd_ws(d).total, split_gradients_bytes(d, false)) + dots + a_bytes;
 }
 
 int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, const float *logits_u, const float *logits_v,
@@ -4412,16 +4429,21 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     if ((d_f1 == nullptr) != (d_f2 == nullptr))
         return fail(SEPCORR_EINVAL, "sepcorr: d_f1 and d_f2 must be given together or both be NULL");
     const BwdWs lay = bwd_ws(d);
-    const size_t best = sepcorr_compression_backward_from_logits_workspace_bytes(B, H1, W1, H2, W2, C, K, d_f1 != nullptr);
-    const size_t need = best - (d_f1 ? lay.full - lay.total : 0);   // (the rest is for split_gradients())
+    const size_t rows = (size_t)B * H1 * W1 * K;
+    const size_t dot_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
+    const size_t au_bytes = (rows * W2 * sizeof(float) + 255) & ~(size_t)255, av_bytes = (rows * H2 * sizeof(float) + 255) & ~(size_t)255;
+    const size_t rest = 2 * dot_bytes + (d_f1 ? au_bytes + av_bytes : 0);
+    size_t own_bytes = d_f1 ? lay.total : (sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255;
+    const size_t need = own_bytes + rest;
     if (workspace == nullptr || workspace_bytes < need)
         return fail(SEPCORR_EWORKSPACE, "sepcorr: backward from logits needs %zu bytes of workspace, got %zu", need,
                     workspace ? workspace_bytes : (size_t)0);
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return fail(SEPCORR_EWORKSPACE, "sepcorr: workspace must be 256-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
-    const size_t rows = (size_t)B * H1 * W1 * K;
-    const size_t dot_bytes = (rows * sizeof(float) + 255) & ~(size_t)255;
-    const size_t own_bytes = d_f1 ? (workspace_bytes >= best ? lay.full : lay.total) : (sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255;
+    if (d_f1) {   // more of it for split_gradients(), where there is more
+        const size_t split_bytes = split_gradients_bytes(d, false);
+        if (split_bytes > own_bytes && workspace_bytes >= split_bytes + rest) own_bytes = split_bytes;
+    }
     char *base = static_cast<char *>(workspace);
     float *dot_u = reinterpret_cast<float *>(base + own_bytes);               // sum_u g_cu * comp_u = sum_v a_u * d_a_u
     float *dot_v = reinterpret_cast<float *>(base + own_bytes + dot_bytes);   // sum_v g_cv * comp_v = sum_u a_v * d_a_v
@@ -4444,7 +4466,7 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     if (rc || d_f1 == nullptr) return rc;
     // feature gradients: the weights themselves, formed once from logits and statistics behind the other scratch
     float *a_u = reinterpret_cast<float *>(base + own_bytes + 2 * dot_bytes);
-    float *a_v = reinterpret_cast<float *>(base + own_bytes + 2 * dot_bytes + ((rows * W2 * sizeof(float) + 255) & ~(size_t)255));
+    float *a_v = reinterpret_cast<float *>(base + own_bytes + 2 * dot_bytes + au_bytes);
     {
         const dim3 grid(row_groups(rows)), block(256);
         ProfScope ps("softmax_apply", s);
@@ -4452,14 +4474,14 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
         hipLaunchKernelGGL(softmax_apply_kernel, grid, block, 0, s, logits_v, stats_v, a_v, (long)rows, H2, (int)(rows_vec4(logits_v, H2) && rows_vec4(a_v, H2)));
         if (int rc2 = check_launch("softmax from statistics")) return rc2;
     }
-    const bool split = split_gradients(d, lay, false, own_bytes);
-    ForkJoin fj(s, !lay.aliased && !split);
     BwdArgs a;
     memset(&a, 0, sizeof(a));
     a.xcd_order = xcd_order_enabled();
     a.f1 = f1; a.f2 = f2; a.a_u = a_u; a.a_v = a_v; a.g_cu = g_cu; a.g_cv = g_cv;
     a.d1 = d_f1; a.d2 = d_f2;
     a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
+    const bool split = split_gradients(d, a, false, K, own_bytes);
+    ForkJoin fj(s, !lay.aliased && !split);
     rc = feature_gradients(d, a, false, K, split, workspace, own_bytes, fj.sa, fj.sb);
     const int rj = fj.join();
     return rc ? rc : rj;
@@ -4673,7 +4695,7 @@ static int fused_backward(const float *f1, const float *f2, const int32_t *argma
     a.add_d1 = add_d_f1 != 0;
     a.B = B; a.N1 = H1 * W1; a.H2 = H2; a.W2 = W2; a.C = C;
     const BwdWs lay = bwd_ws(d);
-    const bool split = split_gradients(d, lay, true, workspace_bytes);
+    const bool split = split_gradients(d, a, true, K, workspace_bytes);
     ForkJoin fj(static_cast<hipStream_t>(stream), !lay.aliased && !split);
     const int rc = feature_gradients(d, a, true, K, split, workspace, workspace_bytes, fj.sa, fj.user);
     const int rj = fj.join();

@@ -48,7 +48,8 @@ struct GradArgs {
 #define SPLIT_GRAD_LINE_ALONE 5e8
 // Scratch split_grad() wants for these sizes, whatever the number of channels, 0 where it does not take them.
 size_t split_grad_bytes(int B, int N1, int H2, int W2, int C);
-// Runs both contractions, with the max/average terms if `both`, when the sizes suit it and ws_bytes suffice; returns 1 without
-// launching anything otherwise, a negative SEPCORR_ code on error.  kc: 1 to 4 weight channels.
+// Whether split_grad() takes a call with these arguments and this much scratch.
+bool split_grad_fits(int both, int kc, const GradArgs &a, size_t ws_bytes);
+// Runs both contractions, with the max/average terms if `both`; a negative SEPCORR_ code on error.  kc: 1 to 4 weight channels.
 int split_grad(int both, int kc, GradArgs a, void *ws, size_t ws_bytes, hipStream_t s);
 #endif

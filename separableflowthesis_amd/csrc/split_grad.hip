@@ -1274,11 +1274,22 @@ size_t split_grad_bytes(int B, int N1, int H2, int W2, int C) {
     return p.ok ? p.bytes() : 0;
 }
 
-int split_grad(int both, int kc, GradArgs a, void *ws, size_t ws_bytes, hipStream_t s) {
+namespace {
+GradPlan plan_of(int both, int kc, const GradArgs &a) {
     uintptr_t bits = reinterpret_cast<uintptr_t>(a.a_u) | reinterpret_cast<uintptr_t>(a.g_cv);
     if (both) bits |= reinterpret_cast<uintptr_t>(a.g_v) | reinterpret_cast<uintptr_t>(a.am_v);
-    const GradPlan p = plan(a.B, a.N1, a.H2, a.W2, a.C, both, kc, a.KT, bits % 16 == 0);
-    if (!p.ok || ws == nullptr || ws_bytes < p.bytes()) return 1;
+    return plan(a.B, a.N1, a.H2, a.W2, a.C, both, kc, a.KT, bits % 16 == 0);
+}
+}  // namespace
+
+bool split_grad_fits(int both, int kc, const GradArgs &a, size_t ws_bytes) {
+    const GradPlan p = plan_of(both, kc, a);
+    return p.ok && ws_bytes >= p.bytes();
+}
+
+int split_grad(int both, int kc, GradArgs a, void *ws, size_t ws_bytes, hipStream_t s) {
+    const GradPlan p = plan_of(both, kc, a);
+    if (!p.ok || ws == nullptr || ws_bytes < p.bytes()) return sepcorr_set_error(SEPCORR_EWORKSPACE, "sepcorr: feature gradients: scratch does not suffice");
     a.ncb = p.ncb; a.nvc = p.nvc; a.H2p = p.H2p; a.N1p = p.N1p; a.npx = p.npx; a.G1 = p.G1; a.G2 = p.G2; a.direct = p.direct;
     char *base = static_cast<char *>(ws);
     auto take = [&](size_t n) { char *r = base; base += n; return r; };
