@@ -595,8 +595,10 @@ __global__ void __launch_bounds__(64) lookup_df2_kernel(const LookupBwdArgs a) {
 #pragma unroll
             for (int pr = 0; pr < NPR; ++pr)
                 if (at + 2 * pr < count) {
+                    const bool mine = at + 2 * pr + half < count;   // (an infinite feature times weight 0 would be a NaN)
 #pragma unroll
-                    for (int cb = 0; cb < NB; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.wa[pr], s.fb[pr][cb], acc[cb], 0, 0, 0);
+                    for (int cb = 0; cb < NB; ++cb)
+                        acc[cb] = __builtin_amdgcn_mfma_f32_32x32x2f32(s.wa[pr], mine ? s.fb[pr][cb] : 0.f, acc[cb], 0, 0, 0);
                 }
         };
         Step s0, s1;

@@ -152,6 +152,21 @@ def test_feature_gradient_at_the_edges_of_the_pixel_lists(device, H, W, C, r, sa
     assert ((d_f2.cpu().double() - exact(f1, up)).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("C", [8, 6])   # channels by four, one by one
+@pytest.mark.parametrize("W", [3, 5])   # an odd number of pixels under a tile: the last one without a partner
+def test_infinite_feature_of_the_last_pixel(device, C, W):
+    """Infinite where its window lies, not NaN: it is multiplied by its own weights only."""
+    from separableflowthesis_amd import MemorySaver
+    g = torch.Generator().manual_seed(C + W)
+    f1, f2 = torch.randn(1, 1, W, C, generator=g), torch.randn(1, 1, W, C, generator=g)
+    f1[0, 0, W - 1, 0] = float("inf")
+    coords = torch.stack((torch.arange(W) + 0.3, torch.full((W,), 0.4))).view(1, 2, 1, W)
+    up = torch.rand(1, 9, 1, W, generator=g) + 0.5
+    _, (d_f2,) = MemorySaver.lookup_backward(f1.to(device), [f2.to(device)], coords.to(device), up.to(device), 1, 1.0)
+    assert bool((d_f2[0, 0, W - 2:, 0] == float("inf")).all())   # (the window of the last pixel begins one column before it)
+    assert bool(d_f2[0, 0, :, 1:].isfinite().all())
+
+
 def test_lookup_backward_is_deterministic_and_checks_its_workspace(device):
     import ctypes
     from separableflowthesis_amd import MemorySaver, _lib
