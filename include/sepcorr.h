@@ -72,9 +72,9 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap);
  * attention-gradient pass of the compression backward) and of d_f1; no counterpart in the reference.
  *   SEPCORR_CONTRACT_SPLIT   forward sweeps of 32 <= C <= 256 channels and at least 1e9 of B H1 W1 H2 W2 (C + 64) with every
  *                            fp32 operand as two 16-bit halves (the note on scratch memory above), and so the
- *                            feature gradients of the compression from 5e8 on, of the combined backward from
- *                            2.5e8 on, where the workspace is what the query gives; fp32 MFMA elsewhere (the
- *                            initial choice).
+ *                            feature gradients of the compression and of the combined backward where that pays (from
+ *                            2.5e8 to 2e9 of the same product on, by rows and weight channels) and the workspace is what the
+ *                            query gives; fp32 MFMA elsewhere (the initial choice).
  *   SEPCORR_CONTRACT_FP32    fp32 MFMA throughout.
  *   SEPCORR_CONTRACT_BF16X3  every fp32 operand is written exactly as the sum of three bf16 numbers and the
  *                            product taken as the six largest of the nine plane products, with bf16 MFMA

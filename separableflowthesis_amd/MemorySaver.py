@@ -51,9 +51,9 @@ def _stream():
     return torch.cuda.current_stream().cuda_stream
 
 
-def _workspace(lib, max_avg, compression, dims, device):
-    """Scratch of the max/average backward (1, 0), the compression's (0, 1) or the combined one (1, 1)."""
-    n = lib.sepcorr_backward_workspace_bytes_for(max_avg, compression, *dims)
+def _workspace(lib, max_avg, K, dims, device):
+    """Scratch of the max/average backward (1, 0), of the compression's with K weight channels (0, K) or the combined one (1, K)."""
+    n = lib.sepcorr_backward_workspace_bytes_for(max_avg, K, *dims)
     ws = torch.empty(max(n, 1), dtype=torch.uint8, device=device)
     return ws, n
 
@@ -162,7 +162,7 @@ def compression_backward(img1_features_l0, img2_features_lk, attention_weights_u
         d2 = torch.empty_like(f2)
         da_u = torch.empty_like(attention_weights_u)
         da_v = torch.empty_like(attention_weights_v)
-        ws, n = _workspace(lib, 0, 1, (B, H1, W1, H2, W2, C), dev)
+        ws, n = _workspace(lib, 0, K, (B, H1, W1, H2, W2, C), dev)
         _lib.check(lib.sepcorr_compression_backward(
             f1.data_ptr(), f2.data_ptr(), attention_weights_u.data_ptr(), attention_weights_v.data_ptr(),
             grad_compressed_output_u.data_ptr(), grad_compressed_output_v.data_ptr(),
@@ -499,7 +499,7 @@ def fused_backward(img1_features_l0, img2_features_lk, argmax_output_u, argmax_o
             _expect("add_to_grad_fmap1", add_to_grad_fmap1, tuple(f1.shape), dev)
         d1 = torch.empty_like(f1) if add_to_grad_fmap1 is None else add_to_grad_fmap1
         d2 = torch.empty_like(f2)
-        ws, n = _workspace(lib, 1, 1, (B, H1, W1, H2, W2, C), dev)
+        ws, n = _workspace(lib, 1, K, (B, H1, W1, H2, W2, C), dev)
         _lib.check((lib.sepcorr_fused_backward if add_to_grad_fmap1 is None else lib.sepcorr_fused_backward_add)(
             f1.data_ptr(), f2.data_ptr(), argmax_output_u.data_ptr(), argmax_output_v.data_ptr(),
             grad_MaxAvg_u.data_ptr(), grad_MaxAvg_v.data_ptr(),

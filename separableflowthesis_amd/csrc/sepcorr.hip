@@ -4092,9 +4092,9 @@ int maxavg_backward(const Dims &d, bool gather, const float *f1, const float *f2
 }
 
 // Scratch the contractions of split_grad.hip are given in a call with these feature gradients, 0 where they do not run.
-size_t split_gradients_bytes(const Dims &d, bool both) {
+size_t split_gradients_bytes(const Dims &d, bool both, int K) {
     const double size = (double)d.B * d.H1 * d.W1 * d.H2 * d.W2 * (d.C + 64);
-    if (size < (both ? SPLIT_GRAD_LINE : SPLIT_GRAD_LINE_ALONE) || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 0;
+    if (size < split_grad_line(both, K, d.W2, d.C) || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 0;
     return split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C);
 }
 
@@ -4112,7 +4112,7 @@ GradArgs grad_args(const Dims &d, const BwdArgs &a, int K, int k0) {
 
 // Whether the feature gradients of a call with this workspace come from them.  (Weights at odd addresses take more scratch.)
 bool split_gradients(const Dims &d, const BwdArgs &a, bool both, int K, size_t ws_bytes) {
-    const size_t n = split_gradients_bytes(d, both);
+    const size_t n = split_gradients_bytes(d, both, K);
     if (n == 0 || ws_bytes < n) return false;
     for (int k0 = 0; k0 < K; k0 += KCH)
         if (!split_grad_fits(both && k0 == 0, std::min(K - k0, KCH), grad_args(d, a, K, k0), ws_bytes)) return false;
@@ -4282,11 +4282,11 @@ size_t sepcorr_backward_workspace_bytes(int B, int H1, int W1, int H2, int W2, i
     return bwd_ws(d).full;
 }
 
-size_t sepcorr_backward_workspace_bytes_for(int max_avg, int compression, int B, int H1, int W1, int H2, int W2, int C) {
-    if (B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1) return 0;
+size_t sepcorr_backward_workspace_bytes_for(int max_avg, int K, int B, int H1, int W1, int H2, int W2, int C) {
+    if (K < 0 || K > MAX_K || B < 1 || H1 < 1 || W1 < 1 || H2 < 1 || W2 < 1 || C < 1) return 0;
     const Dims d = {B, H1, W1, H2, W2, C};
     const size_t need = bwd_ws(d).total;
-    return compression ? std::max(need, split_gradients_bytes(d, max_avg != 0)) : need;
+    return K ? std::max(need, split_gradients_bytes(d, max_avg != 0, K)) : need;
 }
 
 int sepcorr_max_argmax_avg_backward(const float *f1, const float *f2, const int32_t *argmax_u, const int32_t *argmax_v,
@@ -4413,7 +4413,7 @@ size_t sepcorr_compression_backward_from_logits_workspace_bytes(int B, int H1, i
     const size_t dots = 2 * ((rows * sizeof(float) + 255) & ~(size_t)255);
     if (!with_features) return ((sweep_bytes(B, H1, W1, H2, W2, C, K) + 255) & ~(size_t)255) + dots;
     const size_t a_bytes = ((rows * W2 * sizeof(float) + 255) & ~(size_t)255) + ((rows * H2 * sizeof(float) + 255) & ~(size_t)255);
-    return std::max(bwd_ws(d).total, split_gradients_bytes(d, false)) + dots + a_bytes;
+    return std::max(bwd_ws(d).total, split_gradients_bytes(d, false, K)) + dots + a_bytes;
 }
 
 int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, const float *logits_u, const float *logits_v,
@@ -4441,7 +4441,7 @@ int sepcorr_compression_backward_from_logits(const float *f1, const float *f2, c
     if (reinterpret_cast<uintptr_t>(workspace) & 255) return fail(SEPCORR_EWORKSPACE, "sepcorr: workspace must be 256-byte aligned");
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (d_f1) {   // more of it for split_gradients(), where there is more
-        const size_t split_bytes = split_gradients_bytes(d, false);
+        const size_t split_bytes = split_gradients_bytes(d, false, K);
         if (split_bytes > own_bytes && workspace_bytes >= split_bytes + rest) own_bytes = split_bytes;
     }
     char *base = static_cast<char *>(workspace);

@@ -6,11 +6,11 @@
 // Records `msg` as the calling thread's last error and returns `code`.
 int sepcorr_set_error(int code, const char *msg);
 
-// sepcorr_backward_workspace_bytes() for one entry point: max_avg 1, compression 0: max/average backward; 0, 1: compression
-// backward; 1, 1: combined backward.  Leaves out what that one has no use for with the contraction that is set (the
-// operands in halves, below their sizes or for the max/average gradients alone); the call runs as it would with more.  (C
-// linkage: the Python mirror asks.)
-extern "C" size_t sepcorr_backward_workspace_bytes_for(int max_avg, int compression, int B, int H1, int W1, int H2, int W2, int C);
+// sepcorr_backward_workspace_bytes() for one entry point: max_avg 1, K 0: max/average backward; 0 and K weight channels:
+// compression backward; 1 and K: combined backward.  Leaves out what that one has no use for with the contraction that is
+// set (the operands in halves, below the sizes from which they pay); the call runs as it would with more.  (C linkage: the
+// Python mirror asks.)
+extern "C" size_t sepcorr_backward_workspace_bytes_for(int max_avg, int K, int B, int H1, int W1, int H2, int W2, int C);
 
 // Fork/join on the library's two side streams per device, for calls whose kernels are independent of each other.
 // sepcorr_fork makes *sa and *sb wait for everything queued on `user` and returns a token; when overlap is switched

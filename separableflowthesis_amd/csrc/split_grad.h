@@ -39,13 +39,23 @@ struct GradArgs {
     int G1, G2;                               // workgroups of the two contractions
 };
 
-// Below this many pairs of pixels times (channels + 64) split_grad() takes nothing, and below the other one it does not pay
-// for the compression alone.  Five or six launches, three of them over the operands, against two to five: time over that of
-// the fp32 kernels in 70 shapes of 1e8 to 6e9, 32 <= C <= 256, 1 to 4 weight channels: with the max/average terms 1.0 to 2.1
-// below 1.4e8, 0.38 to 1.01 from 2.5e8 on (the fp32 kernels make two passes for one or three weight channels); without
-// them 0.76 to 1.34 up to 5e8, 0.65 to 1.09 up to 1e9; above 1e9 0.28 to 0.80, on average 0.49.
-#define SPLIT_GRAD_LINE 2.5e8
-#define SPLIT_GRAD_LINE_ALONE 5e8
+// Below this many pairs of pixels times (channels + 64) split_grad() takes nothing.
+#define SPLIT_GRAD_LEAST 2.5e8
+// From how many of them on it runs.  It is five or six launches, three of them over the operands, against two to five; the fp32
+// kernels it replaces make a pass of their own for the max/average terms beside one or three weight channels, two for four in rows
+// above 128, and take longer where rows are no multiple of 4.  Time over theirs in 37 000 shapes of 2.5e8 to 4e9, C 32 to
+// 256, just below and just above the line (median / largest but 5 %):
+//   with the max/average terms, one or three channels: rows of a multiple of 4, 4e8: 0.75 / 1.02 and 0.71 / 0.91; others: 0.53 / 0.68
+//   two or four: rows of a multiple of 4, 2e9: 0.96 / 1.19 and 0.85 / 1.01; others, 4.5e8: 0.77 / 1.04 and 0.72 / 0.95
+//   alone: rows of a multiple of 4, 2e9: 0.96 / 1.13 and 0.90 / 1.03; others, 7e8: 0.85 / 1.02 and 0.79 / 0.99
+//   up to 64 channels the same ratios are reached at six tenths of that; rows above 128: 0.45 / 0.60 at all sizes.
+inline double split_grad_line(bool both, int K, int W2, int C) {
+    double line;
+    if (W2 > 128) line = both ? SPLIT_GRAD_LEAST : 5e8;
+    else if (both && (K == 1 || K == 3)) line = W2 % 4 ? SPLIT_GRAD_LEAST : 4e8;
+    else line = W2 % 4 == 0 ? 2e9 : both ? 4.5e8 : 7e8;
+    return C > 64 ? line : 0.6 * line;
+}
 // Scratch split_grad() wants for these sizes, whatever the number of channels, 0 where it does not take them.
 size_t split_grad_bytes(int B, int N1, int H2, int W2, int C);
 // Whether split_grad() takes a call with these arguments and this much scratch.

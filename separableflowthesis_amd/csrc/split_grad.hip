@@ -1231,7 +1231,7 @@ size_t align256(size_t n) { return (n + 255) & ~(size_t)255; }
 GradPlan plan(int B, int N1, int H2, int W2, int C, int both, int kc, int KT, bool aligned) {
     GradPlan p = {};
     if (C < kMinChannels || C > 256 || kc < 1 || kc > 4) return p;
-    if ((double)B * N1 * H2 * W2 * (C + 64) < SPLIT_GRAD_LINE) return p;
+    if ((double)B * N1 * H2 * W2 * (C + 64) < SPLIT_GRAD_LEAST) return p;
     p.ncb = C <= 64 ? 2 : C <= 128 ? 4 : 8;
     p.nvc = (W2 + 31) / 32;
     p.H2p = (H2 + ROWS - 1) / ROWS * ROWS;

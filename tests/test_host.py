@@ -229,26 +229,26 @@ def test_no_scratch_where_no_sweep_uses_any():
         assert MemorySaver._fwd_workspace(lib, dims, 2, "cpu") == (None, None, 0)
 
 
-@pytest.mark.parametrize("dims,alone,combined", [((2, 55, 128, 55, 128, 256), True, True), ((4, 48, 64, 48, 64, 256), True, True),
-                                                 ((1, 30, 40, 30, 40, 256), False, True),     # 4.6e8 of pairs times (C + 64)
-                                                 ((1, 20, 32, 20, 32, 256), False, False), ((2, 55, 128, 55, 128, 16), False, False)])
-def test_scratch_of_one_backward_entry_point(dims, alone, combined):
+@pytest.mark.parametrize("dims,K,alone,combined", [((2, 55, 128, 55, 128, 256), 4, True, True), ((4, 48, 64, 48, 64, 256), 1, True, True),
+                                                   # 4.6e8 of pairs times (C + 64): a third channel is a pass of its own to the fp32 kernels
+                                                   ((1, 30, 40, 30, 40, 256), 3, False, True), ((1, 30, 40, 30, 40, 256), 4, False, False),
+                                                   ((1, 30, 41, 30, 41, 256), 4, False, True), ((1, 36, 41, 37, 41, 256), 4, True, True),
+                                                   ((1, 20, 32, 20, 32, 256), 4, False, False), ((2, 55, 128, 55, 128, 16), 4, False, False)])
+def test_scratch_of_one_backward_entry_point(dims, K, alone, combined):
     """The gradients of the max/average outputs ask for no scratch for operands in halves, the others where they use it."""
     lib = _lib.load()
     one = ctypes.c_void_p(256)
     assert lib.sepcorr_max_argmax_avg_backward(*[one] * 8, *dims, one, 0, None) == -3
     need = int(re.search(rb"needs (\d+) bytes", lib.sepcorr_last_error()).group(1))
     split = lib.sepcorr_backward_workspace_bytes(*dims)
-    assert lib.sepcorr_backward_workspace_bytes_for(1, 0, *dims) == need
-    assert (split > need) == combined
-    assert lib.sepcorr_backward_workspace_bytes_for(0, 1, *dims) == (split if alone else need)
-    assert lib.sepcorr_backward_workspace_bytes_for(1, 1, *dims) == (split if combined else need)
+    assert lib.sepcorr_backward_workspace_bytes_for(1, 0, *dims) == need and (split > need or not combined)
+    assert lib.sepcorr_backward_workspace_bytes_for(0, K, *dims) == (split if alone else need)
+    assert lib.sepcorr_backward_workspace_bytes_for(1, K, *dims) == (split if combined else need)
     old = lib.sepcorr_set_contraction(0)
     try:
-        assert lib.sepcorr_backward_workspace_bytes_for(0, 1, *dims) == lib.sepcorr_backward_workspace_bytes_for(1, 1, *dims) == need
+        assert lib.sepcorr_backward_workspace_bytes_for(0, K, *dims) == lib.sepcorr_backward_workspace_bytes_for(1, K, *dims) == need
     finally:
         lib.sepcorr_set_contraction(old)
-    rest = [lib.sepcorr_compression_backward_from_logits_workspace_bytes(*dims, 2, 1)]
-    assert lib.sepcorr_compression_backward_from_logits(*[one] * 14, *dims, 2, one, 0, None) == -3
-    rest.append(int(re.search(rb"needs (\d+) bytes", lib.sepcorr_last_error()).group(1)))
-    assert rest[0] - rest[1] == (split - need if alone else 0)
+    best = lib.sepcorr_compression_backward_from_logits_workspace_bytes(*dims, K, 1)
+    assert lib.sepcorr_compression_backward_from_logits(*[one] * 14, *dims, K, one, 0, None) == -3
+    assert best - int(re.search(rb"needs (\d+) bytes", lib.sepcorr_last_error()).group(1)) == (split - need if alone else 0)

@@ -14,10 +14,10 @@ from tests._util import op_inputs
 
 pytestmark = pytest.mark.gpu
 
-# (B, H1, W1, H2, W2, C), B H1 W1 H2 W2 (C + 64) of 5e8 and more; weight channels
-SHAPES = [((1, 30, 82, 74, 35, 32), 1), ((2, 31, 64, 61, 36, 33), 4), ((1, 63, 65, 33, 65, 64), 3), ((1, 41, 91, 62, 32, 65), 2),
-          ((1, 36, 64, 33, 68, 128), 4), ((3, 21, 43, 55, 36, 130), 1), ((1, 47, 48, 42, 36, 255), 3), ((2, 24, 49, 27, 97, 256), 2),
-          ((1, 16, 8, 136, 240, 256), 4), ((1, 72, 120, 8, 24, 256), 4), ((1, 33, 47, 17, 100, 256), 6)]
+# (B, H1, W1, H2, W2, C), B H1 W1 H2 W2 (C + 64) above the lines of split_grad_line() alone and combined; weight channels
+SHAPES = [((1, 30, 82, 74, 35, 32), 1), ((3, 31, 64, 61, 36, 33), 4), ((1, 63, 65, 33, 65, 64), 3), ((1, 87, 91, 62, 32, 65), 2),
+          ((1, 74, 64, 33, 68, 128), 4), ((6, 21, 43, 55, 36, 130), 1), ((2, 47, 48, 42, 36, 255), 3), ((2, 24, 49, 27, 97, 256), 2),
+          ((1, 16, 8, 136, 240, 256), 4), ((2, 136, 120, 8, 24, 256), 4), ((2, 43, 47, 17, 100, 256), 6)]
 
 
 # More tiles than workgroups (256), or as many: tiles of d_f1 x their steps, tiles of d_f2 x theirs.  Up to 48 steps a tile's
@@ -122,7 +122,7 @@ def test_against_float64(device, dims, K, both):
 @pytest.mark.parametrize("what", ["avoided 12", "avoided 40", "one loud pixel", "small at random", "peaks", "masked", "tiny"])
 def test_every_row_by_itself(device, what, both):
     """Rows of d_f2 that all attention avoids, or that only pixels with small gradients reach, and rows of d_f1 of such pixels."""
-    B, H1, W1, H2, W2, C = dims = (1, 40, 53, 37, 56, 128)
+    B, H1, W1, H2, W2, C = dims = (1, 40, 53, 90, 56, 128)
     x = _tensors(device, dims, 3, seed=5)
     g = torch.Generator(device=device).manual_seed(6)
     zu, zv = (torch.randn(x[k].shape, generator=g, device=device) for k in ("a_u", "a_v"))
@@ -171,7 +171,7 @@ def test_sums_are_not_biased(device):
 @pytest.mark.parametrize("both", [False, True], ids=["compression", "combined"])
 def test_operands_without_halves(device, what, both):
     # (two channels with the max/average terms: the fp32 kernels then take them in one pass too, and inf comes out alike)
-    dims, K = ((2, 24, 49, 27, 52, 256), 2) if both else ((1, 41, 91, 62, 35, 65), 3)
+    dims, K = ((4, 24, 49, 27, 52, 256), 2) if both else ((1, 41, 91, 62, 35, 65), 3)
     x = _tensors(device, dims, K)
     if what == "f2 inf": x["f2"][0, 3, 4, 5] = float("inf")
     if what == "f1 nan": x["f1"][0, 3, 4, 5] = float("nan")
@@ -209,7 +209,7 @@ def test_fp32_contraction_against_float64(device, dims, K, both):
 
 def test_scratch_and_alignment(device):
     """Less scratch than the query gives, and weights at addresses that are no multiple of 16: the same gradients."""
-    dims, K = (2, 24, 49, 27, 52, 256), 2
+    dims, K = (4, 24, 49, 27, 52, 256), 2
     x = _tensors(device, dims, K)
     ref = _run(x, False)
     y = dict(x)
@@ -232,7 +232,7 @@ def test_scratch_and_alignment(device):
 
 
 def test_replayed_graph(device):
-    x = _tensors(device, (2, 24, 49, 27, 52, 256), 4)
+    x = _tensors(device, (4, 24, 49, 27, 52, 256), 4)
     ref = _run(x, True)
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
