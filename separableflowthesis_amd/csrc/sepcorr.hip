@@ -4094,7 +4094,7 @@ int maxavg_backward(const Dims &d, bool gather, const float *f1, const float *f2
 // Scratch the contractions of split_grad.hip are given in a call with these feature gradients, 0 where they do not run.
 size_t split_gradients_bytes(const Dims &d, bool both, int K) {
     const double size = (double)d.B * d.H1 * d.W1 * d.H2 * d.W2 * (d.C + 64);
-    if (size < split_grad_line(both, K, d.W2, d.C) || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 0;
+    if (size < split_grad_line(both, K, d.B, d.H1 * d.W1, d.H2, d.W2, d.C) || g_contraction.load(std::memory_order_relaxed) != SEPCORR_CONTRACT_SPLIT) return 0;
     return split_grad_bytes(d.B, d.H1 * d.W1, d.H2, d.W2, d.C);
 }
 

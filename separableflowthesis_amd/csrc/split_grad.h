@@ -43,17 +43,23 @@ struct GradArgs {
 #define SPLIT_GRAD_LEAST 2.5e8
 // From how many of them on it runs.  It is five or six launches, three of them over the operands, against two to five; the fp32
 // kernels it replaces make a pass of their own for the max/average terms beside one or three weight channels, two for four in rows
-// above 128, and take longer where rows are no multiple of 4.  Time over theirs in 37 000 shapes of 2.5e8 to 4e9, C 32 to
-// 256, just below and just above the line (median / largest but 5 %):
-//   with the max/average terms, one or three channels: rows of a multiple of 4, 4e8: 0.75 / 1.02 and 0.71 / 0.91; others: 0.53 / 0.68
-//   two or four: rows of a multiple of 4, 2e9: 0.96 / 1.19 and 0.85 / 1.01; others, 4.5e8: 0.77 / 1.04 and 0.72 / 0.95
-//   alone: rows of a multiple of 4, 2e9: 0.96 / 1.13 and 0.90 / 1.03; others, 7e8: 0.85 / 1.02 and 0.79 / 0.99
+// above 128, and take longer where rows are no multiple of 4 and then most for a small second image (they have few workgroups).
+// Time over theirs in 37 000 shapes of 2.5e8 to 4e9, C 32 to 256, just below and just above the line (median / largest but 5 %):
+//   with the max/average terms, one or three channels: 0.75 / 1.00 at 2.5e8, others than multiples of 4 0.53 / 0.66; with fewer than
+//     8 tiles of d_f2, hundreds of pieces each, 0.85 / 1.20, and at 4e8 0.74 / 0.98
+//   two or four: rows of a multiple of 4, 2e9: 0.96 / 1.19 and 0.85 / 1.01; others, 4.5e8: 0.77 / 1.04 and 0.72 / 0.95, small second
+//     images 0.61 / 0.93 at 2.5e8
+//   alone: rows of a multiple of 4, 2e9: 0.96 / 1.13 and 0.90 / 1.03; others, 7e8: 0.85 / 1.02 and 0.79 / 0.99, small second images
+//     0.59 / 0.86 at 5e8
 //   up to 64 channels the same ratios are reached at six tenths of that; rows above 128: 0.45 / 0.60 at all sizes.
-inline double split_grad_line(bool both, int K, int W2, int C) {
+inline double split_grad_line(bool both, int K, int B, int N1, int H2, int W2, int C) {
+    const bool few = (long)B * ((H2 + 7) / 8) * ((W2 + 31) / 32) < 8, small = 12L * H2 * W2 <= N1;
     double line;
     if (W2 > 128) line = both ? SPLIT_GRAD_LEAST : 5e8;
-    else if (both && (K == 1 || K == 3)) line = W2 % 4 ? SPLIT_GRAD_LEAST : 4e8;
-    else line = W2 % 4 == 0 ? 2e9 : both ? 4.5e8 : 7e8;
+    else if (both && (K == 1 || K == 3)) line = W2 % 4 == 0 && few ? 4e8 : SPLIT_GRAD_LEAST;
+    else if (W2 % 4 == 0) line = 2e9;
+    else if (small) line = both ? SPLIT_GRAD_LEAST : 5e8;
+    else line = both ? 4.5e8 : 7e8;
     return C > 64 ? line : 0.6 * line;
 }
 // Scratch split_grad() wants for these sizes, whatever the number of channels, 0 where it does not take them.

@@ -888,7 +888,7 @@ struct D2Shape {
     static constexpr int MC = NCB / 2;                                   // channel blocks of a wave (and two rows)
     static constexpr int FB = NCB * 2048, VB = vfields(BOTH, KC) * 2048; // a step's f1 and v-indexed weights
     static constexpr int RS = 72, GB = ROWS * 2 * 16 * RS;               // dL/dS: [row][half][16 pixels][32 columns]
-    static constexpr size_t LDS = 3 * (size_t)(FB + VB) + 2 * GB + ROWS * 32 * 4;
+    static constexpr size_t LDS = 3 * (size_t)(FB + VB) + 2 * GB + ROWS * 32 * 4 + 1024;
 };
 
 // DIRECT: the v-indexed weights come into LDS from the tensors themselves (rows of a multiple of 4 floats, 16-byte aligned),
@@ -902,6 +902,7 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
     extern __shared__ char smem[];
     char *gbuf = smem + 3 * (FB + VB);
     float *tq = reinterpret_cast<float *>(gbuf + 2 * GB);                // factors of the tile's positions, [row][column]
+    int *ce = reinterpret_cast<int *>(tq + ROWS * 32);                   // what takes the channels' back
     if (unsuitable(a)) {
         contract_fp32<false, BOTH, KC>(a.self, reinterpret_cast<float *>(smem));
         return;
@@ -1030,6 +1031,7 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
         {   // factors of the tile's positions for these steps: eight waves take every eighth block of 16 pixels
             const float *bx = a.bound_v + ((size_t)b * a.nvc + vc) * (a.N1p / 16) * NX * 32 + 4 * (lane & 7);
             const float *by = a.bound_u + (size_t)b * (a.N1p / 16) * NX * a.H2p + ROWS * ug + (lane >> 3);
+            const int channel = a.cback[b * 256 + (tid & 255)];
             v4f top = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int i = 0; i < FLUSH / 8; ++i) {
@@ -1056,6 +1058,8 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
 #pragma unroll
                 for (int i = 0; i < 8; ++i) m = fmaxf(m, red[i * 256 + tid]);
                 tq[tid] = power(scale_exponent(m));
+            } else {
+                ce[tid - 256] = channel;
             }
         }
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(2 * ND) : "memory");
@@ -1074,6 +1078,15 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
             const int gi = (t - ta) & 1, far = buf == 0 ? 2 : buf - 1;
             const char *fb = smem + buf * (FB + VB) + half * MC * 2048 + lane * 16;
             v4f tr[2];
+            v8h F[MC][2];
+            auto load_f = [&]() __attribute__((always_inline)) {
+#pragma unroll
+                for (int j = 0; j < MC; ++j)
+#pragma unroll
+                    for (int q = 0; q < 2; ++q) F[j][q] = *reinterpret_cast<const v8h *>(fb + j * 2048 + q * 1024);
+            };
+            constexpr bool LATE = NCB == 8;   // (there are not the registers to have them while dL/dS is formed)
+            if (!LATE) load_f();
             load_tr(tr);
             __builtin_amdgcn_sched_barrier(0);
             make_g(buf, gi ^ 1, tr);
@@ -1081,11 +1094,7 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
             __builtin_amdgcn_sched_barrier(0);
             dma(t + 2, far);
             __builtin_amdgcn_sched_barrier(0);
-            v8h F[MC][2];   // (not before: there are not the registers to have them while dL/dS is formed)
-#pragma unroll
-            for (int j = 0; j < MC; ++j)
-#pragma unroll
-                for (int q = 0; q < 2; ++q) F[j][q] = *reinterpret_cast<const v8h *>(fb + j * 2048 + q * 1024);
+            if (LATE) load_f();
             __builtin_amdgcn_sched_barrier(0);
             // lane 16 (2 h + w) + 4 r + q asks for columns 16 w + 4 q.. of pixel 8 h + r and gets column 16 w + 4 r + q of four pixels
             const char *gb = gbuf + gi * GB + (8 * h + ((lane >> 2) & 3)) * RS + ((lane >> 4) & 1) * 32 + (lane & 3) * 8 + 2 * rp * 2 * 16 * RS;
@@ -1132,12 +1141,12 @@ __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
             for (int j = 0; j < MC; ++j) {
                 float x[16], y[16];
                 v4f *block = block_of(slot, (2 * rp + r) * NCB + half * MC + j);
-                const int ce = a.cback[b * 256 + 32 * (half * MC + j) + (lane & 31)];
+                const int back = ce[32 * (half * MC + j) + (lane & 31)];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const v4f t = *reinterpret_cast<const v4f *>(tq + (2 * rp + r) * 32 + 8 * q + 4 * h);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) x[4 * q + e] = ldexpf(block_sign(ta / FLUSH) * acc[r][j][4 * q + e], ce - exponent_of(t[e]));
+                    for (int e = 0; e < 4; ++e) x[4 * q + e] = ldexpf(block_sign(ta / FLUSH) * acc[r][j][4 * q + e], back - exponent_of(t[e]));
                 }
                 sums_of_piece(block, first, x, y);
                 if (!out) put_block(block, y);

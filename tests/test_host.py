@@ -233,6 +233,9 @@ def test_no_scratch_where_no_sweep_uses_any():
                                                    # 4.6e8 of pairs times (C + 64): a third channel is a pass of its own to the fp32 kernels
                                                    ((1, 30, 40, 30, 40, 256), 3, False, True), ((1, 30, 40, 30, 40, 256), 4, False, False),
                                                    ((1, 30, 41, 30, 41, 256), 4, False, True), ((1, 36, 41, 37, 41, 256), 4, True, True),
+                                                   # a small second image; few tiles of d_f2
+                                                   ((12, 40, 56, 5, 7, 256), 4, False, True), ((2, 60, 100, 8, 24, 128), 1, False, True),
+                                                   ((1, 60, 100, 8, 24, 256), 1, False, False),
                                                    ((1, 20, 32, 20, 32, 256), 4, False, False), ((2, 55, 128, 55, 128, 16), 4, False, False)])
 def test_scratch_of_one_backward_entry_point(dims, K, alone, combined):
     """The gradients of the max/average outputs ask for no scratch for operands in halves, the others where they use it."""
