@@ -252,7 +252,9 @@ class Workload:
         out_u, out_v = E(B, H, W, 2, H), E(B, H, W, 2, W)
         am_u, am_v = E(B, H, W, 1, H, dt=torch.int32), E(B, H, W, 1, W, dt=torch.int32)
         backward = "C" in ops or "F" in ops
-        nws = lib.sepcorr_backward_workspace_bytes(B, H, W, H, W, C) if backward else 0
+        # (the max/average gradients alone have no use for the compression's operands in halves)
+        per_call = [(1, 0)] + [(m, Kp) for m in (0, 1) if "C" in ops]
+        nws = max(lib.sepcorr_backward_workspace_bytes_for(m, k, B, H, W, H, W, C) for m, k in per_call) if backward else 0
         ws = torch.empty(max(nws, 256), dtype=torch.uint8, device=dev)
         self.workspace_bytes = nws
         dims = (B, H, W, H, W, C)

@@ -74,7 +74,10 @@ int sepcorr_profile_collect(char *names, size_t names_cap, float *ms, int cap);
  *                            fp32 operand as two 16-bit halves (the note on scratch memory above), and so the
  *                            feature gradients of the compression and of the combined backward where that pays (from
  *                            2.5e8 to 2e9 of the same product on, by rows and weight channels) and the workspace is what the
- *                            query gives; fp32 MFMA elsewhere (the initial choice).
+ *                            query gives: features within 2^-22 of themselves or 2^-39 of their channel's largest (inf,
+ *                            NaN and widely spread channels are multiplied in fp32), the gradient of the volume within
+ *                            2^-22 of itself or 2^-39 of the largest of its pixel (d_f1) or around its position (d_f2);
+ *                            fp32 MFMA elsewhere (the initial choice).
  *   SEPCORR_CONTRACT_FP32    fp32 MFMA throughout.
  *   SEPCORR_CONTRACT_BF16X3  every fp32 operand is written exactly as the sum of three bf16 numbers and the
  *                            product taken as the six largest of the nine plane products, with bf16 MFMA

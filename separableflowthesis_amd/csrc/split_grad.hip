@@ -18,9 +18,9 @@
 // (inf, NaN, more than one feature in 2048 below 2^-17 of its channel's largest) are found on the way, and the contractions
 // then run in fp32 from the inputs instead (contract_fp32).
 // Relative error against 64 bits, d_f1 / d_f2, fp32 kernels -> halves: B=2, 55x128, K=4 2.2e-7 / 6.9e-7 -> 1.7e-7 / 3.0e-7;
-// 40x56 1.9e-7 / 2.1e-7 -> 1.3e-7 / 1.5e-7, of single rows at the most 2.6e-7 / 3.1e-7 -> 1.6e-7 / 3.2e-7, also with attention
-// that avoids half of image 2 by 40 in the logits or with gradients of 2^-40..1; 136x240 2.4e-7 / 9.0e-7 -> 1.8e-7 / 3.3e-7;
-// B=2, 47x61, C=100, K=2 2.1e-7 / 3.5e-7 -> 1.3e-7 / 2.0e-7.
+// B=4, 48x64 2.2e-7 / 4.5e-7 -> 1.5e-7 / 2.5e-7; 136x240 2.4e-7 / 9.0e-7 -> 1.8e-7 / 3.3e-7; B=2, 47x61, C=100, K=2 2.1e-7 / 3.5e-7 ->
+// 1.3e-7 / 2.0e-7.  Of single rows at B=2, 40x56, with attention that is flat, peaked or avoids half of image 2 by up to 40 in
+// the logits and gradients of one size or of 2^-40..1, at the most 2.8e-7 / 4.4e-7 -> 1.7e-7 / 3.4e-7.
 //
 // Work split.  A workgroup of eight waves, one per compute unit, owns 128 pixels x all channels of d_f1, or 8 rows x 32
 // columns x all channels of d_f2 (64 or 128 accumulator registers a lane), and takes a step at a time: 32 columns of a row of
@@ -29,10 +29,11 @@
 // registers over the rows, d_f2 has them in LDS and transposes G with ds_read_b64_tr_b16.  The steps of all tiles are dealt
 // out evenly; pieces of tiles are put together by grad_finish_kernel in the order of their steps.
 //
-// Measured at B=2, 55x128, C=256, K=4 (fp32 kernels, then here): d_f1 507 us and 14 before it, 187 + 17; d_f2 517 + 14, 205 + 20;
-// the operands 46 on top.  Backward call 1.28 -> 0.73 ms, 136x240 20.9 -> 7.1 ms.  The matrix instructions alone take 123 us
+// Measured at B=2, 55x128, C=256, K=4 (fp32 kernels, then here): d_f1 507 us and 14 before it, 195 + 16; d_f2 517 + 14, 220 + 19;
+// the operands 54 on top.  Backward call 1.28 -> 0.73 ms, 136x240 20.9 -> 7.2 ms.  The matrix instructions alone take 123 us
 // each at the 1.24 PFLOP/s that a large fp16 product reaches here.  What the rest is, in d_f1 (variants with a part left out,
-// results then wrong): without forming G 148 us, without the DMA 182 of then 209.
+// results then wrong): without forming G 148 us, without the DMA 182 of then 209; in d_f2 the factors by positions are 18 of it,
+// 6 to find them, 3 to take them back, the rest beside forming G.
 #include "split_grad.h"
 
 #include <math.h>
@@ -149,8 +150,9 @@ __device__ __forceinline__ const float *vrow(const GradArgs &a, int f, size_t bp
     return reinterpret_cast<const float *>(a.am_v) + bp * a.W2;
 }
 
-// What both contractions need beforehand, bound by its traffic: 82 MB read and 29 written in 32 us at B=2, 55x128, K=4 (46 with
-// the channels' blocks behind the others and one channel a lane; 59 more with atomics for the channels' maxima).
+// What both contractions need beforehand, bound by its traffic: 82 MB read and 31 written in 37 us at B=2, 55x128, K=4 (32 without
+// the bounds; 44 with the v-indexed rows read twice for them; 14 more with the channels' blocks behind the others and one channel a
+// lane, 59 more with atomics for the channels' maxima).
 // Blocks [0, 2 B SLABS): the largest magnitude of every channel of a slab of f1 or f2.
 // The blocks behind them: the weights of 16 pixels, and what bounds |G| there,
 //   |G[p,u,v]| <= sum_k |a_u[k,v] g_cu[k,u]| + sum_k |a_v[k,u] g_cv[k,v]| (+ the max/average gradients):
@@ -658,7 +660,8 @@ struct D1Shape {
     static constexpr size_t LDS = (size_t)NB * BLK + 2 * 16384 + VLDS;
 };
 
-// Bound by what its waves wait for each other: matrix units 41 % busy, vector units 37 %.  With all waves in the same phase
+// Bound by what its waves wait for each other: matrix units 45 % busy (36 with the max/average terms), vector units 50 %, of the
+// time a compute unit is.  With all waves in the same phase
 // (operands from LDS, G, products) 209 us at B=2, 55x128, K=4, with every second wave a phase behind 195; with the other
 // order of G and products in half of the waves, but one barrier a step, 213; at a raised priority around the products 214.
 template <bool BOTH, int KC, int NCB>
@@ -891,10 +894,11 @@ struct D2Shape {
     static constexpr size_t LDS = 3 * (size_t)(FB + VB) + 2 * GB + ROWS * 32 * 4 + 1024;
 };
 
+// Bound like split_d1_kernel: matrix units 38 % busy (30 with the max/average terms), vector units 38 %.
 // DIRECT: the v-indexed weights come into LDS from the tensors themselves (rows of a multiple of 4 floats, 16-byte aligned),
 // otherwise from a copy laid out for it, 58 MB more written and read back at B=2, 55x128, K=4.  While the compiler waited for
 // the requests of a step before the transposed reads, 260 us; with those in one block of assembly 222; with every second
-// wave a phase behind 216.  Row groups of one column chunk follow each other, so that an XCD's workgroups read the same weights.
+// wave a phase behind 216 (all three before the factors by positions).  Row groups of one column chunk follow each other, so that an XCD's workgroups read the same weights.
 template <bool BOTH, int KC, int NCB, bool DIRECT>
 __global__ void __launch_bounds__(512) split_d2_kernel(const GradArgs a) {
     typedef D2Shape<BOTH, KC, NCB> S;
